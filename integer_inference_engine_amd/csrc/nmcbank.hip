@@ -131,115 +131,394 @@ __global__ __launch_bounds__(256) void nb_router_kernel(const int64_t* __restric
   logits[row * experts + e] = (int64_t)acc >> fw;
 }
 
-// lowest-index top-k by logit and their sigmoid gates (cohere2.py:162-165, :181-182); one thread per row
-__global__ void nb_topk_kernel(const int64_t* __restrict__ logits, int64_t rows, int experts, int used, int fa,
-                               int* __restrict__ ids, int64_t* __restrict__ gates) {
-  const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= rows) return;
+// lowest-index top-k by logit and their sigmoid gates (cohere2.py:162-165, :181-182); one wave per row. The order
+// (logit descending, index ascending) is total, so pick k is the first element of that order behind pick k - 1: a
+// wave maximum over the lanes' strided elements per pick, and no list of the taken ones. Bound by the latency of its
+// `used` reductions; the gates are formed by one lane each at the end. (One thread per row scanning every logit
+// for every pick took 467 us at 128 experts, top-8; this takes 12.)
+__global__ __launch_bounds__(64) void nb_topk_kernel(const int64_t* __restrict__ logits, int experts, int used, int fa,
+                                                     int* __restrict__ ids, int64_t* __restrict__ gates) {
+  const int64_t r = blockIdx.x;
+  const int lane = threadIdx.x;
   const int64_t* lr = logits + r * experts;
+  constexpr int kKeep = 4;                            // logits kept in registers: 256 experts without a reload
+  int64_t v[kKeep];
+#pragma unroll
+  for (int i = 0; i < kKeep; ++i) v[i] = lane + 64 * i < experts ? lr[lane + 64 * i] : 0;
+  int64_t prev = 0;
+  int prev_id = -1;
   for (int k = 0; k < used; ++k) {
-    int best_id = -1;
     int64_t best = INT64_MIN;
-    for (int e = 0; e < experts; ++e) {
-      bool taken = false;
-      for (int j = 0; j < k; ++j) taken = taken || ids[r * used + j] == e;
-      if (!taken && (best_id < 0 || lr[e] > best)) { best = lr[e]; best_id = e; }
+    int best_id = INT_MAX;                            // none yet
+    auto take = [&](int64_t x, int e) {
+      const bool behind = prev_id < 0 || x < prev || (x == prev && e > prev_id);
+      if (e < experts && behind && (best_id == INT_MAX || x > best)) { best = x; best_id = e; }
+    };
+#pragma unroll
+    for (int i = 0; i < kKeep; ++i) take(v[i], lane + 64 * i);
+    for (int e = lane + 64 * kKeep; e < experts; e += 64) take(lr[e], e);
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) {
+      const int64_t x = (int64_t)__shfl_xor((long long)best, o, 64);
+      const int e = __shfl_xor(best_id, o, 64);
+      if (e != INT_MAX && (best_id == INT_MAX || x > best || (x == best && e < best_id))) { best = x; best_id = e; }
     }
-    ids[r * used + k] = best_id;
-    gates[r * used + k] = nb_sigmoid(best, fa);
+    prev = best;
+    prev_id = best_id;
+    if (lane == 0) {
+      ids[r * used + k] = best_id;
+      gates[r * used + k] = best;
+    }
   }
+  __syncthreads();                                    // lane 0's logits are visible to the lanes that squash them
+  for (int k = lane; k < used; k += 64) gates[r * used + k] = nb_sigmoid(gates[r * used + k], fa);
 }
 
-// interleaved RoPE of q (H heads) and k (Hkv heads) at position pos, with the reference's envelope guard
-// (2 max|x| max|cos, sin| <= INT64_MAX, rope.py:26-39) and exact per-element checks; one workgroup
-__global__ __launch_bounds__(256) void nb_rope_kernel(int64_t* __restrict__ q, int64_t nq, int64_t* __restrict__ k,
-                                                      int64_t nk, int hd, const int64_t* __restrict__ cs,
-                                                      const int64_t* __restrict__ sn, int64_t pos, int fa,
-                                                      int* __restrict__ status) {
+// Interleaved RoPE of q (in place) and k, the K / V append at `pos` (cache [Hkv][max_len][hd]) and the running
+// max|K|, max|V| (kv_max[0..1]); one workgroup per q or kv head. The reference's envelope guard
+// (2 max|x| max|cos, sin| <= INT64_MAX over all of q, and over all of k, rope.py:26-39) fires when any head's own
+// maximum breaks it, so every workgroup tests its head and none waits for the others; after a guard the outputs
+// are discarded, so what is written then does not matter. Latency-bound (one dependent load, two reductions): one
+// launch in place of three single-workgroup ones (RoPE 13 us, append and max|q| 5 us each).
+__global__ __launch_bounds__(128) void nb_rope_append_kernel(int64_t* __restrict__ q, int heads,
+                                                             const int64_t* __restrict__ k,
+                                                             const int64_t* __restrict__ v, int hd,
+                                                             const int64_t* __restrict__ cs,
+                                                             const int64_t* __restrict__ sn, int64_t pos,
+                                                             int64_t max_len, int fa, int rope,
+                                                             int64_t* __restrict__ ck, int64_t* __restrict__ cv,
+                                                             uint64_t* __restrict__ kv_max, int* __restrict__ status) {
+  const bool is_q = (int)blockIdx.x < heads;
+  const int64_t kvh = is_q ? 0 : (int64_t)blockIdx.x - heads;
+  const int64_t* x = is_q ? q + (int64_t)blockIdx.x * hd : k + kvh * hd;
+  int64_t* y = is_q ? q + (int64_t)blockIdx.x * hd : ck + (kvh * max_len + pos) * hd;
   const int half = hd / 2;
-  const int64_t* c = cs + pos * half;
-  const int64_t* s = sn + pos * half;
-  uint64_t mq = 0, mk = 0, mc = 0;
-  for (int64_t i = threadIdx.x; i < nq; i += 256) { const uint64_t a = nb_uabs(q[i]); mq = a > mq ? a : mq; }
-  for (int64_t i = threadIdx.x; i < nk; i += 256) { const uint64_t a = nb_uabs(k[i]); mk = a > mk ? a : mk; }
-  for (int i = threadIdx.x; i < half; i += 256) {
-    const uint64_t a = nb_uabs(c[i]), b = nb_uabs(s[i]);
-    mc = a > mc ? a : mc;
-    mc = b > mc ? b : mc;
-  }
-  mq = nb_block_max(mq);
-  mk = nb_block_max(mk);
-  mc = nb_block_max(mc);
-  if ((u128)2 * mq * mc > (u128)INT64_MAX || (u128)2 * mk * mc > (u128)INT64_MAX) {
-    if (threadIdx.x == 0) atomicOr(status, kGuard);
-    return;
-  }
-  for (int64_t i = threadIdx.x; i < (nq + nk) / 2; i += 256) {
-    int64_t* x = i < nq / 2 ? q + 2 * i : k + 2 * (i - nq / 2);
-    const int pr = (int)((i < nq / 2 ? i : i - nq / 2) % half);
-    const int64_t a = x[0], b = x[1];
-    const i128 p0 = (i128)a * c[pr] - (i128)b * s[pr], p1 = (i128)a * s[pr] + (i128)b * c[pr];
-    if (p0 > (i128)INT64_MAX || p0 < (i128)INT64_MIN || p1 > (i128)INT64_MAX || p1 < (i128)INT64_MIN) {
-      atomicOr(status, kGuard);
-      continue;
+  uint64_t mx = 0, mc = 0, mk = 0, mv = 0;
+  for (int i = threadIdx.x; i < half; i += 128) {
+    int64_t a = x[2 * i], b = x[2 * i + 1];
+    if (rope) {
+      const int64_t c = cs[pos * half + i], s = sn[pos * half + i];
+      const uint64_t ua = nb_uabs(a), ub = nb_uabs(b), uc = nb_uabs(c), us = nb_uabs(s);
+      mx = ua > mx ? ua : mx;
+      mx = ub > mx ? ub : mx;
+      mc = uc > mc ? uc : mc;
+      mc = us > mc ? us : mc;
+      const i128 p0 = (i128)a * c - (i128)b * s, p1 = (i128)a * s + (i128)b * c;
+      if (p0 > (i128)INT64_MAX || p0 < (i128)INT64_MIN || p1 > (i128)INT64_MAX || p1 < (i128)INT64_MIN)
+        atomicOr(status, kGuard);
+      a = (int64_t)p0 >> fa;
+      b = (int64_t)p1 >> fa;
     }
-    x[0] = (int64_t)p0 >> fa;
-    x[1] = (int64_t)p1 >> fa;
+    if (rope || !is_q) { y[2 * i] = a; y[2 * i + 1] = b; }
+    if (!is_q) {
+      const uint64_t ua = nb_uabs(a), ub = nb_uabs(b);
+      mk = ua > mk ? ua : mk;
+      mk = ub > mk ? ub : mk;
+    }
   }
-}
-
-// K / V append at `pos` (cache [Hkv][max_len][hd]) and the running max|K|, max|V| (kv_max[0..1])
-__global__ __launch_bounds__(256) void nb_append_kernel(const int64_t* __restrict__ k, const int64_t* __restrict__ v,
-                                                        int nkv, int hd, int64_t pos, int64_t max_len,
-                                                        int64_t* __restrict__ ck, int64_t* __restrict__ cv,
-                                                        uint64_t* __restrict__ kv_max) {
-  uint64_t mk = 0, mv = 0;
-  for (int64_t i = threadIdx.x; i < (int64_t)nkv * hd; i += 256) {
-    const int64_t h = i / hd, l = i - h * hd;
-    const int64_t dst = (h * max_len + pos) * hd + l;
-    ck[dst] = k[i];
-    cv[dst] = v[i];
-    const uint64_t a = nb_uabs(k[i]), b = nb_uabs(v[i]);
-    mk = a > mk ? a : mk;
-    mv = b > mv ? b : mv;
+  if (!is_q)
+    for (int i = threadIdx.x; i < hd; i += 128) {
+      const int64_t a = v[kvh * hd + i];
+      cv[(kvh * max_len + pos) * hd + i] = a;
+      const uint64_t u = nb_uabs(a);
+      mv = u > mv ? u : mv;
+    }
+  if (rope) {
+    mx = imie_wave_max_u64_full(mx);
+    mc = imie_wave_max_u64_full(mc);
+    __shared__ uint64_t s_m[2][2];
+    if ((threadIdx.x & 63) == 0) { s_m[threadIdx.x >> 6][0] = mx; s_m[threadIdx.x >> 6][1] = mc; }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      const uint64_t m0 = s_m[0][0] > s_m[1][0] ? s_m[0][0] : s_m[1][0];
+      const uint64_t m1 = s_m[0][1] > s_m[1][1] ? s_m[0][1] : s_m[1][1];
+      if ((u128)2 * m0 * m1 > (u128)INT64_MAX) atomicOr(status, kGuard);
+    }
   }
-  mk = nb_block_max(mk);
-  mv = nb_block_max(mv);
-  if (threadIdx.x == 0) {
-    if (mk > kv_max[0]) kv_max[0] = mk;
-    if (mv > kv_max[1]) kv_max[1] = mv;
+  if (!is_q) {
+    mk = imie_wave_max_u64_full(mk);
+    mv = imie_wave_max_u64_full(mv);
+    if ((threadIdx.x & 63) == 0) {
+      atomicMax((unsigned long long*)&kv_max[0], (unsigned long long)mk);
+      atomicMax((unsigned long long*)&kv_max[1], (unsigned long long)mv);
+    }
   }
-}
-
-// max|x| of n values into out (one workgroup)
-__global__ __launch_bounds__(256) void nb_maxabs_kernel(const int64_t* __restrict__ x, int64_t n,
-                                                        uint64_t* __restrict__ out) {
-  uint64_t m = 0;
-  for (int64_t i = threadIdx.x; i < n; i += 256) { const uint64_t a = nb_uabs(x[i]); m = a > m ? a : m; }
-  m = nb_block_max(m);
-  if (threadIdx.x == 0) *out = m;
 }
 
 // GQA fixed-point attention of the new position `pos` over keys [first, pos] (sliding window when window > 0):
 // score = (((q . k) >> fa) * inv_sqrt) >> fa, softmax of the 2^-d cubic, out = (p . V) >> fa; every int64
-// narrowing is checked (nmc_qk_cuda.cu:343-432). One workgroup per query head; scores in prob (global).
-__global__ __launch_bounds__(256) void nb_attention_kernel(const int64_t* __restrict__ q, const int64_t* __restrict__ ck,
-                                                           const int64_t* __restrict__ cv, int heads, int nkv, int hd,
-                                                           int64_t pos, int64_t max_len, int window, int fa,
-                                                           int64_t inv_sqrt, const uint64_t* __restrict__ qmax,
-                                                           const uint64_t* __restrict__ kv_max,
-                                                           int64_t* __restrict__ prob, int64_t* __restrict__ out,
-                                                           int* __restrict__ status) {
+// narrowing is checked (nmc_qk_cuda.cu:343-432).
+//
+// The keys are split into chunks (a multiple of 64 keys, at most kNbMaxChunks of them); a workgroup takes one chunk of
+// one KV head and up to eight of its query heads, so K and V are read once. Four launches: scores and chunk maxima;
+// e and chunk Z; p and chunk PV sums; the sum over chunks. Under the envelope (max|q| max|K| hd and 2^fa max|V| within
+// int64; otherwise the status is set and the result discarded) the dots and the PV sums fit int64, so 64-bit sums are
+// exact in any order; only the narrowing of (q . k >> fa) * inv_sqrt needs 128 bits, once per score.
+// Bound by latency (34 MB of K and V at 4096 keys x 4 heads take 5 us at 7 TB/s): at a 4096-key window, 32 / 4 heads
+// of 128, 1923 us as one workgroup per query head with 128-bit dots, whose PV walked the keys serially in 128
+// threads, against 18 + 5 + 11 + 4 us for the four launches.
+constexpr int kNbHeads = 8;                           // query heads of one KV head per workgroup
+constexpr int kNbMaxChunks = 128;
+
+struct NbAttn {
+  const int64_t *q, *ck, *cv;
+  int64_t first, pos, max_len, chunk;                 // keys [first, pos], chunk keys per workgroup
+  int heads, nkv, hd, fa;
+  int64_t inv_sqrt;
+  const uint64_t* kv_max;
+  int64_t *prob, *cmax;                               // scores, then e [heads][max_len]; chunk maxima [chunk][heads]
+  uint64_t *cz, *part;                                // chunk Z [chunk][heads]; chunk PV sums [chunk][heads][hd]
+  int64_t* out;
+  int* status;
+};
+
+struct NbGroup { int kv, h0, nh; };                   // KV head, first query head, query heads of this workgroup
+__device__ inline NbGroup nb_group(const NbAttn& a) {
+  const int rep = a.heads / a.nkv, ng = (rep + kNbHeads - 1) / kNbHeads;
+  const int kv = (int)blockIdx.x / ng, g = (int)blockIdx.x % ng;
+  return NbGroup{kv, kv * rep + g * kNbHeads, min(kNbHeads, rep - g * kNbHeads)};
+}
+
+// NIT: 32-dim steps of a key row (hd <= 32 NIT). 16 lanes share a key (2 dims a lane and step), each lane takes four
+// keys of the 64-key step at once, so a step's K loads are all in flight together.
+template <int NIT>
+__global__ __launch_bounds__(256) void nb_scores_kernel(NbAttn a) {
+  __shared__ __align__(16) int64_t s_q[kNbHeads][32 * NIT];
+  __shared__ int64_t s_b[4][kNbHeads];
+  __shared__ uint64_t s_m[4];
+  const NbGroup g = nb_group(a);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = tid & 15, grp = tid >> 4;
+  uint64_t mq = 0;
+  for (int i = tid; i < kNbHeads * 32 * NIT; i += 256) {
+    const int hh = i / (32 * NIT), c = i % (32 * NIT);
+    const int64_t v = hh < g.nh && c < a.hd ? a.q[(int64_t)(g.h0 + hh) * a.hd + c] : 0;
+    s_q[hh][c] = v;
+    const uint64_t u = nb_uabs(v);
+    mq = u > mq ? u : mq;
+  }
+  mq = imie_wave_max_u64_full(mq);
+  if (lane == 0) s_m[wave] = mq;
+  __syncthreads();
+  if (blockIdx.y == 0 && tid == 0) {                  // the envelope: any group's max|q| breaks it alone
+    for (int w = 1; w < 4; ++w) mq = s_m[w] > mq ? s_m[w] : mq;
+    if ((u128)mq * a.kv_max[0] * (u128)(uint64_t)a.hd > (u128)INT64_MAX ||
+        ((u128)1 << a.fa) * a.kv_max[1] > (u128)INT64_MAX)
+      atomicOr(a.status, kGuard);
+  }
+  const int64_t jbeg = a.first + (int64_t)blockIdx.y * a.chunk, jend = min(jbeg + a.chunk, a.pos + 1);
+  const int64_t* kb = a.ck + (int64_t)g.kv * a.max_len * a.hd;
+  int64_t best[2] = {INT64_MIN, INT64_MIN};
+  const int key4 = l16 >> 2, hA = 2 * (l16 & 3);
+  for (int64_t j0 = jbeg; j0 < jend; j0 += 64) {
+    longlong2 kk[NIT][4];
+#pragma unroll
+    for (int it = 0; it < NIT; ++it) {
+      const int c = 2 * l16 + 32 * it;
+#pragma unroll
+      for (int k4 = 0; k4 < 4; ++k4) {                // keys and dims past the end: an in-range duplicate, not used
+        const int64_t j = min(j0 + 16 * k4 + grp, a.pos);
+        kk[it][k4] = *(const longlong2*)(kb + j * a.hd + (c < a.hd ? c : 0));
+      }
+    }
+    uint64_t acc[4 * kNbHeads];
+#pragma unroll
+    for (int i = 0; i < 4 * kNbHeads; ++i) acc[i] = 0;
+#pragma unroll
+    for (int it = 0; it < NIT; ++it)
+#pragma unroll
+      for (int hh = 0; hh < kNbHeads; ++hh) {
+        const longlong2 qv = *(const longlong2*)&s_q[hh][2 * l16 + 32 * it];   // zero past hd
+#pragma unroll
+        for (int k4 = 0; k4 < 4; ++k4)
+          acc[k4 * kNbHeads + hh] += (uint64_t)qv.x * (uint64_t)kk[it][k4].x + (uint64_t)qv.y * (uint64_t)kk[it][k4].y;
+      }
+    // the 16 lanes' sums, halving the kept set each step: lane l ends with sums 2 l and 2 l + 1 (key 2 l / 8)
+#pragma unroll
+    for (int n = 2 * kNbHeads, m = 8; m >= 1; n >>= 1, m >>= 1) {
+      const bool up = (l16 & m) != 0;
+#pragma unroll
+      for (int i = 0; i < n; ++i) {
+        const uint64_t send = up ? acc[i] : acc[i + n], keep = up ? acc[i + n] : acc[i];
+        acc[i] = keep + (uint64_t)__shfl_xor((long long)send, m, 64);
+      }
+    }
+    const int64_t j = j0 + 16 * key4 + grp;
+#pragma unroll
+    for (int r = 0; r < 2; ++r) {
+      if (j >= jend || hA + r >= g.nh) continue;
+      const int64_t sh = (int64_t)acc[r] >> a.fa;
+      const i128 sc = ((i128)sh * a.inv_sqrt) >> a.fa;
+      int64_t score = 0;
+      if (sc > (i128)INT64_MAX || sc < (i128)INT64_MIN) atomicOr(a.status, kGuard);
+      else score = (int64_t)sc;
+      a.prob[(int64_t)(g.h0 + hA + r) * a.max_len + j] = score;
+      best[r] = score > best[r] ? score : best[r];
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+#pragma unroll
+    for (int o = 32; o >= 4; o >>= 1) {               // lanes of one (l16 & 3) hold the same two heads
+      const int64_t u = (int64_t)__shfl_xor((long long)best[r], o, 64);
+      best[r] = u > best[r] ? u : best[r];
+    }
+    if (lane < 4) s_b[wave][hA + r] = best[r];
+  }
+  __syncthreads();
+  if (tid < g.nh) {
+    int64_t b = s_b[0][tid];
+    for (int w = 1; w < 4; ++w) b = s_b[w][tid] > b ? s_b[w][tid] : b;
+    a.cmax[(int64_t)blockIdx.y * a.heads + g.h0 + tid] = b;
+  }
+}
+
+// e_j = 2^-d_j in place of the scores and the chunk's Z; 32 lanes per query head
+__global__ __launch_bounds__(256) void nb_exp_kernel(NbAttn a) {
+  const NbGroup g = nb_group(a);
+  const int hh = threadIdx.x >> 5, l = threadIdx.x & 31;
+  const bool live = hh < g.nh;
+  const int64_t h = g.h0 + (live ? hh : 0);
+  int64_t best = INT64_MIN;
+  for (int c = l; c < (int)gridDim.y; c += 32) {
+    const int64_t v = a.cmax[(int64_t)c * a.heads + h];
+    best = v > best ? v : best;
+  }
+#pragma unroll
+  for (int o = 16; o >= 1; o >>= 1) {
+    const int64_t u = (int64_t)__shfl_xor((long long)best, o, 64);
+    best = u > best ? u : best;
+  }
+  const int64_t l2 = nb_log2e(a.fa);
+  int64_t dclip = ((int64_t)(a.fa + 2) << (2 * a.fa)) / l2;
+  const int64_t hard = ((int64_t)1 << 62) / l2;
+  dclip = hard < dclip ? hard : dclip;
+  const int64_t jbeg = a.first + (int64_t)blockIdx.y * a.chunk, jend = min(jbeg + a.chunk, a.pos + 1);
+  int64_t* ph = a.prob + h * a.max_len;
+  uint64_t z = 0;
+  if (live)
+    for (int64_t j = jbeg + l; j < jend; j += 32) {
+      const uint64_t wide = (uint64_t)best - (uint64_t)ph[j];   // best is the row's maximum: exact below 2^64
+      const int64_t d = wide > (uint64_t)dclip ? dclip : (int64_t)wide;
+      const int64_t e = nb_exp2_neg((int64_t)((uint64_t)d * (uint64_t)l2) >> a.fa, a.fa);
+      ph[j] = e;
+      z += (uint64_t)e;
+    }
+#pragma unroll
+  for (int o = 16; o >= 1; o >>= 1) z += (uint64_t)__shfl_xor((long long)z, o, 64);
+  if (live && l == 0) a.cz[(int64_t)blockIdx.y * a.heads + h] = z;
+}
+
+// p_j = (e_j << fa) / Z, staged per 64 keys, and the chunk's PV sums; thread = dim (DPT dims apart by 128) x key half
+template <int DPT>
+__global__ __launch_bounds__(256) void nb_pv_kernel(NbAttn a) {
+  __shared__ __align__(16) uint32_t s_p[64][kNbHeads];   // p <= 2^fa, fa <= 29
+  __shared__ uint64_t s_z[kNbHeads];
+  __shared__ uint64_t s_sum[128][kNbHeads + 1];
+  const NbGroup g = nb_group(a);
+  const int tid = threadIdx.x;
+  {
+    const int hh = tid >> 5, l = tid & 31;
+    const int64_t h = g.h0 + (hh < g.nh ? hh : 0);
+    uint64_t z = 0;
+    for (int c = l; c < (int)gridDim.y; c += 32) z += a.cz[(int64_t)c * a.heads + h];
+#pragma unroll
+    for (int o = 16; o >= 1; o >>= 1) z += (uint64_t)__shfl_xor((long long)z, o, 64);
+    if (l == 0) s_z[hh] = z;
+  }
+  const int64_t jbeg = a.first + (int64_t)blockIdx.y * a.chunk, jend = min(jbeg + a.chunk, a.pos + 1);
+  const int64_t* vb = a.cv + (int64_t)g.kv * a.max_len * a.hd;
+  const int d0 = tid & 127, half = tid >> 7;
+  uint64_t acc[DPT][kNbHeads];
+#pragma unroll
+  for (int x = 0; x < DPT; ++x)
+#pragma unroll
+    for (int hh = 0; hh < kNbHeads; ++hh) acc[x][hh] = 0;
+  for (int64_t j0 = jbeg; j0 < jend; j0 += 64) {
+    __syncthreads();                                  // the step before is read; s_z is written
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int hh = (tid >> 6) + 4 * i, k = tid & 63;
+      uint32_t p = 0;
+      if (hh < g.nh && j0 + k < jend) {
+        const uint64_t e = (uint64_t)a.prob[(int64_t)(g.h0 + hh) * a.max_len + j0 + k], z = s_z[hh];
+        p = z ? (uint32_t)((e << a.fa) / z) : 0;      // e <= 2^fa: e << fa fits
+      }
+      s_p[k][hh] = p;
+    }
+    __syncthreads();
+    for (int k0 = 32 * half; k0 < 32 * half + 32 && j0 + k0 < jend; k0 += 16) {
+      int64_t v[DPT][16];
+#pragma unroll
+      for (int k = 0; k < 16; ++k)
+#pragma unroll
+        for (int x = 0; x < DPT; ++x)                 // keys past the end carry p = 0; dims past hd are not stored
+          v[x][k] = vb[min(j0 + k0 + k, a.pos) * a.hd + (d0 + 128 * x < a.hd ? d0 + 128 * x : 0)];
+#pragma unroll
+      for (int k = 0; k < 16; ++k) {
+        const uint4 pa = *(const uint4*)&s_p[k0 + k][0], pb = *(const uint4*)&s_p[k0 + k][4];
+        const uint32_t p[kNbHeads] = {pa.x, pa.y, pa.z, pa.w, pb.x, pb.y, pb.z, pb.w};
+#pragma unroll
+        for (int x = 0; x < DPT; ++x)
+#pragma unroll
+          for (int hh = 0; hh < kNbHeads; ++hh) acc[x][hh] += (uint64_t)p[hh] * (uint64_t)v[x][k];
+      }
+    }
+  }
+#pragma unroll
+  for (int x = 0; x < DPT; ++x) {
+    __syncthreads();
+    if (half == 1)
+#pragma unroll
+      for (int hh = 0; hh < kNbHeads; ++hh) s_sum[d0][hh] = acc[x][hh];
+    __syncthreads();
+    const int d = d0 + 128 * x;
+    if (half == 0 && d < a.hd)
+#pragma unroll
+      for (int hh = 0; hh < kNbHeads; ++hh)
+        if (hh < g.nh)
+          a.part[((int64_t)blockIdx.y * a.heads + g.h0 + hh) * a.hd + d] = acc[x][hh] + s_sum[d0][hh];
+  }
+}
+
+// out = (sum of the chunks' PV sums) >> fa; 64 outputs x 4 chunk quarters per workgroup
+__global__ __launch_bounds__(256) void nb_final_kernel(NbAttn a, int nch) {
+  __shared__ uint64_t s_p[4][64];
+  const int64_t n = (int64_t)a.heads * a.hd, i = (int64_t)blockIdx.x * 64 + (threadIdx.x & 63);
+  const int w = threadIdx.x >> 6;
+  uint64_t sum = 0;
+  if (i < n) {
+#pragma unroll 8
+    for (int c = w; c < nch; c += 4) sum += a.part[(int64_t)c * n + i];
+  }
+  s_p[w][threadIdx.x & 63] = sum;
+  __syncthreads();
+  if (w == 0 && i < n) {
+    const int t = threadIdx.x;
+    a.out[i] = (int64_t)(s_p[0][t] + s_p[1][t] + s_p[2][t] + s_p[3][t]) >> a.fa;
+  }
+}
+
+// The same attention for heads wider than the kernels above take (head_dim > kNbMaxHd): one workgroup per query head,
+// 128-bit dots, scores in prob (global).
+constexpr int kNbMaxHd = 256;
+__global__ __launch_bounds__(256) void nb_attention_wide_kernel(NbAttn a) {
+  const int64_t *q = a.q, *ck = a.ck, *cv = a.cv;
+  const int64_t first = a.first, pos = a.pos, max_len = a.max_len, inv_sqrt = a.inv_sqrt;
+  const int heads = a.heads, nkv = a.nkv, hd = a.hd, fa = a.fa;
+  const uint64_t* kv_max = a.kv_max;
+  int64_t *prob = a.prob, *out = a.out;
+  int* status = a.status;
   __shared__ int64_t s_v[4];
   __shared__ uint64_t s_z[4];
   const int head = blockIdx.x, kv = head / (heads / nkv), t = threadIdx.x;
-  // envelope (max|q| max|K| hd and 2^fa max|V| within int64), checked once
-  if (head == 0 && t == 0 &&
-      ((u128)qmax[0] * kv_max[0] * (u128)(uint64_t)hd > (u128)INT64_MAX ||
-       ((u128)1 << fa) * kv_max[1] > (u128)INT64_MAX))
-    atomicOr(status, kGuard);
-  const int64_t first = (window > 0 && pos - window >= 0) ? pos - window + 1 : 0;
   const int64_t* qh = q + (int64_t)head * hd;
+  // envelope (max|q| max|K| hd and 2^fa max|V| within int64): any head's max|q| breaks it alone
+  uint64_t mq = 0;
+  for (int i = t; i < hd; i += 256) { const uint64_t u = nb_uabs(qh[i]); mq = u > mq ? u : mq; }
+  mq = nb_block_max(mq);
+  if (t == 0 && ((u128)mq * kv_max[0] * (u128)(uint64_t)hd > (u128)INT64_MAX ||
+                 ((u128)1 << fa) * kv_max[1] > (u128)INT64_MAX))
+    atomicOr(status, kGuard);
   int64_t* ph = prob + (int64_t)head * max_len;
   int64_t best = INT64_MIN;
   for (int64_t key = first + t; key <= pos; key += 256) {
@@ -321,7 +600,7 @@ struct Bank {
   int64_t max_len = 0, d_model = 0;
   DevBuf cos, sin;
   std::vector<Layer> layers;
-  DevBuf res[2], norm, logits, ids, gates, attn, qkv, ao, prob, status, qmax, moe;
+  DevBuf res[2], norm, logits, ids, gates, attn, qkv, ao, prob, part, status, moe;
   int res_slot = 0;
   bool has_res = false;
   int retained = -1;
@@ -357,7 +636,7 @@ int ensure_layer_kv(Bank& b, Layer& L) {
 size_t bank_bytes(const Bank& b) {
   size_t t = b.cos.cap + b.sin.cap;
   for (const DevBuf* d : {&b.res[0], &b.res[1], &b.norm, &b.logits, &b.ids, &b.gates, &b.attn, &b.qkv, &b.ao, &b.prob,
-                          &b.status, &b.qmax, &b.moe})
+                          &b.part, &b.status, &b.moe})
     t += d->cap;
   for (const Layer& L : b.layers) t += L.k.cap + L.v.cap + L.kvmax.cap;
   return t;
@@ -367,7 +646,7 @@ void bank_release(Bank& b) {
   (void)hipStreamSynchronize(imie_stream());
   for (Layer& L : b.layers) { L.k.release(); L.v.release(); L.kvmax.release(); }
   for (DevBuf* d : {&b.cos, &b.sin, &b.res[0], &b.res[1], &b.norm, &b.logits, &b.ids, &b.gates, &b.attn, &b.qkv,
-                    &b.ao, &b.prob, &b.status, &b.qmax, &b.moe})
+                    &b.ao, &b.prob, &b.part, &b.status, &b.moe})
     d->release();
   b = Bank();
 }
@@ -386,7 +665,7 @@ int attention_preflight(Bank& b, int layer, long long qh, long long kh, long lon
     return IMIE_EARG;
   if (ensure_layer_kv(b, L) || b.qkv.ensure((size_t)(qw + 2 * kw) * 8) || b.attn.ensure((size_t)qw * 8) ||
       b.ao.ensure((size_t)b.d_model * 8) || b.prob.ensure((size_t)(b.heads * b.max_len) * 8) ||
-      b.status.ensure(64) || b.qmax.ensure(64))
+      b.part.ensure((size_t)(kNbMaxChunks * (qw + 2 * b.heads)) * 8) || b.status.ensure(64))
     return IMIE_EARG;
   return IMIE_OK;
 }
@@ -403,16 +682,33 @@ int attention_enqueue(Bank& b, int layer, long long qh, long long kh, long long 
   if (!rc) rc = imie_qk_linear_dev(kh, x, 1, fw, k, status, st);
   if (!rc) rc = imie_qk_linear_dev(vh, x, 1, fw, v, status, st);
   if (rc) return rc;
-  if (rope)
-    hipLaunchKernelGGL(nb_rope_kernel, dim3(1), dim3(256), 0, st, q, qw, k, kw, b.hd, (const int64_t*)b.cos.p,
-                       (const int64_t*)b.sin.p, L.length, b.fa, status);
-  hipLaunchKernelGGL(nb_append_kernel, dim3(1), dim3(256), 0, st, (const int64_t*)k, (const int64_t*)v, b.nkv, b.hd,
-                     L.length, b.max_len, (int64_t*)L.k.p, (int64_t*)L.v.p, (uint64_t*)L.kvmax.p);
-  hipLaunchKernelGGL(nb_maxabs_kernel, dim3(1), dim3(256), 0, st, (const int64_t*)q, qw, (uint64_t*)b.qmax.p);
-  hipLaunchKernelGGL(nb_attention_kernel, dim3((unsigned)b.heads), dim3(256), 0, st, (const int64_t*)q,
-                     (const int64_t*)L.k.p, (const int64_t*)L.v.p, b.heads, b.nkv, b.hd, L.length, b.max_len, window,
-                     b.fa, inv_sqrt, (const uint64_t*)b.qmax.p, (const uint64_t*)L.kvmax.p, (int64_t*)b.prob.p,
-                     (int64_t*)b.attn.p, status);
+  hipLaunchKernelGGL(nb_rope_append_kernel, dim3((unsigned)(b.heads + b.nkv)), dim3(128), 0, st, q, b.heads,
+                     (const int64_t*)k, (const int64_t*)v, b.hd, (const int64_t*)b.cos.p, (const int64_t*)b.sin.p,
+                     L.length, b.max_len, b.fa, rope, (int64_t*)L.k.p, (int64_t*)L.v.p, (uint64_t*)L.kvmax.p, status);
+  NbAttn a = {};
+  a.q = q; a.ck = (const int64_t*)L.k.p; a.cv = (const int64_t*)L.v.p;
+  a.pos = L.length; a.first = (window > 0 && a.pos - window >= 0) ? a.pos - window + 1 : 0;
+  a.max_len = b.max_len; a.heads = b.heads; a.nkv = b.nkv; a.hd = b.hd; a.fa = b.fa; a.inv_sqrt = inv_sqrt;
+  a.kv_max = (const uint64_t*)L.kvmax.p; a.prob = (int64_t*)b.prob.p; a.out = (int64_t*)b.attn.p; a.status = status;
+  if (b.hd > kNbMaxHd) {
+    hipLaunchKernelGGL(nb_attention_wide_kernel, dim3((unsigned)b.heads), dim3(256), 0, st, a);
+  } else {
+    // 64-key chunks (one step a workgroup: the shortest chain) until there would be more than kNbMaxChunks of them
+    const int64_t steps = (a.pos - a.first + 64) / 64;
+    a.chunk = 64 * ((steps + kNbMaxChunks - 1) / kNbMaxChunks);
+    const int nch = (int)((a.pos - a.first + a.chunk) / a.chunk);
+    a.part = (uint64_t*)b.part.p;
+    a.cz = a.part + (int64_t)kNbMaxChunks * qw;
+    a.cmax = (int64_t*)(a.cz + (int64_t)kNbMaxChunks * b.heads);
+    const int rep = b.heads / b.nkv;
+    const dim3 grid((unsigned)(b.nkv * ((rep + kNbHeads - 1) / kNbHeads)), (unsigned)nch);
+    if (b.hd <= 128) hipLaunchKernelGGL(nb_scores_kernel<4>, grid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL(nb_scores_kernel<8>, grid, dim3(256), 0, st, a);
+    hipLaunchKernelGGL(nb_exp_kernel, grid, dim3(256), 0, st, a);
+    if (b.hd <= 128) hipLaunchKernelGGL(nb_pv_kernel<1>, grid, dim3(256), 0, st, a);
+    else hipLaunchKernelGGL(nb_pv_kernel<2>, grid, dim3(256), 0, st, a);
+    hipLaunchKernelGGL(nb_final_kernel, dim3((unsigned)((qw + 63) / 64)), dim3(256), 0, st, a, nch);
+  }
   IMIE_HIP(hipGetLastError());
   return imie_qk_linear_dev(oh, (const int64_t*)b.attn.p, 1, fw, (int64_t*)b.ao.p, status, st);
 }
@@ -472,8 +768,8 @@ int qk_rmsnorm_router(long long gain_h, long long router_h, const int64_t* x, lo
   if (rc) return rc;
   hipLaunchKernelGGL(nb_router_kernel, dim3((unsigned)rrows, (unsigned)rows), dim3(256), 0, st, (const int64_t*)dh.p,
                      width, (const int64_t*)rp, (int)rrows, fw, (int64_t*)dl.p, (int*)ds.p);
-  hipLaunchKernelGGL(nb_topk_kernel, dim3((unsigned)((rows + 63) / 64)), dim3(64), 0, st, (const int64_t*)dl.p, rows,
-                     (int)rrows, used, fa, (int*)di.p, (int64_t*)dg.p);
+  hipLaunchKernelGGL(nb_topk_kernel, dim3((unsigned)rows), dim3(64), 0, st, (const int64_t*)dl.p, (int)rrows, used,
+                     fa, (int*)di.p, (int64_t*)dg.p);
   IMIE_HIP(hipGetLastError());
   int stat = 0;
   IMIE_HIP(hipMemcpyAsync(&stat, ds.p, 4, hipMemcpyDeviceToHost, st));
@@ -669,8 +965,8 @@ int qk_attention_bank_moe_begin(long long h, int layer, long long gain_h, long l
   if (rc) return rc;
   hipLaunchKernelGGL(nb_router_kernel, dim3((unsigned)L.experts, 1), dim3(256), 0, st, (const int64_t*)b->norm.p,
                      L.d_model, (const int64_t*)rp, L.experts, fw, (int64_t*)b->logits.p, status);
-  hipLaunchKernelGGL(nb_topk_kernel, dim3(1), dim3(64), 0, st, (const int64_t*)b->logits.p, (int64_t)1, L.experts,
-                     L.used, b->fa, (int*)b->ids.p, (int64_t*)b->gates.p);
+  hipLaunchKernelGGL(nb_topk_kernel, dim3(1), dim3(64), 0, st, (const int64_t*)b->logits.p, L.experts, L.used,
+                     b->fa, (int*)b->ids.p, (int64_t*)b->gates.p);
   IMIE_HIP(hipGetLastError());
   rc = attention_enqueue(*b, layer, qh, kh, vh, oh, (const int64_t*)b->norm.p, fw, window, rope, inv_sqrt, st);
   if (rc) { (void)hipStreamSynchronize(st); L.poisoned = true; return IMIE_EARG; }

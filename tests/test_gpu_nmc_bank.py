@@ -204,3 +204,55 @@ def test_token_executor_chains_layers_like_the_oracle(gpu):
     bank2.close()
     bank.close()
     qk_gpu.free_all()
+
+
+@pytest.mark.parametrize("heads,nkv,hd,ctx,window,rope", [
+    (12, 1, 64, 63, None, True),        # 8 + 4 query heads of one KV head; exactly one 64-key step
+    (2, 1, 128, 64, None, False),       # one key into the second chunk
+    (8, 4, 160, 130, 100, True),        # heads wider than 128 dims, a window that starts inside the cache
+    (4, 2, 64, 8300, None, True),       # more than 128 steps: chunks of two steps
+    (4, 4, 320, 70, None, True),        # heads wider than the chunked kernels take
+])
+def test_bank_attention_split_edges(gpu, heads, nkv, hd, ctx, window, rope):
+    """The attention sublayer at the edges of its key split, bit for bit against the oracle."""
+    from integer_inference_engine_amd import qk_gpu
+    from oracle.rope import apply_interleaved
+    shapes = {"wq": (heads * hd, D, 0), "wk": (nkv * hd, D, 1), "wv": (nkv * hd, D, 0), "wo": (D, heads * hd, 1)}
+    W, hs = {}, {}
+    for i, (n, (of, nin, qt)) in enumerate(shapes.items()):
+        raw = qk.random_blocks(21, i, of, nin // 256, qt)
+        W[n], hs[n] = qk.dequant(raw, of, nin // 256, qt, FW), qk_gpu.register_weight(raw, of, nin // 256, qt)
+    cap = ctx + 1
+    rng = np.random.default_rng(ctx)
+    cos = rng.integers(-(1 << 16), (1 << 16) + 1, size=(cap, hd // 2), dtype=np.int64)
+    sin = rng.integers(-(1 << 16), (1 << 16) + 1, size=(cap, hd // 2), dtype=np.int64)
+    bank = qk_gpu.ResidentAttentionCache(1, cap, D, heads, nkv, hd, FA, cos, sin)
+    kc, vc = (rng.integers(-(1 << 17), 1 << 17, size=(nkv, cap, hd), dtype=np.int64) for _ in range(2))
+    bank.import_layer(0, kc[:, :ctx], vc[:, :ctx])
+    x = rng.integers(-(1 << 14), 1 << 14, size=(1, D), dtype=np.int64)
+    got = bank.apply(0, hs["wq"], hs["wk"], hs["wv"], hs["wo"], x, FW, window, rope)
+    q, k, v = (qk.linear(x, W[n], FW).reshape(-1, hd) for n in ("wq", "wk", "wv"))
+    if rope:
+        q = apply_interleaved(q[:, None, :], cos[ctx:], sin[ctx:], FA)[:, 0, :]
+        k = apply_interleaved(k[:, None, :], cos[ctx:], sin[ctx:], FA)[:, 0, :]
+    kc[:, ctx], vc[:, ctx] = k, v
+    att = onb.attention_step(q, kc, vc, ctx, window, FA, fx.inv_sqrt_fp(hd, FA)).reshape(1, heads * hd)
+    assert np.array_equal(got, qk.linear(att, W["wo"], FW))
+    bank.close()
+    qk_gpu.free_all()
+
+
+@pytest.mark.parametrize("experts,used", [(3, 3), (64, 8), (65, 1), (300, 12)])
+def test_router_topk_ties(gpu, experts, used):
+    """Lowest-index picks among equal logits, below, at and beyond one wave's 64 experts and its 256 kept logits."""
+    from integer_inference_engine_amd import qk_gpu
+    rng = np.random.default_rng(experts)
+    gain = rng.integers(1 << 15, 1 << 17, size=D, dtype=np.int64)
+    router = rng.integers(-(1 << 20), 1 << 20, size=(experts, D), dtype=np.int64)
+    router[rng.integers(0, experts, size=experts // 2)] = router[0]
+    x = rng.integers(-(1 << 20), 1 << 20, size=(5, D), dtype=np.int64)
+    x[1] = 0                                            # every logit equal
+    got = qk_gpu.rmsnorm_router(qk_gpu.register_i64(gain.reshape(1, D)), qk_gpu.register_i64(router), x, used, FA, FW, 1)
+    sel, gates = qk.moe_route(onb.router_logits(fx.rmsnorm(x, FA, 1, gain), router, FW), used, FA)
+    assert np.array_equal(got[1], sel.astype(np.int32)) and np.array_equal(got[2], gates)
+    qk_gpu.free_all()
