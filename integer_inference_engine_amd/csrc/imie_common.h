@@ -69,6 +69,23 @@ __host__ __device__ __forceinline__ int imie_limbs_needed(uint64_t maxabs) {
   return L;
 }
 
+// Balanced base-256 digits, digit l in byte l: adding 128 at every digit position leaves digit + 128 in each byte (the
+// carries are the balanced form's), and flipping the top bits takes the 128 back. Exact for |v| <= 0x7F7F7F7F (four
+// digits of a 32-bit value), and for the low digits of any 64-bit value (mod 2^64).
+__device__ __forceinline__ uint32_t imie_digits32(uint32_t v) { return (v + 0x80808080u) ^ 0x80808080u; }
+__device__ __forceinline__ uint64_t imie_digits64(uint64_t v) {
+  return (v + 0x8080808080808080ull) ^ 0x8080808080808080ull;
+}
+// 4 x 4 byte transpose: o[l] = byte l of a, b, c, d
+__device__ __forceinline__ void imie_bytes4x4(uint32_t a, uint32_t b, uint32_t c, uint32_t d, uint32_t (&o)[4]) {
+  const uint32_t ab0 = __builtin_amdgcn_perm(b, a, 0x05010400u), ab1 = __builtin_amdgcn_perm(b, a, 0x07030602u);
+  const uint32_t cd0 = __builtin_amdgcn_perm(d, c, 0x05010400u), cd1 = __builtin_amdgcn_perm(d, c, 0x07030602u);
+  o[0] = __builtin_amdgcn_perm(cd0, ab0, 0x05040100u);
+  o[1] = __builtin_amdgcn_perm(cd0, ab0, 0x07060302u);
+  o[2] = __builtin_amdgcn_perm(cd1, ab1, 0x05040100u);
+  o[3] = __builtin_amdgcn_perm(cd1, ab1, 0x07060302u);
+}
+
 __device__ __forceinline__ uint64_t imie_wave_max_u64(uint64_t v) {
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) {

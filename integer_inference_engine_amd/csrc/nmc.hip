@@ -14,6 +14,7 @@
 // from HBM once per call no matter how many tokens use it.
 #include "imie_common.h"
 #include "imie_kernels.h"
+#include "imie_silu.h"
 #include <string.h>
 #include <stdlib.h>
 #include <algorithm>
@@ -323,6 +324,16 @@ __global__ void qk_combine_kernel(const int64_t* __restrict__ dd, int m, int k, 
   for (int j = 0; j < k; ++j) acc += ((i128)dd[(t * k + j) * d_model + o] * gates[t * k + j]) >> fa;
   if (acc > (i128)INT64_MAX || acc < (i128)INT64_MIN) atomicOr(status, IMIE_EOVF);
   out[idx] = (int64_t)acc;
+}
+
+// out = residual + attention + moe, int64 wrap (the reference's committed numpy int64 addition); the MoE's status
+// bits join the layer's
+__global__ void qk_add3_kernel(const int64_t* __restrict__ a, const int64_t* __restrict__ b,
+                               const int64_t* __restrict__ c, int64_t n, int64_t* __restrict__ out,
+                               const int* __restrict__ moe_status, int* __restrict__ status) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) out[i] = (int64_t)((uint64_t)a[i] + (uint64_t)b[i] + (uint64_t)c[i]);
+  if (i == 0 && *moe_status) atomicOr(status, *moe_status);
 }
 
 // ---------------------------------------------------------------------------------------------------------
@@ -760,16 +771,10 @@ __device__ inline int64_t acc_shift(Acc128 a, int fw, bool* fits) {
   return (int64_t)y;
 }
 
-// exact nmc SiLU * up of one element (qk_silu_mul_kernel): false when an intermediate leaves int64
+// exact nmc SiLU * up of one element (qk_silu_mul_kernel): false when an intermediate leaves int64. The sigmoid is the
+// one-exponential form (one of the two clipped exponents is 0), the same values as the two-exponential one there.
 __device__ inline int64_t nmc_silu_mul(int64_t x, int64_t u, int fa, int64_t log2e, int64_t dclip, bool* ok) {
-  const int64_t m = x > 0 ? x : 0;
-  int64_t d0 = m, d1 = (int64_t)((uint64_t)m - (uint64_t)x);
-  if (d0 > dclip) d0 = dclip;
-  if (d1 > dclip) d1 = dclip;
-  const int64_t e0 = exp2_neg_fixed((int64_t)((uint64_t)d0 * (uint64_t)log2e) >> fa, fa);
-  const int64_t e1 = exp2_neg_fixed((int64_t)((uint64_t)d1 * (uint64_t)log2e) >> fa, fa);
-  const int64_t z = e0 + e1;
-  const int64_t sig = z == 0 ? 0 : (int64_t)(((uint64_t)e1 << fa) / (uint64_t)z);
+  const int64_t sig = imie_silu::sigmoid_fixed_fast(x, fa, log2e, dclip);
   const i128 s = ((i128)x * sig) >> fa;
   bool good = s <= (i128)INT64_MAX && s >= (i128)INT64_MIN;
   const i128 gu = ((i128)(int64_t)s * u) >> fa;
@@ -1225,6 +1230,467 @@ __global__ __launch_bounds__(256) void moe_down_kernel(const MoeItem* __restrict
 }
 
 // int8-MFMA path on/off (IMIE_QK_MFMA=0 forces the VALU kernel; tests compare both)
+// ---------------------------------------------------------------------------------------------------------
+// Single-row products (decode): a Q4_K / Q6_K weight against one activation row, and the MoE block of a few tokens.
+// One launch each: every workgroup peels the row's balanced base-256 digits into LDS itself (no prep launch, no flag
+// to reset, no item list to upload: the weight pointers are kernel arguments), a weight row is spread over a half
+// wave, 64 weights (a quarter of a 256-block) per lane, so a row of up to 2048 is one load round and one pass of
+// v_dot4_i32_i8 per limb, and the lanes' 128-bit partial sums are added by shuffles. A row beyond kQkLimbs limbs takes
+// exact 128-bit products in the same kernel. Bound by latency: the weights of one projection are 1 to 5 MB.
+// The digits of 64 consecutive activations are an LDS unit of 80 bytes: 16 lanes reading 16 bytes each at that stride
+// touch every bank once (at 64 bytes the same 16 banks four times over).
+// Measured: a 4096 x 2048 Q4_K product 3.3 + 1.3 + 28 + 4.4 us (prep, flag, 64 workgroups walking the blocks with two
+// barriers each, fallback launch) and three uploads; Q, K and V of one token in one launch, or O: 8.7 us.
+// ---------------------------------------------------------------------------------------------------------
+constexpr int kG1Unit = 80;
+constexpr int kG1MaxNb = 32;       // digits of 32 blocks: 51 KB of LDS
+constexpr int kG1Items = 16;
+constexpr int kG1Rows = 2;         // weight rows per half wave
+
+struct G1Raw {                     // one lane's 64 weights: Q4_K header, quants; Q6_K low, high bits, scales, d
+  uint4 v[6];
+  uint32_t s, d;
+};
+
+template <int QT>
+__device__ inline G1Raw g1_load(const uint8_t* row, int u) {
+  const uint8_t* blk = row + (int64_t)(u >> 2) * (QT == 0 ? 144 : 210);
+  const int q = u & 3;
+  G1Raw r;
+  if (QT == 0) {
+    r.v[0] = gload<uint4>(blk);
+    r.v[1] = gload<uint4>(blk + 16 + 32 * q);
+    r.v[2] = gload<uint4>(blk + 32 + 32 * q);
+    r.s = r.d = 0;
+  } else {
+    const int half = q >> 1;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r.v[i] = gload<uint4>(blk + 64 * half + 16 * i);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) r.v[4 + i] = gload<uint4>(blk + 128 + 32 * half + 16 * i);
+    const uint8_t* sc = blk + 192 + 8 * half + 4 * (q & 1);
+    r.s = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r.s |= (uint32_t)gload<uint8_t>(sc + i) << (8 * i);
+    r.d = (uint32_t)gload<uint8_t>(blk + 208) | ((uint32_t)gload<uint8_t>(blk + 209) << 8);
+  }
+  return r;
+}
+
+// the lane's 64 weights as 16 dwords of int8 (positions 0..31 and 32..63), and their factors: Q4_K sc / mn per 32,
+// Q6_K 4 w and sc per 16; dq, dmq
+struct G1W {
+  int w[16];
+  int sc[4], mn[2];
+  int64_t dq, dmq;
+};
+// fp16_fixed_fast, in 32 bits when every lane's result is below 2^31 (m 2^sh with sh <= 20: single precision holds
+// it exactly either way, so one ldexp and rint serve both directions of the shift)
+__device__ inline int64_t g1_fp16(uint32_t h, int fw) {
+  const uint32_t e = (h >> 10) & 31, mant = h & 0x3FF;
+  const int sh = (e == 0 ? 1 : (int)e) - 25 + fw;
+  if (__any(sh > 20)) return fp16_fixed_fast(h, fw);
+  const float m = (float)(e == 0 ? mant : (mant | 0x400));
+  const int r = (int)__builtin_rintf(__builtin_ldexpf(m, sh));
+  return ((h >> 15) & 1) ? -r : r;
+}
+
+template <int QT>
+__device__ inline G1W g1_unpack(const G1Raw& r, int q, int fw) {
+  G1W o;
+  if (QT == 0) {
+    o.dq = g1_fp16(r.v[0].x & 0xFFFFu, fw);
+    o.dmq = g1_fp16(r.v[0].x >> 16, fw);
+    const uint32_t hd[3] = {r.v[0].y, r.v[0].z, r.v[0].w};   // the 12 scale bytes
+    const int j0 = 2 * (q & 1);                       // sub-blocks 2 q, 2 q + 1; byte j of a dword each
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int sh = 8 * (j0 + h);
+      const uint32_t b0 = (hd[0] >> sh) & 255, b1 = (hd[1] >> sh) & 255, b2 = (hd[2] >> sh) & 255;
+      if (q < 2) { o.sc[h] = b0 & 63; o.mn[h] = b1 & 63; }
+      else { o.sc[h] = (b2 & 0xF) | ((b0 >> 6) << 4); o.mn[h] = (b2 >> 4) | ((b1 >> 6) << 4); }
+    }
+    o.sc[2] = o.sc[3] = 0;
+    const uint32_t qd[8] = {r.v[1].x, r.v[1].y, r.v[1].z, r.v[1].w, r.v[2].x, r.v[2].y, r.v[2].z, r.v[2].w};
+#pragma unroll
+    for (int d = 0; d < 8; ++d) {
+      o.w[d] = (int)(qd[d] & 0x0F0F0F0Fu);
+      o.w[8 + d] = (int)((qd[d] >> 4) & 0x0F0F0F0Fu);
+    }
+  } else {
+    o.dq = g1_fp16(r.d, fw);
+    o.dmq = 0;
+    o.mn[0] = o.mn[1] = 0;
+    const uint32_t lq[16] = {r.v[0].x, r.v[0].y, r.v[0].z, r.v[0].w, r.v[1].x, r.v[1].y, r.v[1].z, r.v[1].w,
+                             r.v[2].x, r.v[2].y, r.v[2].z, r.v[2].w, r.v[3].x, r.v[3].y, r.v[3].z, r.v[3].w};
+    const uint32_t hq[8] = {r.v[4].x, r.v[4].y, r.v[4].z, r.v[4].w, r.v[5].x, r.v[5].y, r.v[5].z, r.v[5].w};
+    // bytewise 4 (q6 - 32) as int8: the 6 bits moved to the top of the byte and its sign bit flipped
+    const int sl = (q & 1) ? 4 : 0, sh = (q & 1) ? 4 : 0;
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int d = 0; d < 8; ++d) {
+        const uint32_t lo = (sl ? lq[8 * u + d] >> 2 : lq[8 * u + d] << 2) & 0x3C3C3C3Cu;
+        const uint32_t hi = (sh ? hq[d] << (2 - 2 * u) : hq[d] << (6 - 2 * u)) & 0xC0C0C0C0u;
+        o.w[8 * u + d] = (int)((lo | hi) ^ 0x80808080u);
+      }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o.sc[i] = (int)(int8_t)(uint8_t)(r.s >> (8 * i));
+  }
+  return o;
+}
+
+// acc[r] += the lane's 64 weights of row r x activations, R rows sharing the digits read; xu: the unit's digits of
+// limb 0 in LDS, ls: bytes between limbs
+template <int QT, int R>
+__device__ inline void g1_dot(const G1W (&w)[R], const int8_t* xu, int ls, int L, Acc128 (&acc)[R]) {
+  // S1 = sum sc w.x (Q6_K: of the 4 w) and S2 = sum mn xsum: a limb's part stays in int32 (Q4_K: 2 x 63 x 32 x 128 x 15
+  // < 2^23, and 2 x 63 x 32 x 128 < 2^19; Q6_K: 4 x 128 x 16 x 128 x 128 = 2^27) and joins with one 32 x 32 + 64
+  int64_t S1[R], S2[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) S1[r] = S2[r] = 0;
+  for (int l = 0; l < L; ++l) {
+    const int wt = 1 << (8 * (l & 3));                // limb 4 (2^32): shifted once more below
+    int xv[16];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int4 x = *(const int4*)(xu + l * ls + 16 * c);
+      xv[4 * c] = x.x;
+      xv[4 * c + 1] = x.y;
+      xv[4 * c + 2] = x.z;
+      xv[4 * c + 3] = x.w;
+    }
+    int b0 = 0, b1 = 0;
+    if (QT == 0) {
+#pragma unroll
+      for (int d = 0; d < 8; ++d) {
+        b0 = __builtin_amdgcn_sdot4(xv[d], 0x01010101, b0, false);
+        b1 = __builtin_amdgcn_sdot4(xv[8 + d], 0x01010101, b1, false);
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      int a[4] = {0, 0, 0, 0}, t1, t2 = 0;
+#pragma unroll
+      for (int d = 0; d < 16; ++d) a[d >> 2] = __builtin_amdgcn_sdot4(xv[d], w[r].w[d], a[d >> 2], false);
+      if (QT == 0) {
+        t1 = __mul24(w[r].sc[0], a[0] + a[1]) + __mul24(w[r].sc[1], a[2] + a[3]);
+        t2 = __mul24(w[r].mn[0], b0) + __mul24(w[r].mn[1], b1);
+      } else {
+        t1 = __mul24(w[r].sc[0], a[0]) + __mul24(w[r].sc[1], a[1]) + __mul24(w[r].sc[2], a[2]) + __mul24(w[r].sc[3], a[3]);
+      }
+      if (l < 4) {
+        S1[r] += (int64_t)t1 * wt;
+        if (QT == 0) S2[r] += (int64_t)t2 * wt;
+      } else {
+        S1[r] += (int64_t)((uint64_t)(uint32_t)t1 << 32);
+        if (QT == 0) S2[r] += (int64_t)((uint64_t)(uint32_t)t2 << 32);
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    acc_madd(acc[r], w[r].dq, QT == 0 ? S1[r] : S1[r] >> 2);   // Q6_K: exact, every weight is a multiple of 4
+    if (QT == 0) acc_madd(acc[r], -w[r].dmq, S2[r]);
+  }
+}
+
+// The lane's 64 weights (unit u of a row) x the 64-bit activations themselves, in 128 bits: a row that needs more than
+// kQkLimbs limbs. Rare, so one compact copy that decodes a weight at a time (unrolled into every caller it cost
+// registers and instruction fetches on the common path).
+__device__ __attribute__((noinline)) void g1_wide(const uint8_t* row, int u, int qtype, int fw, const int64_t* x,
+                                                  Acc128* acc) {
+  const uint8_t* blk = row + (int64_t)(u >> 2) * (qtype == 0 ? 144 : 210);
+  const int q = u & 3;
+  i128 a = (i128)(((unsigned __int128)(uint64_t)acc->hi << 64) | acc->lo);
+  const int n = qtype == 0 ? 32 : 16;                 // one sub-block at a time
+#pragma unroll 1
+  for (int e0 = 0; e0 < 64; e0 += n) {
+    i128 qd = 0, xs = 0;
+#pragma unroll 1
+    for (int e = e0; e < e0 + n; ++e) {
+      int w;
+      if (qtype == 0) {
+        const uint8_t b = gload<uint8_t>(blk + 16 + 32 * q + (e & 31));
+        w = e < 32 ? b & 15 : b >> 4;
+      } else {
+        const int half = q >> 1, qq = 2 * (q & 1) + (e >> 5), l = e & 31;
+        const uint8_t lo = gload<uint8_t>(blk + 64 * half + 32 * (qq & 1) + l);
+        const uint8_t hi = gload<uint8_t>(blk + 128 + 32 * half + l);
+        w = (((qq & 2) ? lo >> 4 : lo & 15) | (((hi >> (2 * qq)) & 3) << 4)) - 32;
+      }
+      qd += (i128)w * x[64 * (int64_t)u + e];
+      xs += x[64 * (int64_t)u + e];
+    }
+    if (qtype == 0) {
+      const int j = 2 * q + (e0 >> 5);
+      const uint8_t* sc = blk + 4;
+      const int s = j < 4 ? gload<uint8_t>(sc + j) & 63
+                          : (gload<uint8_t>(sc + j + 4) & 15) | ((gload<uint8_t>(sc + j - 4) >> 6) << 4);
+      const int m = j < 4 ? gload<uint8_t>(sc + j + 4) & 63
+                          : (gload<uint8_t>(sc + j + 4) >> 4) | ((gload<uint8_t>(sc + j) >> 6) << 4);
+      const uint32_t d = gload<uint8_t>(blk) | ((uint32_t)gload<uint8_t>(blk + 1) << 8);
+      const uint32_t dm = gload<uint8_t>(blk + 2) | ((uint32_t)gload<uint8_t>(blk + 3) << 8);
+      a += (i128)(fp16_fixed_fast(d, fw) * s) * qd - (i128)(fp16_fixed_fast(dm, fw) * m) * xs;
+    } else {
+      const int s = (int8_t)gload<uint8_t>(blk + 192 + 8 * (q >> 1) + 4 * (q & 1) + (e0 >> 4));
+      const uint32_t d = gload<uint8_t>(blk + 208) | ((uint32_t)gload<uint8_t>(blk + 209) << 8);
+      a += (i128)(fp16_fixed_fast(d, fw) * s) * qd;
+    }
+  }
+  acc->lo = (uint64_t)a;
+  acc->hi = (int64_t)((unsigned __int128)a >> 64);
+}
+
+// Digit units of the n activations x (n a multiple of 64) into LDS, kQkLimbs limbs of n / 64 units; returns the limb
+// count that all of them need, 0 when one needs more than kQkLimbs. Ends with a barrier.
+template <int NT>
+__device__ inline int g1_stage(const int64_t* __restrict__ x, int n, int8_t* s_x, uint64_t* s_red) {
+  const int ls = (n >> 6) * kG1Unit;
+  uint64_t mx = 0;
+  for (int c0 = 8 * (int)threadIdx.x; c0 < n; c0 += 8 * NT) {
+    int64_t v[8];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const longlong2 p = *(const longlong2*)(x + c0 + 2 * e);
+      v[2 * e] = p.x;
+      v[2 * e + 1] = p.y;
+    }
+    uint64_t m8 = 0, d[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const uint64_t a = imie_absu64(v[e]);
+      m8 = a > m8 ? a : m8;
+    }
+    mx = m8 > mx ? m8 : mx;
+    if (m8 <= imie_balanced_cap(4)) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) d[e] = imie_digits32((uint32_t)v[e]);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) d[e] = imie_digits64((uint64_t)v[e]);
+    }
+    uint32_t lo[4], hi[4], top[4] = {0, 0, 0, 0};
+    imie_bytes4x4((uint32_t)d[0], (uint32_t)d[1], (uint32_t)d[2], (uint32_t)d[3], lo);
+    imie_bytes4x4((uint32_t)d[4], (uint32_t)d[5], (uint32_t)d[6], (uint32_t)d[7], hi);
+    int8_t* dst = s_x + (c0 >> 6) * kG1Unit + (c0 & 63);
+#pragma unroll
+    for (int l = 0; l < 4; ++l) *(uint2*)(dst + l * ls) = uint2{lo[l], hi[l]};
+    static_assert(kQkLimbs == 5, "one digit above the low four");
+    imie_bytes4x4((uint32_t)(d[0] >> 32), (uint32_t)(d[1] >> 32), (uint32_t)(d[2] >> 32), (uint32_t)(d[3] >> 32), top);
+    uint2 t5;
+    t5.x = top[0];
+    imie_bytes4x4((uint32_t)(d[4] >> 32), (uint32_t)(d[5] >> 32), (uint32_t)(d[6] >> 32), (uint32_t)(d[7] >> 32), top);
+    t5.y = top[0];
+    *(uint2*)(dst + 4 * ls) = t5;
+  }
+  mx = imie_wave_max_u64_full(mx);
+  if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = mx;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < NT / 64; ++w) mx = s_red[w] > mx ? s_red[w] : mx;
+  return mx <= imie_balanced_cap(kQkLimbs) ? imie_limbs_needed(mx) : 0;
+}
+
+// R weight rows (LPR lanes, lane lr of them) against the staged digits of U units at s_x; cur: the lane's first unit
+// of each. Every lane gets the rows' sums. next: called once cur is used up (the caller may refill it and row).
+template <int QT, int LPR, int R, typename Next>
+__device__ inline void g1_rows(const uint8_t* (&row)[R], int lr, int U, G1Raw (&cur)[R], const int8_t* s_x, int ls,
+                               int L, int fw, const int64_t* x, Acc128 (&acc)[R], Next next) {
+#pragma unroll
+  for (int r = 0; r < R; ++r) acc[r] = Acc128{0, 0};
+  if (L == 0) {                                       // a wide row
+    for (int u = lr; u < U; u += LPR)
+#pragma unroll
+      for (int r = 0; r < R; ++r) g1_wide(row[r], u, QT, fw, x, &acc[r]);
+    next();
+  }
+  for (int u = lr; L && u - lr < U; u += LPR) {       // every lane walks the same steps; past the end: no product
+    G1W w[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) w[r] = g1_unpack<QT>(cur[r], u & 3, fw);
+    if (u - lr + LPR < U) {
+#pragma unroll
+      for (int r = 0; r < R; ++r) cur[r] = g1_load<QT>(row[r], u + LPR < U ? u + LPR : 0);
+    } else {
+      next();                                         // the caller's next rows, requested before this step's products
+    }
+    if (u < U) g1_dot<QT, R>(w, s_x + u * kG1Unit, ls, L, acc);
+  }
+  auto add = [&](Acc128& a, uint64_t lo, uint64_t hi) {
+    a.lo += lo;
+    a.hi += (int64_t)hi + (a.lo < lo ? 1 : 0);
+  };
+  static_assert(LPR == 16 || LPR == 32, "one or two DPP rows");
+#pragma unroll
+  for (int r = 0; r < R; ++r) {                       // xor 1, xor 2, half-row mirror, row mirror, xor 16
+    add(acc[r], imie_dpp64<0xB1>(acc[r].lo), imie_dpp64<0xB1>((uint64_t)acc[r].hi));
+    add(acc[r], imie_dpp64<0x4E>(acc[r].lo), imie_dpp64<0x4E>((uint64_t)acc[r].hi));
+    add(acc[r], imie_dpp64<0x141>(acc[r].lo), imie_dpp64<0x141>((uint64_t)acc[r].hi));
+    add(acc[r], imie_dpp64<0x140>(acc[r].lo), imie_dpp64<0x140>((uint64_t)acc[r].hi));
+    if (LPR == 32)
+      add(acc[r], (uint64_t)__shfl_xor((long long)acc[r].lo, 16, 64), (uint64_t)__shfl_xor((long long)acc[r].hi, 16, 64));
+  }
+}
+
+struct G1Item {
+  const uint8_t* w;
+  int64_t* y;
+  int64_t out_f;
+  int qtype, wg0;           // first workgroup of the item
+};
+struct G1Args {
+  G1Item it[kG1Items];
+  const int64_t* x;
+  int* status;
+  int cnt, nb, fw;
+};
+
+template <int QT>
+__device__ inline void g1_linear(const G1Args& a, const G1Item& it, int8_t* s_x, uint64_t* s_red) {
+  const int lane = threadIdx.x & 63, l32 = lane & 31, U = 4 * a.nb;
+  const int64_t o0 = ((int64_t)(blockIdx.x - it.wg0) * 8 + (threadIdx.x >> 5)) * kG1Rows;
+  const int64_t rb = (int64_t)a.nb * (QT == 0 ? 144 : 210);
+  const uint8_t* row[kG1Rows];
+  G1Raw first[kG1Rows];
+#pragma unroll
+  for (int r = 0; r < kG1Rows; ++r) {                 // requested before the digits are formed; past the end: row 0
+    row[r] = it.w + (o0 + r < it.out_f ? o0 + r : 0) * rb;
+    first[r] = g1_load<QT>(row[r], l32 < U ? l32 : 0);
+  }
+  const int L = g1_stage<256>(a.x, 64 * U, s_x, s_red);
+  Acc128 acc[kG1Rows];
+  g1_rows<QT, 32, kG1Rows>(row, l32, U, first, s_x, U * kG1Unit, L, a.fw, a.x, acc, [] {});
+#pragma unroll
+  for (int r = 0; r < kG1Rows; ++r)
+    if (l32 == r && o0 + r < it.out_f) {
+      bool fits;
+      it.y[o0 + r] = acc_shift(acc[r], a.fw, &fits);
+      if (!fits) atomicOr(a.status, IMIE_EOVF);
+    }
+}
+
+__global__ __launch_bounds__(256) void qk_gemv1_kernel(G1Args a) {
+  extern __shared__ __align__(16) int8_t s_x[];
+  __shared__ uint64_t s_red[4];
+  int i = 0;
+  while (i + 1 < a.cnt && (int)blockIdx.x >= a.it[i + 1].wg0) ++i;
+  if (a.it[i].qtype == 0) g1_linear<0>(a, a.it[i], s_x, s_red);
+  else g1_linear<1>(a, a.it[i], s_x, s_red);
+}
+
+// The MoE block of a few tokens (Q4_K gate / up, Q6_K down) in two launches: gate, up and SiLU(g) u per (pair, row) --
+// the gate row in one half of the wave, the up row in the other --, then down and the gated sum over a token's
+// experts, with the residual of the retained layer chain added when `res` is given. The expert pointers are kernel
+// arguments. Each pair reads its expert's weights, so up to kMoe1Pairs pairs, where few experts repeat. Bound by VALU
+// (about 500 instructions a weight row pair and half wave at one to two waves per SIMD), 13 + 12 us for one token's
+// eight experts of 768 at hidden 2048, where the grouped form's seven launches took 18 + 10 + 20 us.
+constexpr int kMoe1Pairs = 32;
+constexpr int kMoe1Rows = 2;       // weight rows per lane group
+constexpr int kMoe1Wave = 4;       // gate and up rows of a wave (one SiLU pass for all of them)
+constexpr int kMoe1Out = 8;        // output rows of a down workgroup
+constexpr int kMoe1MaxK = 16;      // experts of a token
+struct Moe1Args {
+  const uint8_t* w[3][kMoe1Pairs];
+  const int64_t *h, *gates;
+  int64_t *gu, *out;
+  const int64_t *res, *ao;
+  int k, d_model, e_ffn, fa, fw;
+  int64_t log2e, dclip;
+  int* status;
+};
+
+__global__ __launch_bounds__(256) void moe1_gateup_kernel(Moe1Args a) {
+  extern __shared__ __align__(16) int8_t s_x[];
+  __shared__ uint64_t s_red[4];
+  const int p = blockIdx.y, lane = threadIdx.x & 63, l32 = lane & 31;
+  const int o0 = ((int)blockIdx.x * 4 + (int)(threadIdx.x >> 6)) * kMoe1Wave, U = a.d_model / 64;
+  const uint8_t* w = lane < 32 ? a.w[0][p] : a.w[1][p];
+  const int64_t rb = (int64_t)(a.d_model / 256) * 144;
+  const int64_t* x = a.h + (int64_t)(p / a.k) * a.d_model;
+  const uint8_t* row[kMoe1Rows];
+  G1Raw cur[kMoe1Rows];
+  auto fetch = [&](int o) {
+#pragma unroll
+    for (int r = 0; r < kMoe1Rows; ++r) {             // rows past the end: the last one again, not stored
+      row[r] = w + (o + r < a.e_ffn ? o + r : a.e_ffn - 1) * rb;
+      cur[r] = g1_load<0>(row[r], l32 < U ? l32 : 0);
+    }
+  };
+  fetch(o0);
+  const int L = g1_stage<256>(x, a.d_model, s_x, s_red);
+  int64_t mine = 0;
+  bool good = true;
+#pragma unroll 1
+  for (int i = 0; i < kMoe1Wave; i += kMoe1Rows) {
+    Acc128 acc[kMoe1Rows];
+    g1_rows<0, 32, kMoe1Rows>(row, l32, U, cur, s_x, U * kG1Unit, L, a.fw, x, acc,
+                              [&] { if (i + kMoe1Rows < kMoe1Wave) fetch(o0 + i + kMoe1Rows); });
+#pragma unroll
+    for (int r = 0; r < kMoe1Rows; ++r)
+      if (l32 == i + r) {                             // lanes r / 32 + r keep row r's gate / up
+        bool fits;
+        mine = acc_shift(acc[r], a.fw, &fits);
+        good = fits;
+      }
+  }
+  const int64_t u = (int64_t)__shfl_xor((long long)mine, 32, 64);
+  if (lane < kMoe1Wave && o0 + lane < a.e_ffn) {
+    bool ok;
+    a.gu[(int64_t)p * a.e_ffn + o0 + lane] = nmc_silu_mul(mine, u, a.fa, a.log2e, a.dclip, &ok);
+    good = good && ok;
+  }
+  if (!good) atomicOr(a.status, IMIE_EOVF);
+}
+
+__global__ __launch_bounds__(512) void moe1_down_kernel(Moe1Args a) {
+  extern __shared__ __align__(16) int8_t s_x[];
+  __shared__ uint64_t s_red[8];
+  __shared__ int64_t s_d[kMoe1Out][kMoe1MaxK];
+  const int t = blockIdx.y, l16 = threadIdx.x & 15, grp = threadIdx.x >> 4;
+  const int o0 = (int)blockIdx.x * kMoe1Out, U = a.e_ffn / 64;
+  // a job: kMoe1Rows output rows of one expert, 16 lanes; 32 jobs at a time (all of them for eight experts)
+  constexpr int kPer = kMoe1Out / kMoe1Rows;
+  const int jobs = kPer * a.k;
+  const int64_t rb = (int64_t)(a.e_ffn / 256) * 210;
+  const int64_t* x = a.gu + (int64_t)t * a.k * a.e_ffn;
+  const uint8_t* row[kMoe1Rows];
+  G1Raw first[kMoe1Rows];
+  auto fetch = [&](int job) {
+    const uint8_t* w = a.w[2][t * a.k + job / kPer] + (int64_t)(o0 + (job % kPer) * kMoe1Rows) * rb;
+#pragma unroll
+    for (int r = 0; r < kMoe1Rows; ++r) {
+      row[r] = w + r * rb;
+      first[r] = g1_load<1>(row[r], l16 < U ? l16 : 0);
+    }
+  };
+  fetch(grp < jobs ? grp : 0);
+  const int L = g1_stage<512>(x, a.k * a.e_ffn, s_x, s_red);
+  for (int job = grp; job < jobs; job += 32) {
+    const int e = job / kPer;
+    Acc128 acc[kMoe1Rows];
+    g1_rows<1, 16, kMoe1Rows>(row, l16, U, first, s_x + e * U * kG1Unit, a.k * U * kG1Unit, L, a.fw,
+                              x + (int64_t)e * a.e_ffn, acc, [&] { if (job + 32 < jobs) fetch(job + 32); });
+#pragma unroll
+    for (int r = 0; r < kMoe1Rows; ++r)
+      if (l16 == r) {
+        bool fits;
+        s_d[(job % kPer) * kMoe1Rows + r][e] = acc_shift(acc[r], a.fw, &fits);
+        if (!fits) atomicOr(a.status, IMIE_EOVF);
+      }
+  }
+  __syncthreads();
+  if (threadIdx.x < kMoe1Out) {
+    i128 acc = 0;
+    for (int j = 0; j < a.k; ++j) acc += ((i128)s_d[threadIdx.x][j] * a.gates[t * a.k + j]) >> a.fa;
+    if (acc > (i128)INT64_MAX || acc < (i128)INT64_MIN) atomicOr(a.status, IMIE_EOVF);
+    const int64_t i = (int64_t)t * a.d_model + o0 + threadIdx.x;
+    uint64_t y = (uint64_t)acc;
+    if (a.res) y += (uint64_t)a.res[i] + (uint64_t)a.ao[i];   // int64 wrap, as the committed numpy addition
+    a.out[i] = (int64_t)y;
+  }
+}
+
 bool qk_mfma_enabled() {
   static const bool v = [] { const char* e = getenv("IMIE_QK_MFMA"); return !(e && atoi(e) == 0); }();
   return v;
@@ -1234,6 +1700,26 @@ bool qk_mfma_enabled() {
 const QKWeight* qk_get(int64_t h) {
   if (h < 0 || h >= (int64_t)g_qk.size() || !g_qk[(size_t)h].p || g_qk[(size_t)h].qtype > 1) return nullptr;
   return &g_qk[(size_t)h];
+}
+
+// One activation row against up to kG1Items weights of the same input width, in one launch (qk_gemv1_kernel).
+bool gemv1_ok(int64_t nb) { return nb <= kG1MaxNb && qk_mfma_enabled(); }
+
+int gemv1_launch(const QKWeight* const* ws, int64_t* const* ys, int cnt, const int64_t* x, int fw, int* status,
+                 hipStream_t st) {
+  G1Args a = {};
+  a.x = x; a.status = status; a.cnt = cnt; a.nb = (int)ws[0]->nb; a.fw = fw;
+  int64_t wgs = 0;
+  for (int i = 0; i < cnt; ++i) {
+    a.it[i] = G1Item{ws[i]->p, ys[i], ws[i]->out_f, ws[i]->qtype, (int)wgs};
+    wgs += (ws[i]->out_f + 8 * kG1Rows - 1) / (8 * kG1Rows);
+  }
+  if (wgs > INT32_MAX) return IMIE_EARG;
+  imie_prof_mark(IMIE_K_QK, st, true);
+  hipLaunchKernelGGL(qk_gemv1_kernel, dim3((unsigned)wgs), dim3(256), (size_t)kQkLimbs * 4 * a.nb * kG1Unit, st, a);
+  imie_prof_mark(IMIE_K_QK, st, false);
+  IMIE_HIP(hipGetLastError());
+  return IMIE_OK;
 }
 
 // Enqueue a set of items over device X (rows x K) into device Y (rows x ldy). pairs: host arrays. The int8-MFMA
@@ -1362,6 +1848,38 @@ int moe_batched_items(const long long* gate_h, const long long* up_h, const long
   return IMIE_OK;
 }
 
+// A few tokens take moe1_gateup_kernel / moe1_down_kernel (every pair reads its expert's weights, no item lists, two
+// launches); more tokens share decoded weights in the grouped kernels below. At 128 experts of 768, top-8, hidden 2048,
+// this form against the grouped one for 1, 2, 3, 4 tokens: 23.5 / 41.3, 39 / 44.5, 57.5 / 58.6, 72 / 65 us.
+constexpr int kMoe1Tokens = 2;
+bool moe1_ok(int64_t m, int64_t k, int64_t d_model, int64_t e_ffn) {
+  return m <= kMoe1Tokens && k <= kMoe1MaxK && m * k <= kMoe1Pairs && d_model / 256 <= kG1MaxNb &&
+         k * (e_ffn / 256) <= kG1MaxNb && d_model % kMoe1Out == 0;
+}
+
+// handles already checked by the caller; res, ao: the residual and attention rows to add (both or none)
+int moe1_launch(const long long* gate_h, const long long* up_h, const long long* down_h, int m, int k,
+                const int64_t* h_dev, const int64_t* gates_dev, int64_t d_model, int64_t e_ffn, int fa, int fw,
+                int64_t* out_dev, const int64_t* res, const int64_t* ao, int* status, hipStream_t st) {
+  Moe1Args a = {};
+  for (int p = 0; p < m * k; ++p) {
+    a.w[0][p] = qk_get(gate_h[p])->p;
+    a.w[1][p] = qk_get(up_h[p])->p;
+    a.w[2][p] = qk_get(down_h[p])->p;
+  }
+  a.h = h_dev; a.gates = gates_dev; a.gu = (int64_t*)g_mws.g.p; a.out = out_dev; a.res = res; a.ao = ao;
+  a.k = k; a.d_model = (int)d_model; a.e_ffn = (int)e_ffn; a.fa = fa; a.fw = fw; a.status = status;
+  silu_consts_nmc(fa, &a.log2e, &a.dclip);
+  imie_prof_mark(IMIE_K_QK, st, true);
+  hipLaunchKernelGGL(moe1_gateup_kernel, dim3((unsigned)((e_ffn + 4 * kMoe1Wave - 1) / (4 * kMoe1Wave)), (unsigned)(m * k)), dim3(256),
+                     (size_t)kQkLimbs * (d_model / 64) * kG1Unit, st, a);
+  hipLaunchKernelGGL(moe1_down_kernel, dim3((unsigned)(d_model / kMoe1Out), (unsigned)m), dim3(512),
+                     (size_t)kQkLimbs * k * (e_ffn / 64) * kG1Unit, st, a);
+  imie_prof_mark(IMIE_K_QK, st, false);
+  IMIE_HIP(hipGetLastError());
+  return IMIE_OK;
+}
+
 // Batched MoE with the fused expert kernels (Q4_K gate/up, Q6_K down): one item per expert, its pairs listed
 // once. Sequence: prep(h) -> gate/up + SiLU*up -> prep(gu) -> down -> combine. When an activation row needs more
 // than kQkLimbs digit limbs, the prep sets a device flag: the fused kernels return at once and the exact VALU item
@@ -1386,6 +1904,11 @@ int moe_batched(const long long* gate_h, const long long* up_h, const long long*
     if (g->out_f != e_ffn || g->nb * 256 != d_model || u->out_f != e_ffn || u->nb * 256 != d_model ||
         d->out_f != d_model || d->nb * 256 != e_ffn)
       return IMIE_EARG;
+  }
+  if (moe1_ok(m, k, d_model, e_ffn)) {
+    if (g_mws.g.ensure((size_t)(P * e_ffn) * 8) || g_mws.status.ensure(64)) return IMIE_EARG;
+    return moe1_launch(gate_h, up_h, down_h, m, k, h_dev, gates_dev, d_model, e_ffn, fa, fw, out_dev, nullptr, nullptr,
+                       (int*)g_mws.status.p, st);
   }
   if (g_mws.g.ensure((size_t)(P * e_ffn) * 8) || g_mws.u.ensure((size_t)(P * e_ffn) * 8) ||
       g_mws.d.ensure((size_t)(P * d_model) * 8) || g_mws.status.ensure(64))
@@ -1480,8 +2003,22 @@ int host_linear(const std::vector<int64_t>& handles, const int64_t* x, int64_t T
   IMIE_HIP(hipMemsetAsync(g_mws.status.p, 0, 4, st));
   prof(PM_H2D_CALLS); prof(PM_H2D_BYTES, (unsigned long long)(T * K * 8));
   int64_t off = 0;
+  const bool one = T == 1 && gemv1_ok(w0->nb);
+  for (size_t i0 = 0; one && i0 < handles.size(); i0 += kG1Items) {   // one row: all weights in one launch
+    const QKWeight* ws[kG1Items];
+    int64_t* ys[kG1Items];
+    int cnt = 0;
+    for (; cnt < kG1Items && i0 + cnt < handles.size(); ++cnt) {
+      ws[cnt] = qk_get(handles[i0 + cnt]);
+      ys[cnt] = (int64_t*)g_mws.y.p + off;
+      off += ws[cnt]->out_f;
+    }
+    const int rc = gemv1_launch(ws, ys, cnt, (const int64_t*)g_mws.x.p, fw, (int*)g_mws.status.p, st);
+    if (rc) return rc;
+  }
   static DevBuf ib, pb;
   for (auto h : handles) {
+    if (one) break;
     const QKWeight* w = qk_get(h);
     std::vector<Item> items{Item{w->p, w->out_f, w->nb, w->qtype, 0, (int)T}};
     std::vector<int> xi((size_t)T), yi((size_t)T);
@@ -1544,6 +2081,7 @@ int64_t imie_qk_register_i64(const int64_t* W, int64_t rows, int64_t cols) {
 int imie_qk_linear_dev(int64_t h, const int64_t* x, int64_t T, int fw, int64_t* out, int* status, hipStream_t st) {
   const QKWeight* w = qk_get(h);
   if (!w || !x || !out || !status || T <= 0) return IMIE_EARG;
+  if (T == 1 && gemv1_ok(w->nb)) return gemv1_launch(&w, &out, 1, x, fw, status, st);
   std::vector<Item> items{Item{w->p, w->out_f, w->nb, w->qtype, 0, (int)T}};
   std::vector<int> xi((size_t)T), yi((size_t)T);
   for (int64_t t = 0; t < T; ++t) { xi[(size_t)t] = (int)t; yi[(size_t)t] = (int)t; }
@@ -1553,18 +2091,50 @@ int imie_qk_linear_dev(int64_t h, const int64_t* x, int64_t T, int fw, int64_t* 
   return run_items(items, xi, yi, x, w->nb * 256, out, w->out_f, fw, status, st, ib[slot], pb[slot]);
 }
 
-// one token's MoE over k selected experts (host handle arrays), gates on the device; synchronous; 0, or IMIE_EOVF
-// where the oracle's int64 conversions would raise
+// one row against cnt weights of the same input width (the Q / K / V projections of one token)
+int imie_qk_linears_dev(const int64_t* hs, int cnt, const int64_t* x, int fw, int64_t* const* outs, int* status,
+                        hipStream_t st) {
+  const QKWeight* ws[kG1Items];
+  bool one = cnt <= kG1Items;
+  for (int i = 0; i < cnt && one; ++i) {
+    if (!(ws[i] = qk_get(hs[i]))) return IMIE_EARG;
+    one = ws[i]->nb == ws[0]->nb && gemv1_ok(ws[i]->nb);
+  }
+  if (one) return gemv1_launch(ws, outs, cnt, x, fw, status, st);
+  for (int i = 0; i < cnt; ++i) {
+    const int rc = imie_qk_linear_dev(hs[i], x, 1, fw, outs[i], status, st);
+    if (rc) return rc;
+  }
+  return IMIE_OK;
+}
+
+// One token's MoE over k selected experts (host handle arrays), gates on the device, and the layer's residual:
+// out = res + ao + moe (int64 wrap). Enqueued on st (no synchronisation); *status_dev gets IMIE_EOVF where the
+// oracle's int64 conversions would raise.
 int imie_qk_moe_dev(const long long* gate_h, const long long* up_h, const long long* down_h, int k,
                     const int64_t* h_dev, const int64_t* gates_dev, int64_t d_model, int64_t e_ffn, int fa, int fw,
-                    int64_t* out_dev, hipStream_t st) {
+                    const int64_t* res, const int64_t* ao, int64_t* moe, int64_t* out_dev, int* status_dev,
+                    hipStream_t st) {
+  bool small = fw <= kMaxFw && qk_mfma_enabled() && moe1_ok(1, k, d_model, e_ffn) && d_model % 256 == 0 &&
+               e_ffn % 256 == 0 && fa >= 1 && fa <= 28 && fw >= 0;
+  for (int p = 0; p < k && small; ++p) {
+    const QKWeight *g = qk_get(gate_h[p]), *u = qk_get(up_h[p]), *d = qk_get(down_h[p]);
+    if (!g || !u || !d) return IMIE_EARG;
+    small = g->qtype == 0 && u->qtype == 0 && d->qtype == 1;
+  }
+  if (small) {                                        // shapes are those of the layer (checked when it was bound)
+    if (g_mws.g.ensure((size_t)(k * e_ffn) * 8)) return IMIE_EARG;
+    return moe1_launch(gate_h, up_h, down_h, 1, k, h_dev, gates_dev, d_model, e_ffn, fa, fw, out_dev, res, ao,
+                       status_dev, st);
+  }
   if (g_mws.status.ensure(64)) return IMIE_EARG;
-  IMIE_HIP(hipMemsetAsync(g_mws.status.p, 0, 4, st));
-  int rc = moe_batched(gate_h, up_h, down_h, 1, k, h_dev, gates_dev, d_model, e_ffn, fa, fw, out_dev, st);
+  hipLaunchKernelGGL(qk_flag_reset_kernel, dim3(1), dim3(1), 0, st, (int*)g_mws.status.p);
+  const int rc = moe_batched(gate_h, up_h, down_h, 1, k, h_dev, gates_dev, d_model, e_ffn, fa, fw, moe, st);
   if (rc) return rc;
-  int stat = 0;
-  if (read_status_and(st, &stat)) return IMIE_EARG;
-  return stat ? IMIE_EOVF : IMIE_OK;
+  hipLaunchKernelGGL(qk_add3_kernel, dim3((unsigned)((d_model + 255) / 256)), dim3(256), 0, st, res, ao, moe, d_model,
+                     out_dev, (const int*)g_mws.status.p, status_dev);
+  IMIE_HIP(hipGetLastError());
+  return IMIE_OK;
 }
 
 extern "C" {

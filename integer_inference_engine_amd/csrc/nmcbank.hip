@@ -18,9 +18,12 @@
 int imie_qk_info(int64_t h, int64_t* out_f, int64_t* nb, int* qtype, const uint8_t** p);
 int64_t imie_qk_register_i64(const int64_t* W, int64_t rows, int64_t cols);
 int imie_qk_linear_dev(int64_t h, const int64_t* x, int64_t T, int fw, int64_t* out, int* status, hipStream_t st);
+int imie_qk_linears_dev(const int64_t* hs, int cnt, const int64_t* x, int fw, int64_t* const* outs, int* status,
+                        hipStream_t st);
 int imie_qk_moe_dev(const long long* gate_h, const long long* up_h, const long long* down_h, int k,
                     const int64_t* h_dev, const int64_t* gates_dev, int64_t d_model, int64_t e_ffn, int fa, int fw,
-                    int64_t* out_dev, hipStream_t st);
+                    const int64_t* res, const int64_t* ao, int64_t* moe, int64_t* out_dev, int* status_dev,
+                    hipStream_t st);
 
 namespace {
 
@@ -91,87 +94,108 @@ __global__ __launch_bounds__(256) void nb_router_kernel(const int64_t* __restric
   const int e = blockIdx.x;
   const int64_t* hr = h + row * width;
   const int64_t* wr = W + (int64_t)e * width;
-  uint64_t mh = 0, mw = 0;
+  // one pass: the wrapping sum and both maxima together (the sum counts only where the maxima say it is exact)
+  __shared__ uint64_t s_h[4], s_w[4];
+  uint64_t mh = 0, mw = 0, acc = 0;
+#pragma unroll 8
   for (int64_t i = threadIdx.x; i < width; i += 256) {
-    const uint64_t a = nb_uabs(hr[i]), b = nb_uabs(wr[i]);
+    const int64_t hv = hr[i], wv = wr[i];
+    const uint64_t a = nb_uabs(hv), b = nb_uabs(wv);
     mh = a > mh ? a : mh;
     mw = b > mw ? b : mw;
+    acc += (uint64_t)hv * (uint64_t)wv;
   }
-  mh = nb_block_max(mh);
-  mw = nb_block_max(mw);
-  const bool fast = mh == 0 || mw == 0 || (u128)mh * mw * (u128)(uint64_t)width <= (u128)INT64_MAX;
-  if (fast) {
-    int64_t acc = 0;
-    for (int64_t i = threadIdx.x; i < width; i += 256) acc += hr[i] * wr[i];
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) acc += (int64_t)__shfl_xor((long long)acc, o, 64);
-    __syncthreads();
-    if ((threadIdx.x & 63) == 0) s_sum[threadIdx.x >> 6] = acc;
-    __syncthreads();
-    if (threadIdx.x == 0) logits[row * experts + e] = (s_sum[0] + s_sum[1] + s_sum[2] + s_sum[3]) >> fw;
+  mh = imie_wave_max_u64_full(mh);
+  mw = imie_wave_max_u64_full(mw);
+  acc = imie_wave_sum_u64_full(acc);
+  if ((threadIdx.x & 63) == 0) {
+    const int w = threadIdx.x >> 6;
+    s_h[w] = mh;
+    s_w[w] = mw;
+    s_sum[w] = (int64_t)acc;
+  }
+  __syncthreads();
+  if (threadIdx.x) return;
+  for (int w = 1; w < 4; ++w) {
+    mh = s_h[w] > mh ? s_h[w] : mh;
+    mw = s_w[w] > mw ? s_w[w] : mw;
+    acc += (uint64_t)s_sum[w];
+  }
+  if (mh == 0 || mw == 0 || (u128)mh * mw * (u128)(uint64_t)width <= (u128)INT64_MAX) {
+    logits[row * experts + e] = (int64_t)acc >> fw;
     return;
   }
-  if (threadIdx.x) return;
   const i128 mx = (i128)(((u128)1 << 127) - 1), mn = -mx - 1;
-  i128 acc = 0;
+  i128 sum = 0;
   for (int64_t i = 0; i < width; ++i) {
     const i128 t = (i128)hr[i] * wr[i];
-    if ((t > 0 && acc > mx - t) || (t < 0 && acc < mn - t)) {
+    if ((t > 0 && sum > mx - t) || (t < 0 && sum < mn - t)) {
       atomicOr(status, kGuard);
       logits[row * experts + e] = 0;
       return;
     }
-    acc += t;
+    sum += t;
   }
-  if (acc > (i128)INT64_MAX || acc < (i128)INT64_MIN) {
+  if (sum > (i128)INT64_MAX || sum < (i128)INT64_MIN) {
     atomicOr(status, kGuard);
     logits[row * experts + e] = 0;
     return;
   }
-  logits[row * experts + e] = (int64_t)acc >> fw;
+  logits[row * experts + e] = (int64_t)sum >> fw;
 }
 
 // lowest-index top-k by logit and their sigmoid gates (cohere2.py:162-165, :181-182); one wave per row. The order
 // (logit descending, index ascending) is total, so pick k is the first element of that order behind pick k - 1: a
-// wave maximum over the lanes' strided elements per pick, and no list of the taken ones. Bound by the latency of its
-// `used` reductions; the gates are formed by one lane each at the end. (One thread per row scanning every logit
-// for every pick took 467 us at 128 experts, top-8; this takes 12.)
+// wave maximum over the lanes' strided elements, then the lowest index that holds it from the lanes' ballots; no list
+// of the taken ones. Bound by the latency of its `used` reductions (DPP, no LDS); lane k forms gate k at the end.
+// (One thread per row scanning every logit for every pick took 467 us at 128 experts, top-8; this takes 10.)
 __global__ __launch_bounds__(64) void nb_topk_kernel(const int64_t* __restrict__ logits, int experts, int used, int fa,
                                                      int* __restrict__ ids, int64_t* __restrict__ gates) {
   const int64_t r = blockIdx.x;
   const int lane = threadIdx.x;
   const int64_t* lr = logits + r * experts;
-  constexpr int kKeep = 4;                            // logits kept in registers: 256 experts without a reload
-  int64_t v[kKeep];
+  constexpr uint64_t kSign = (uint64_t)1 << 63;       // logits as unsigned keys in the same order
+  constexpr int kKeep = 4;                            // keys kept in registers: 256 experts without a reload
+  uint64_t v[kKeep];
 #pragma unroll
-  for (int i = 0; i < kKeep; ++i) v[i] = lane + 64 * i < experts ? lr[lane + 64 * i] : 0;
-  int64_t prev = 0;
+  for (int i = 0; i < kKeep; ++i) v[i] = lane + 64 * i < experts ? (uint64_t)lr[lane + 64 * i] ^ kSign : 0;
+  const int ni = (experts + 63) / 64;
+  uint64_t prev = 0;
   int prev_id = -1;
-  for (int k = 0; k < used; ++k) {
-    int64_t best = INT64_MIN;
-    int best_id = INT_MAX;                            // none yet
-    auto take = [&](int64_t x, int e) {
-      const bool behind = prev_id < 0 || x < prev || (x == prev && e > prev_id);
-      if (e < experts && behind && (best_id == INT_MAX || x > best)) { best = x; best_id = e; }
-    };
+  for (int k0 = 0; k0 < used; k0 += 64) {
+    int64_t mine = 0;
+    for (int k = k0; k < used && k < k0 + 64; ++k) {
+      auto behind = [&](uint64_t x, int e) {
+        return e < experts && (prev_id < 0 || x < prev || (x == prev && e > prev_id));
+      };
+      uint64_t best = 0;                              // 0: the lowest key, so also the value of "none" in the maximum
 #pragma unroll
-    for (int i = 0; i < kKeep; ++i) take(v[i], lane + 64 * i);
-    for (int e = lane + 64 * kKeep; e < experts; e += 64) take(lr[e], e);
+      for (int i = 0; i < kKeep; ++i) best = behind(v[i], lane + 64 * i) && v[i] > best ? v[i] : best;
+      for (int i = kKeep; i < ni; ++i) {
+        const int e = lane + 64 * i;
+        const uint64_t x = e < experts ? (uint64_t)lr[e] ^ kSign : 0;
+        best = behind(x, e) && x > best ? x : best;
+      }
+      best = imie_wave_max_u64_full(best);
+      int id = -1;
 #pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) {
-      const int64_t x = (int64_t)__shfl_xor((long long)best, o, 64);
-      const int e = __shfl_xor(best_id, o, 64);
-      if (e != INT_MAX && (best_id == INT_MAX || x > best || (x == best && e < best_id))) { best = x; best_id = e; }
+      for (int i = 0; i < kKeep; ++i) {
+        const uint64_t b = __ballot(behind(v[i], lane + 64 * i) && v[i] == best);
+        if (id < 0 && b) id = 64 * i + __builtin_ctzll(b);
+      }
+      for (int i = kKeep; i < ni && id < 0; ++i) {
+        const int e = lane + 64 * i;
+        const uint64_t x = e < experts ? (uint64_t)lr[e] ^ kSign : 0;
+        const uint64_t b = __ballot(behind(x, e) && x == best);
+        if (b) id = 64 * i + __builtin_ctzll(b);
+      }
+      prev = best;
+      prev_id = id;
+      if (lane == 0) ids[r * used + k] = id;
+      if (lane == k - k0) mine = (int64_t)(best ^ kSign);
     }
-    prev = best;
-    prev_id = best_id;
-    if (lane == 0) {
-      ids[r * used + k] = best_id;
-      gates[r * used + k] = best;
-    }
+    if (k0 + lane < used) gates[r * used + k0 + lane] = nb_sigmoid(mine, fa);
   }
-  __syncthreads();                                    // lane 0's logits are visible to the lanes that squash them
-  for (int k = lane; k < used; k += 64) gates[r * used + k] = nb_sigmoid(gates[r * used + k], fa);
 }
 
 // Interleaved RoPE of q (in place) and k, the K / V append at `pos` (cache [Hkv][max_len][hd]) and the running
@@ -575,13 +599,6 @@ __global__ __launch_bounds__(256) void nb_attention_wide_kernel(NbAttn a) {
   }
 }
 
-// next = residual + attention + moe, int64 wrap (the reference's committed numpy int64 addition)
-__global__ void nb_add3_kernel(const int64_t* __restrict__ a, const int64_t* __restrict__ b,
-                               const int64_t* __restrict__ c, int64_t n, int64_t* __restrict__ out) {
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) out[i] = (int64_t)((uint64_t)a[i] + (uint64_t)b[i] + (uint64_t)c[i]);
-}
-
 struct Binding { long long g = -1, u = -1, d = -1; bool bound = false; };
 
 struct Layer {
@@ -600,9 +617,12 @@ struct Bank {
   int64_t max_len = 0, d_model = 0;
   DevBuf cos, sin;
   std::vector<Layer> layers;
-  DevBuf res[2], norm, logits, ids, gates, attn, qkv, ao, prob, part, status, moe;
+  DevBuf res[2], norm, logits, gates, attn, qkv, ao, prob, part, status, moe;
   int res_slot = 0;
   bool has_res = false;
+  bool status_clear = false;                          // the device status word is known to be 0
+  char* host = nullptr;                               // pinned: status, ids and hidden row as read back
+  size_t host_cap = 0;
   int retained = -1;
   bool pending = false;
   int pending_layer = -1;
@@ -635,7 +655,7 @@ int ensure_layer_kv(Bank& b, Layer& L) {
 
 size_t bank_bytes(const Bank& b) {
   size_t t = b.cos.cap + b.sin.cap;
-  for (const DevBuf* d : {&b.res[0], &b.res[1], &b.norm, &b.logits, &b.ids, &b.gates, &b.attn, &b.qkv, &b.ao, &b.prob,
+  for (const DevBuf* d : {&b.res[0], &b.res[1], &b.norm, &b.logits, &b.gates, &b.attn, &b.qkv, &b.ao, &b.prob,
                           &b.part, &b.status, &b.moe})
     t += d->cap;
   for (const Layer& L : b.layers) t += L.k.cap + L.v.cap + L.kvmax.cap;
@@ -645,12 +665,26 @@ size_t bank_bytes(const Bank& b) {
 void bank_release(Bank& b) {
   (void)hipStreamSynchronize(imie_stream());
   for (Layer& L : b.layers) { L.k.release(); L.v.release(); L.kvmax.release(); }
-  for (DevBuf* d : {&b.cos, &b.sin, &b.res[0], &b.res[1], &b.norm, &b.logits, &b.ids, &b.gates, &b.attn, &b.qkv,
+  for (DevBuf* d : {&b.cos, &b.sin, &b.res[0], &b.res[1], &b.norm, &b.logits, &b.gates, &b.attn, &b.qkv,
                     &b.ao, &b.prob, &b.part, &b.status, &b.moe})
     d->release();
+  if (b.host) (void)hipHostFree(b.host);
   b = Bank();
 }
 
+// What the host waits for (n 8-byte words), written straight into its pinned buffer: one small launch and one
+// synchronisation where a copy into pageable memory takes a staging copy of its own.
+__global__ void nb_publish_kernel(const uint64_t* __restrict__ src, int n, uint64_t* __restrict__ dst) {
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) dst[i] = src[i];
+}
+
+// The bank's status word (b.status), followed by the routed expert ids. It is zero between calls: a call that
+// leaves it otherwise poisons its layer, and the next one clears it first (a new allocation too).
+constexpr size_t kIdsAt = 64;
+int status_ensure(Bank& b, size_t bytes) {
+  if (b.status.cap < bytes) b.status_clear = false;
+  return b.status.ensure(bytes);
+}
 // validate the attention handles / window and reserve the layer's storage (qk_cuda.py:548-572 envelope)
 int attention_preflight(Bank& b, int layer, long long qh, long long kh, long long vh, long long oh, int window) {
   if (layer < 0 || layer >= b.n_layers || window == 0 || window < -1) return IMIE_EARG;
@@ -665,7 +699,7 @@ int attention_preflight(Bank& b, int layer, long long qh, long long kh, long lon
     return IMIE_EARG;
   if (ensure_layer_kv(b, L) || b.qkv.ensure((size_t)(qw + 2 * kw) * 8) || b.attn.ensure((size_t)qw * 8) ||
       b.ao.ensure((size_t)b.d_model * 8) || b.prob.ensure((size_t)(b.heads * b.max_len) * 8) ||
-      b.part.ensure((size_t)(kNbMaxChunks * (qw + 2 * b.heads)) * 8) || b.status.ensure(64))
+      b.part.ensure((size_t)(kNbMaxChunks * (qw + 2 * b.heads)) * 8) || status_ensure(b, kIdsAt))
     return IMIE_EARG;
   return IMIE_OK;
 }
@@ -678,9 +712,9 @@ int attention_enqueue(Bank& b, int layer, long long qh, long long kh, long long 
   int64_t* q = (int64_t*)b.qkv.p;
   int64_t *k = q + qw, *v = k + kw;
   int* status = (int*)b.status.p;
-  int rc = imie_qk_linear_dev(qh, x, 1, fw, q, status, st);
-  if (!rc) rc = imie_qk_linear_dev(kh, x, 1, fw, k, status, st);
-  if (!rc) rc = imie_qk_linear_dev(vh, x, 1, fw, v, status, st);
+  const int64_t hs[3] = {qh, kh, vh};
+  int64_t* const ys[3] = {q, k, v};
+  const int rc = imie_qk_linears_dev(hs, 3, x, fw, ys, status, st);
   if (rc) return rc;
   hipLaunchKernelGGL(nb_rope_append_kernel, dim3((unsigned)(b.heads + b.nkv)), dim3(128), 0, st, q, b.heads,
                      (const int64_t*)k, (const int64_t*)v, b.hd, (const int64_t*)b.cos.p, (const int64_t*)b.sin.p,
@@ -713,15 +747,37 @@ int attention_enqueue(Bank& b, int layer, long long qh, long long kh, long long 
   return imie_qk_linear_dev(oh, (const int64_t*)b.attn.p, 1, fw, (int64_t*)b.ao.p, status, st);
 }
 
-// status after the enqueued work: 0 ok, 3 a guard fired (layer poisoned), 1 runtime failure
-int finish(Bank& b, Layer& L, hipStream_t st) {
-  int stat = 0;
-  if (hipMemcpyAsync(&stat, b.status.p, 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
-      hipStreamSynchronize(st) != hipSuccess) {
-    L.poisoned = true;
-    return IMIE_EARG;
+int status_begin(Bank& b, hipStream_t st) {
+  if (!b.status_clear) IMIE_HIP(hipMemsetAsync(b.status.p, 0, 4, st));
+  b.status_clear = false;
+  return IMIE_OK;
+}
+
+// status after the enqueued work: 0 ok, 3 a guard fired (layer poisoned), 1 runtime failure; n_ids routed expert ids
+// and a hidden row (d_model words of `row`, to `row_out`) come back with it
+int finish(Bank& b, Layer& L, hipStream_t st, int n_ids = 0, int* ids = nullptr, const int64_t* row = nullptr,
+           int64_t* row_out = nullptr) {
+  const size_t head = (kIdsAt + (size_t)n_ids * 4 + 7) / 8 * 8, bytes = head + (row ? (size_t)b.d_model * 8 : 0);
+  auto fail = [&]() -> int { L.poisoned = true; return IMIE_EARG; };
+  if (b.host_cap < bytes) {
+    if (b.host) (void)hipHostFree(b.host);
+    b.host = nullptr;
+    b.host_cap = 0;
+    if (hipHostMalloc((void**)&b.host, bytes) != hipSuccess) { (void)hipStreamSynchronize(st); return fail(); }
+    b.host_cap = bytes;
   }
+  hipLaunchKernelGGL(nb_publish_kernel, dim3(1), dim3(256), 0, st, (const uint64_t*)b.status.p, (int)(head / 8),
+                     (uint64_t*)b.host);
+  if (row)
+    hipLaunchKernelGGL(nb_publish_kernel, dim3((unsigned)((b.d_model + 255) / 256)), dim3(256), 0, st,
+                       (const uint64_t*)row, (int)b.d_model, (uint64_t*)(b.host + head));
+  if (hipGetLastError() != hipSuccess || hipStreamSynchronize(st) != hipSuccess) return fail();
+  int stat = 0;
+  memcpy(&stat, b.host, 4);
   if (stat) { L.poisoned = true; return 3; }
+  b.status_clear = true;
+  if (n_ids) memcpy(ids, b.host + kIdsAt, (size_t)n_ids * 4);
+  if (row) memcpy(row_out, b.host + head, (size_t)b.d_model * 8);
   return IMIE_OK;
 }
 
@@ -871,11 +927,11 @@ int qk_attention_bank_apply(long long h, int layer, long long qh, long long kh, 
   hipStream_t st = imie_stream();
   Layer& L = b->layers[(size_t)layer];
   IMIE_HIP(hipMemcpyAsync(b->norm.p, x, (size_t)b->d_model * 8, hipMemcpyHostToDevice, st));
-  IMIE_HIP(hipMemsetAsync(b->status.p, 0, 4, st));
-  int rc = attention_enqueue(*b, layer, qh, kh, vh, oh, (const int64_t*)b->norm.p, fw, window, rope, inv_sqrt, st);
+  int rc = status_begin(*b, st);
+  if (rc) return rc;
+  rc = attention_enqueue(*b, layer, qh, kh, vh, oh, (const int64_t*)b->norm.p, fw, window, rope, inv_sqrt, st);
   if (rc) { (void)hipStreamSynchronize(st); L.poisoned = true; return IMIE_EARG; }
-  if ((rc = finish(*b, L, st))) return rc;
-  IMIE_HIP(hipMemcpy(out, b->ao.p, (size_t)b->d_model * 8, hipMemcpyDeviceToHost));
+  if ((rc = finish(*b, L, st, 0, nullptr, (const int64_t*)b->ao.p, out))) return rc;
   ++L.length;
   return IMIE_OK;
 }
@@ -950,7 +1006,7 @@ int qk_attention_bank_moe_begin(long long h, int layer, long long gain_h, long l
   if (attention_preflight(*b, layer, qh, kh, vh, oh, window)) return IMIE_EARG;
   const size_t dm = (size_t)L.d_model;
   if (b->res[0].ensure(dm * 8) || b->res[1].ensure(dm * 8) || b->norm.ensure(dm * 8) ||
-      b->logits.ensure((size_t)L.experts * 8) || b->ids.ensure((size_t)L.used * 4) ||
+      b->logits.ensure((size_t)L.experts * 8) || status_ensure(*b, kIdsAt + (size_t)(L.used + 1) * 4) ||
       b->gates.ensure((size_t)L.used * 8) || b->moe.ensure(dm * 8))
     return IMIE_EARG;
   hipStream_t st = imie_stream();
@@ -960,19 +1016,20 @@ int qk_attention_bank_moe_begin(long long h, int layer, long long gain_h, long l
   }
   const int64_t* resid = (const int64_t*)b->res[b->res_slot].p;
   int* status = (int*)b->status.p;
-  IMIE_HIP(hipMemsetAsync(status, 0, 4, st));
-  int rc = imie_rmsnorm_launch(resid, 1, L.d_model, b->fa, e, (const int64_t*)gp, (int64_t*)b->norm.p, status, st);
+  int* ids = (int*)((char*)b->status.p + kIdsAt);
+  int rc = status_begin(*b, st);
+  if (rc) return rc;
+  rc = imie_rmsnorm_launch(resid, 1, L.d_model, b->fa, e, (const int64_t*)gp, (int64_t*)b->norm.p, status, st);
   if (rc) return rc;
   hipLaunchKernelGGL(nb_router_kernel, dim3((unsigned)L.experts, 1), dim3(256), 0, st, (const int64_t*)b->norm.p,
                      L.d_model, (const int64_t*)rp, L.experts, fw, (int64_t*)b->logits.p, status);
   hipLaunchKernelGGL(nb_topk_kernel, dim3(1), dim3(64), 0, st, (const int64_t*)b->logits.p, L.experts, L.used,
-                     b->fa, (int*)b->ids.p, (int64_t*)b->gates.p);
+                     b->fa, ids, (int64_t*)b->gates.p);
   IMIE_HIP(hipGetLastError());
   rc = attention_enqueue(*b, layer, qh, kh, vh, oh, (const int64_t*)b->norm.p, fw, window, rope, inv_sqrt, st);
   if (rc) { (void)hipStreamSynchronize(st); L.poisoned = true; return IMIE_EARG; }
   b->route_ids.assign((size_t)L.used, -1);
-  IMIE_HIP(hipMemcpyAsync(b->route_ids.data(), b->ids.p, (size_t)L.used * 4, hipMemcpyDeviceToHost, st));
-  if ((rc = finish(*b, L, st))) return rc;
+  if ((rc = finish(*b, L, st, L.used, b->route_ids.data()))) return rc;
   std::vector<int> cold;
   for (int id : b->route_ids) {
     if (id < 0 || id >= L.experts) { L.poisoned = true; return 3; }
@@ -1009,17 +1066,14 @@ int qk_attention_bank_moe_continue(long long h, int layer, int fw, int publish, 
     gh.push_back(bd.g); uh.push_back(bd.u); dh.push_back(bd.d);
   }
   hipStream_t st = imie_stream();
-  int rc = imie_qk_moe_dev(gh.data(), uh.data(), dh.data(), L.used, (const int64_t*)b->norm.p,
-                           (const int64_t*)b->gates.p, L.d_model, L.e_ffn, b->fa, fw, (int64_t*)b->moe.p, st);
-  if (rc == IMIE_EOVF) { L.poisoned = true; return 3; }
-  if (rc) { L.poisoned = true; return IMIE_EARG; }
   const int next = b->res_slot ^ 1;
-  hipLaunchKernelGGL(nb_add3_kernel, dim3((unsigned)((L.d_model + 255) / 256)), dim3(256), 0, st,
-                     (const int64_t*)b->res[b->res_slot].p, (const int64_t*)b->ao.p, (const int64_t*)b->moe.p,
-                     L.d_model, (int64_t*)b->res[next].p);
-  IMIE_HIP(hipGetLastError());
-  if (publish) IMIE_HIP(hipMemcpyAsync(out, b->res[next].p, (size_t)L.d_model * 8, hipMemcpyDeviceToHost, st));
-  IMIE_HIP(hipStreamSynchronize(st));
+  int rc = status_begin(*b, st);
+  if (rc) return rc;
+  rc = imie_qk_moe_dev(gh.data(), uh.data(), dh.data(), L.used, (const int64_t*)b->norm.p, (const int64_t*)b->gates.p,
+                       L.d_model, L.e_ffn, b->fa, fw, (const int64_t*)b->res[b->res_slot].p, (const int64_t*)b->ao.p,
+                       (int64_t*)b->moe.p, (int64_t*)b->res[next].p, (int*)b->status.p, st);
+  if (rc) { (void)hipStreamSynchronize(st); L.poisoned = true; return IMIE_EARG; }
+  if ((rc = finish(*b, L, st, 0, nullptr, publish ? (const int64_t*)b->res[next].p : nullptr, out))) return rc;
   b->res_slot = next; b->has_res = true; b->retained = layer; b->pending = false; b->pending_layer = -1;
   return IMIE_OK;
 }
