@@ -14,7 +14,7 @@ namespace imie_q1 {
 constexpr int kSlabBlocks = 4;     // 128-blocks per slab (= K 512 per wave step)
 constexpr int kMaxLimbs = 8;
 constexpr int kMaxSegs = 3;        // weights sharing one activation in a single matvec launch
-constexpr int kGemmMinT = 8;       // from this many tokens the Q1 linear runs as an MFMA GEMM (own digit layout)
+constexpr int kGemmMinT = 9;        // from this many tokens the Q1 linear runs as an MFMA GEMM (own digit layout)
 
 struct Q1PrepOut {                 // where a prep writes its table (sized for T tokens of nb blocks)
   uint32_t* xq;
@@ -58,6 +58,38 @@ __device__ inline int64_t prep_pos(int lane, int64_t sl, int q) {
   return (sl * kSlabBlocks + g) * 128 + 32 * d + 8 * c + s;
 }
 
+// The balanced digits of the lane's 8 values, limb by limb: put(l, w0, w1) for l < n with the digits of values 0..3 and
+// 4..7 as bytes. mx: the wave's max|v|. Up to four limbs (mx <= 0x7F7F7F7F, any real activation) all digits come from
+// one add and one xor per value and a byte transpose; more take the 64-bit form, four limbs at a time.
+// (Peeling a digit per limb and value in 64 bits was 200 to 300 instructions, this is 40.)
+template <typename Put>
+__device__ inline void prep_digits(const int64_t* v, uint64_t mx, int n, Put put) {
+  uint32_t a[4], b[4];
+  if (mx <= 0x7F7F7F7Full) {
+    uint32_t d[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) d[q] = imie_digits32((uint32_t)(uint64_t)v[q]);
+    imie_bytes4x4(d[0], d[1], d[2], d[3], a);
+    imie_bytes4x4(d[4], d[5], d[6], d[7], b);
+#pragma unroll
+    for (int l = 0; l < 4; ++l)
+      if (l < n) put(l, a[l], b[l]);
+    for (int l = 4; l < n; ++l) put(l, 0u, 0u);
+    return;
+  }
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    uint32_t d[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) d[q] = (uint32_t)(imie_digits64((uint64_t)v[q]) >> (32 * h));
+    imie_bytes4x4(d[0], d[1], d[2], d[3], a);
+    imie_bytes4x4(d[4], d[5], d[6], d[7], b);
+#pragma unroll
+    for (int l = 0; l < 4; ++l)
+      if (4 * h + l < n) put(4 * h + l, a[l], b[l]);
+  }
+}
+
 // v[q] = x at prep_pos(lane, sl, q) (0 for blocks >= nb); every lane of the wave participates.
 __device__ inline void prep_slab(int64_t v[8], const Q1PrepOut& po, int64_t t, int64_t sl) {
   const int lane = threadIdx.x & 63;
@@ -77,18 +109,9 @@ __device__ inline void prep_slab(int64_t v[8], const Q1PrepOut& po, int64_t t, i
   part = (int64_t)imie_row_sum_u64_full((uint64_t)part);
   if ((lane & 15) == 0) po.totals[t * po.nbp + blk] = part;
   if (lane == 0) po.lslab[t * po.nslabs + sl] = L;
-  for (int l = 0; l < L; ++l) {
-    uint32_t w0 = 0, w1 = 0;
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int64_t dig = ((v[q] + 128) & 255) - 128;          // balanced digit in [-128, 127]
-      v[q] = (int64_t)(((uint64_t)v[q] - (uint64_t)dig)) >> 8;  // exact: v - dig is a multiple of 256
-      const uint32_t byte = (uint32_t)(dig & 0xFF) << (8 * (q & 3));
-      if (q < 4) w0 |= byte; else w1 |= byte;
-    }
-    uint32_t* dst = po.xq + ((((t * kMaxLimbs + l) * po.nbp + blk) * 8 + s) * 4);
-    *(uint2*)(dst + 2 * dh) = uint2{w0, w1};
-  }
+  prep_digits(v, mx, L, [&](int l, uint32_t w0, uint32_t w1) {
+    *(uint2*)(po.xq + ((((t * kMaxLimbs + l) * po.nbp + blk) * 8 + s) * 4) + 2 * dh) = uint2{w0, w1};
+  });
 }
 
 // prep_slab into LDS: the slab's limb count, block totals and digits for a workgroup-local table laid out as the
@@ -109,17 +132,9 @@ __device__ inline void prep_slab_lds(int64_t v[8], uint4* dst, int* L_out, int64
   part = (int64_t)imie_row_sum_u64_full((uint64_t)part);
   if ((lane & 15) == 0) tot_out[g] = part;
   if (lane == 0) *L_out = L;
-  for (int l = 0; l < L; ++l) {
-    uint32_t w0 = 0, w1 = 0;
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int64_t dig = ((v[q] + 128) & 255) - 128;
-      v[q] = (int64_t)(((uint64_t)v[q] - (uint64_t)dig)) >> 8;
-      const uint32_t byte = (uint32_t)(dig & 0xFF) << (8 * (q & 3));
-      if (q < 4) w0 |= byte; else w1 |= byte;
-    }
+  prep_digits(v, mx, L, [&](int l, uint32_t w0, uint32_t w1) {
     *(uint2*)((uint32_t*)(dst + l * 32 + g * 8 + s) + 2 * dh) = uint2{w0, w1};
-  }
+  });
 }
 
 // workgroup `wg` of `nwg` clears its share of the zero list (threads tid of nthreads)
@@ -149,19 +164,9 @@ __device__ inline void prep_gemm_slab(int64_t v[8], const GemmPrepOut& gp, int64
   if ((lane & 15) == 0) gp.tg[blk * gp.Tp + t] = part;
   if (lane == 0) gp.lt[t * gp.nslabs + sl] = L;
   const int Lw = L > kGemmNarrowLimbs ? L : kGemmNarrowLimbs;
-  for (int l = 0; l < Lw; ++l) {
-    uint32_t w0 = 0, w1 = 0;
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      const int64_t dig = ((v[q] + 128) & 255) - 128;
-      v[q] = (int64_t)(((uint64_t)v[q] - (uint64_t)dig)) >> 8;
-      const uint32_t byte = (uint32_t)(dig & 0xFF) << (8 * (q & 3));
-      if (q < 4) w0 |= byte; else w1 |= byte;
-    }
-    uint32_t* dst = (uint32_t*)(gp.xg + ((l * gp.nbp + blk) * gp.Tp + t) * 8 + s);
-    dst[2 * dh] = w0;
-    dst[2 * dh + 1] = w1;
-  }
+  prep_digits(v, mx, Lw, [&](int l, uint32_t w0, uint32_t w1) {
+    *(uint2*)((uint32_t*)(gp.xg + ((l * gp.nbp + blk) * gp.Tp + t) * 8 + s) + 2 * dh) = uint2{w0, w1};
+  });
 }
 
 }  // namespace imie_q1

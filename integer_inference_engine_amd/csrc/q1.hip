@@ -232,17 +232,17 @@ struct Q1Segs {                    // up to kMaxSegs weights (same n_blocks) app
 // wave walks tile groups gi, gi + W, gi + 2W, ... (W waves in the grid), so the digit staging is paid once per
 // workgroup and the pipeline runs on across group boundaries (the next group's first slab is in flight while the
 // current group's last slab computes).
-template <bool S64, int R, int TT, int PF = 0, int PRO = kProNone, int NT = 256, bool PERS = false>
+template <bool S64, int R, int PF = 0, int PRO = kProNone, int NT = 256, bool PERS = false>
 __global__ __launch_bounds__(NT) void q1_gemv_mfma_kernel(
     Q1Segs sg, const uint4* __restrict__ xq, const int64_t* __restrict__ totals, const int* __restrict__ lslab,
-    int64_t nslabs, int64_t nbp, int T, int frac, int64_t spk, int Lcap, int atomic_out, Q1Pro pro) {
-  static_assert(PRO == kProNone || (R == 1 && TT == 1 && PF > 0) || (PERS && PRO == kProCopy),
-                "prologue: one token, one tile, prefetched range (or the persistent kernel's copy prologue)");
+    int64_t nslabs, int64_t nbp, int frac, int64_t spk, int Lcap, int atomic_out, Q1Pro pro) {
+  static_assert(PRO == kProNone || (R == 1 && PF > 0) || (PERS && PRO == kProCopy),
+                "prologue: one tile, prefetched range (or the persistent kernel's copy prologue)");
   static_assert(PRO != kProNone || NT == 256, "NT: workgroup size of the prologue variants");
-  static_assert(!PERS || (TT == 1 && PF == 0 && (PRO == kProNone || PRO == kProCopy) && NT == 256),
-                "persistent: one token, pipelined slabs, at most 8 slabs staged by a copy prologue");
+  static_assert(!PERS || (PF == 0 && (PRO == kProNone || PRO == kProCopy) && NT == 256),
+                "persistent: pipelined slabs, at most 8 slabs staged by a copy prologue");
   extern __shared__ __align__(16) unsigned char smem[];
-  uint4* stage = (uint4*)smem;                                   // [TT][spk][Lcap][32]
+  uint4* stage = (uint4*)smem;                                   // [spk][Lcap][32]
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave-uniform: keeps the segment scalar
   const int64_t s0 = (int64_t)blockIdx.y * spk;
@@ -266,11 +266,9 @@ __global__ __launch_bounds__(NT) void q1_gemv_mfma_kernel(
   const int n = lane & 15;       // output row within the tile
   const bool aact = (n >> 2) == g;   // A row n (block n / 4) meets this lane's K group g
 
-  uint64_t acc[TT][R];
+  uint64_t acc[R];
 #pragma unroll
-  for (int t = 0; t < TT; ++t)
-#pragma unroll
-    for (int r = 0; r < R; ++r) acc[t][r] = 0;
+  for (int r = 0; r < R; ++r) acc[r] = 0;
 
   // PF > 0: the wave's whole slab range (at most PF slabs) is requested at once, before the digit staging
   // (decode-sized matvecs: every weight byte in flight in one round); PF == 0: two-slab software pipeline
@@ -278,8 +276,8 @@ __global__ __launch_bounds__(NT) void q1_gemv_mfma_kernel(
   uint4 wb[NB][R];
   using ScT = typename std::conditional<S64, int64_t, int32_t>::type;   // widened at use: no wait at the load
   ScT sc[NB][R];
-  int Lv[NB][TT];
-  int64_t tv[NB][TT];
+  int Lv[NB];
+  int64_t tv[NB];
   auto load_t = [&](int buf, int64_t tb, int64_t sl) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
@@ -290,44 +288,38 @@ __global__ __launch_bounds__(NT) void q1_gemv_mfma_kernel(
       sc[buf][r] = __builtin_nontemporal_load(&((const ScT*)scaleT)[idx]);
     }
     // the slab's digit count and block total travel with its weights (one prefetch, one wait)
-#pragma unroll
-    for (int t = 0; t < TT; ++t)
-      if (PRO == kProNone && t < T) {
-        Lv[buf][t] = lslab[t * nslabs + sl];
-        tv[buf][t] = totals[(int64_t)t * nbp + sl * kSlabBlocks + g];
-      }
+    if (PRO == kProNone) {
+      Lv[buf] = lslab[sl];
+      tv[buf] = totals[sl * kSlabBlocks + g];
+    }
   };
   auto load = [&](int buf, int64_t sl) { load_t(buf, tile0, sl); };
   // persistent mode: unit u = (group gi_raw + (u / nsl) W, slab s0 + u % nsl)
   const int64_t W = (int64_t)gridDim.x * (NT / 64);
   auto load_unit = [&](int buf, int64_t u) { load_t(buf, (gi_raw + (u / nsl) * W) * R, s0 + u % nsl); };
-  // A operands of (token t, limb group lg): the 8 bit positions' digit rows, loaded once and shared by the R
+  // A operands of limb group lg: the 8 bit positions' digit rows, loaded once and shared by the R
   // tiles; from LDS (staged limbs), the global table (limbs beyond Lcap), or the 8-entry zero slot for lanes
   // whose row is not their block or whose limb is beyond the slab's count
-  const uint4* zslot = stage + (int64_t)TT * spk * Lcap * 32;
+  const uint4* zslot = stage + spk * Lcap * 32;
   // PRO: slab limb counts, block totals and the element values after the zero slot
-  int* sL = (int*)(stage + (int64_t)TT * spk * Lcap * 32 + 8);
+  int* sL = (int*)(stage + spk * Lcap * 32 + 8);
   int64_t* stot = (int64_t*)(sL + 8);
   // element values (PRO), aliasing the table: each wave reads its slab's values before writing digits over them
   int64_t* s_y = (int64_t*)stage;
   const int arow_l = n & 3;
   auto compute = [&](int buf, int64_t sl) {
-    uint64_t pos[TT][R];
+    uint64_t pos[R];
 #pragma unroll
-    for (int t = 0; t < TT; ++t)
-#pragma unroll
-      for (int r = 0; r < R; ++r) pos[t][r] = 0;
-#pragma unroll
-    for (int t = 0; t < TT; ++t) {
-      if (t >= T) break;
-      const int L = PRO != kProNone ? sL[sl - s0] : Lv[buf][t];
+    for (int r = 0; r < R; ++r) pos[r] = 0;
+    {
+      const int L = PRO != kProNone ? sL[sl - s0] : Lv[buf];
       if (L == 1) {
         // one limb (e.g. int8 activations): rows = (block, bit position mod 4) with mask-only B operands
         // (bytes 0 / 2^s, 0x80 reading as -128); 128 * pos = sum d0[q] << (7 - q) + sum d1[q] << (3 - q)
         const int as = n & 3;
         uint4 a0 = uint4{0, 0, 0, 0}, a1 = uint4{0, 0, 0, 0};
         if (Lcap < 4) {
-          const uint4* src = xq + ((int64_t)t * kMaxLimbs * nbp + sl * kSlabBlocks + g) * 8 + as;
+          const uint4* src = xq + (sl * kSlabBlocks + g) * 8 + as;
           a0 = aact ? src[0] : uint4{0, 0, 0, 0};
           a1 = aact ? src[4] : uint4{0, 0, 0, 0};
         }
@@ -335,7 +327,7 @@ __global__ __launch_bounds__(NT) void q1_gemv_mfma_kernel(
         if (Lcap >= 4) {
           // from LDS: each register reads either the lane's digits or the zero slot (a per-lane address select
           // instead of four data selects per register)
-          const uint4* src = aact ? stage + ((t * spk + (sl - s0)) * Lcap) * 32 + g * 8 + as : zslot;
+          const uint4* src = aact ? stage + (sl - s0) * Lcap * 32 + g * 8 + as : zslot;
 #pragma unroll
           for (int sh = 0; sh < 4; ++sh) {
             const uint4* p0 = as == sh ? src : zslot;
@@ -364,10 +356,9 @@ __global__ __launch_bounds__(NT) void q1_gemv_mfma_kernel(
           }
           const int p128 = (d0[0] << 7) + (d0[1] << 6) + (d0[2] << 5) + (d0[3] << 4) + (d1[0] << 3) +
                            (d1[1] << 2) + (d1[2] << 1) - d1[3];
-          pos[t][r] += (uint64_t)(int64_t)(p128 >> 7);
+          pos[r] += (uint64_t)(int64_t)(p128 >> 7);
         }
-        continue;
-      }
+      } else {
 #pragma unroll
       for (int lg = 0; lg < 2; ++lg) {
         if (4 * lg >= L) break;                       // wave-uniform
@@ -375,14 +366,14 @@ __global__ __launch_bounds__(NT) void q1_gemv_mfma_kernel(
         const bool on = aact && l < L;
         v4i A[8];
         if (4 * lg + 4 <= Lcap) {
-          const uint4* src = on ? stage + ((t * spk + (sl - s0)) * Lcap + l) * 32 + g * 8 : zslot;
+          const uint4* src = on ? stage + ((sl - s0) * Lcap + l) * 32 + g * 8 : zslot;
 #pragma unroll
           for (int sh = 0; sh < 8; ++sh) {
             const uint4 a = src[sh];
             A[sh] = v4i{(int)a.x, (int)a.y, (int)a.z, (int)a.w};
           }
         } else {
-          const uint4* src = xq + ((int64_t)t * kMaxLimbs * nbp + (int64_t)l * nbp + sl * kSlabBlocks + g) * 8;
+          const uint4* src = xq + ((int64_t)l * nbp + sl * kSlabBlocks + g) * 8;
 #pragma unroll
           for (int sh = 0; sh < 8; ++sh) {
             const uint4 a = src[sh];
@@ -403,19 +394,16 @@ __global__ __launch_bounds__(NT) void q1_gemv_mfma_kernel(
             else D0 = __builtin_amdgcn_mfma_i32_16x16x64_i8(A[sh], b, D0, 0, 0, 0);
           }
 #pragma unroll
-          for (int q = 0; q < 4; ++q) pos[t][r] += (uint64_t)(int64_t)(D0[q] + D1[q]) << (8 * (4 * lg + q));
+          for (int q = 0; q < 4; ++q) pos[r] += (uint64_t)(int64_t)(D0[q] + D1[q]) << (8 * (4 * lg + q));
         }
       }
-    }
-#pragma unroll
-    for (int t = 0; t < TT; ++t) {
-      if (t >= T) break;
+      }
 #pragma unroll
       for (int r = 0; r < R; ++r) {
-        const int64_t tot = PRO != kProNone ? stot[(sl - s0) * 4 + g] : tv[buf][t];
-        const uint64_t S = 2u * pos[t][r] - (uint64_t)tot;
+        const int64_t tot = PRO != kProNone ? stot[(sl - s0) * 4 + g] : tv[buf];
+        const uint64_t S = 2u * pos[r] - (uint64_t)tot;
         const int64_t prod = (int64_t)(S * (uint64_t)(int64_t)sc[buf][r]);
-        acc[t][r] += (uint64_t)imie_floor_shift(prod, frac);
+        acc[r] += (uint64_t)imie_floor_shift(prod, frac);
       }
     }
   };
@@ -538,16 +526,15 @@ __global__ __launch_bounds__(NT) void q1_gemv_mfma_kernel(
     __syncthreads();
   } else {
   // stage the digit operands of this slab range (the same x for every wave of the workgroup)
-  for (int t = 0; t < T; ++t)
-    for (int64_t j = 0; j < nsl; ++j) {
-      const int L = min(lslab[t * nslabs + s0 + j], Lcap);
-      uint4* dst = stage + ((t * spk + j) * Lcap) * 32;
-      for (int i = threadIdx.x; i < L * 32; i += blockDim.x) {
-        const int l = i >> 5, e = i & 31;
-        dst[i] = xq[(((int64_t)t * kMaxLimbs + l) * nbp + (s0 + j) * kSlabBlocks) * 8 + e];
-      }
+  for (int64_t j = 0; j < nsl; ++j) {
+    const int L = min(lslab[s0 + j], Lcap);
+    uint4* dst = stage + j * Lcap * 32;
+    for (int i = threadIdx.x; i < L * 32; i += blockDim.x) {
+      const int l = i >> 5, e = i & 31;
+      dst[i] = xq[((int64_t)l * nbp + (s0 + j) * kSlabBlocks) * 8 + e];
     }
-  if (threadIdx.x < 8) stage[(int64_t)TT * spk * Lcap * 32 + threadIdx.x] = uint4{0, 0, 0, 0};
+  }
+  if (threadIdx.x < 8) stage[spk * Lcap * 32 + threadIdx.x] = uint4{0, 0, 0, 0};
   __syncthreads();
   }
 
@@ -558,7 +545,7 @@ __global__ __launch_bounds__(NT) void q1_gemv_mfma_kernel(
     auto flush = [&](int64_t tb) {
 #pragma unroll
       for (int r = 0; r < R; ++r) {
-        uint64_t v = acc[0][r];
+        uint64_t v = acc[r];
         v += (uint64_t)__shfl_xor((int64_t)v, 16, 64);
         v += (uint64_t)__shfl_xor((int64_t)v, 32, 64);
         const int64_t row = (tb + r) * kTileRows + n;
@@ -566,7 +553,7 @@ __global__ __launch_bounds__(NT) void q1_gemv_mfma_kernel(
           if (atomic_out == 2) out[row] = (int64_t)((uint64_t)out[row] + v);
           else out[row] = (int64_t)v;
         }
-        acc[0][r] = 0;
+        acc[r] = 0;
       }
     };
     const int64_t ngroups = sg.gbegin[1];
@@ -603,25 +590,19 @@ __global__ __launch_bounds__(NT) void q1_gemv_mfma_kernel(
 
   // sum the 4 blocks of each row (lane groups g) and write / accumulate row totals
 #pragma unroll
-  for (int t = 0; t < TT; ++t) {
-    if (t >= T) break;
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      uint64_t v = acc[t][r];
-      v += (uint64_t)__shfl_xor((int64_t)v, 16, 64);
-      v += (uint64_t)__shfl_xor((int64_t)v, 32, 64);
-      const int64_t row = (tile0 + r) * kTileRows + n;
-      if (g == 0 && tile0 + r < ntiles && row < N) {
-        if (atomic_out == 1) atomicAdd((unsigned long long*)&out[(int64_t)t * N + row], (unsigned long long)v);
-        else if (atomic_out == 2) out[(int64_t)t * N + row] = (int64_t)((uint64_t)out[(int64_t)t * N + row] + v);
-        else out[(int64_t)t * N + row] = (int64_t)v;
-      }
+  for (int r = 0; r < R; ++r) {
+    uint64_t v = acc[r];
+    v += (uint64_t)__shfl_xor((int64_t)v, 16, 64);
+    v += (uint64_t)__shfl_xor((int64_t)v, 32, 64);
+    const int64_t row = (tile0 + r) * kTileRows + n;
+    if (g == 0 && tile0 + r < ntiles && row < N) {
+      if (atomic_out == 1) atomicAdd((unsigned long long*)&out[row], (unsigned long long)v);
+      else if (atomic_out == 2) out[row] = (int64_t)((uint64_t)out[row] + v);
+      else out[row] = (int64_t)v;
     }
   }
 }
 
-// Straightforward exact kernel (thread per output): used for shapes the MFMA path declines and as an
-// in-library cross-check. Reads the natural (N, nb, 16) layout.
 __global__ void q1_linear_simple_kernel(const int64_t* __restrict__ x, const uint8_t* __restrict__ bits,
                                         const int64_t* __restrict__ scale, int64_t T, int64_t N, int64_t nb,
                                         int frac, int64_t* __restrict__ out) {
@@ -646,6 +627,297 @@ __global__ void q1_linear_simple_kernel(const int64_t* __restrict__ x, const uin
   out[idx] = (int64_t)tot;
 }
 
+
+// ------------------------------------------------------------------------------------------------------
+// One token, host-driven single projections: one launch without a prep kernel, cleared outputs or atomics. Workgroup =
+// 8 waves that split K (wave w takes slabs w, w + 8, ...) and walk the same tiles; a wave forms the digits of its own
+// slabs (nothing is shared, so no barrier) while its first weights are in flight, and the waves' row sums meet in LDS,
+// one barrier a tile. Bound by latency: one launch, one load round, the digits, one tile's MFMAs.
+// A 4096 x 4096 projection: 10.4 us as prep launch and K-split launch (3.6 + 4.3 and the gap), 4.9 as one (7.7 us a call with the host's share).
+// ------------------------------------------------------------------------------------------------------
+constexpr int kRowMaxSlabs = 32;    // 4 KB of digits a slab
+
+template <bool S64>
+__global__ __launch_bounds__(512) void q1_row_kernel(const v4i* __restrict__ bitsT, const void* __restrict__ scaleT,
+                                                     int64_t N, int64_t ntiles, int nslabs, int64_t K,
+                                                     const int64_t* __restrict__ x, int frac, int accumulate,
+                                                     int64_t* __restrict__ out) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  uint4* sA = (uint4*)smem;                                      // [slab][kMaxLimbs][32]
+  uint4* zslot = sA + (int64_t)nslabs * kMaxLimbs * 32;
+  int64_t* stot = (int64_t*)(zslot + 8);
+  int* sL = (int*)(stot + nslabs * kSlabBlocks);
+  __shared__ uint64_t s_sum[2][8][kTileRows];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 4, n = lane & 15, al = n & 3;
+  const bool aact = (n >> 2) == g;
+  using ScT = typename std::conditional<S64, int64_t, int32_t>::type;
+  v4i wb[2];
+  ScT sc[2];
+  auto load = [&](int buf, int64_t tile, int sl) {
+    const int64_t idx = (tile * nslabs + sl) * 64 + lane;
+    wb[buf] = __builtin_nontemporal_load(&bitsT[idx]);
+    sc[buf] = __builtin_nontemporal_load(&((const ScT*)scaleT)[idx]);
+  };
+  const int nmine = wave < nslabs ? (nslabs - 1 - wave) / 8 + 1 : 0;
+  const int64_t nt = (ntiles - 1 - blockIdx.x) / gridDim.x + 1;  // the host keeps gridDim.x <= ntiles
+  if (nmine) load(0, blockIdx.x, wave);
+  if (threadIdx.x < 8) zslot[threadIdx.x] = uint4{0, 0, 0, 0};
+  for (int sl = wave; sl < nslabs; sl += 8) {
+    int64_t v[8];
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int64_t c = prep_pos(lane, sl, q);
+      v[q] = x[c < K ? c : 0];
+      v[q] = c < K ? v[q] : 0;
+    }
+    prep_slab_lds(v, sA + (int64_t)sl * kMaxLimbs * 32, &sL[sl], &stot[sl * kSlabBlocks]);
+  }
+  __syncthreads();                                               // the zero slot (and each wave's own digits)
+  auto compute = [&](int buf, int sl) -> uint64_t {
+    const v4i w = wb[buf];
+    const int L = __builtin_amdgcn_readfirstlane(sL[sl]);
+    uint64_t pos = 0;
+#pragma unroll
+    for (int lg = 0; lg < 2; ++lg) {
+      if (4 * lg >= L) break;
+      const uint4* src = aact && 4 * lg + al < L ? sA + ((int64_t)sl * kMaxLimbs + 4 * lg + al) * 32 + g * 8 : zslot;
+      v4i D0 = {0, 0, 0, 0}, D1 = {0, 0, 0, 0};
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const uint4 a4 = src[k];
+        const v4i A = v4i{(int)a4.x, (int)a4.y, (int)a4.z, (int)a4.w};
+        const v4i b = v4i{(int)(((uint32_t)w[0] >> k) & 0x01010101u), (int)(((uint32_t)w[1] >> k) & 0x01010101u),
+                          (int)(((uint32_t)w[2] >> k) & 0x01010101u), (int)(((uint32_t)w[3] >> k) & 0x01010101u)};
+        if (k & 1) D1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(A, b, D1, 0, 0, 0);
+        else D0 = __builtin_amdgcn_mfma_i32_16x16x64_i8(A, b, D0, 0, 0, 0);
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) pos += (uint64_t)(int64_t)(D0[q] + D1[q]) << (8 * (4 * lg + q));
+    }
+    const uint64_t S = 2u * pos - (uint64_t)stot[sl * kSlabBlocks + g];
+    return (uint64_t)imie_floor_shift((int64_t)(S * (uint64_t)(int64_t)sc[buf]), frac);
+  };
+  int buf = 0;
+  for (int64_t it = 0; it < nt; ++it) {
+    const int64_t tile = blockIdx.x + it * gridDim.x;
+    uint64_t acc = 0;
+    for (int k = 0; k < nmine; ++k) {
+      const int sl = wave + 8 * k;
+      const bool last = k + 1 == nmine;
+      if (!last || it + 1 < nt) {                                // the next (tile, slab) in flight
+        if (buf) load(0, last ? tile + gridDim.x : tile, last ? wave : sl + 8);
+        else load(1, last ? tile + gridDim.x : tile, last ? wave : sl + 8);
+      }
+      acc += buf ? compute(1, sl) : compute(0, sl);
+      buf ^= 1;
+    }
+    acc += (uint64_t)__shfl_xor((int64_t)acc, 16, 64);
+    acc += (uint64_t)__shfl_xor((int64_t)acc, 32, 64);
+    uint64_t (&sum)[8][kTileRows] = s_sum[it & 1];               // two sets: the next tile's barrier frees this one
+    if (g == 0) sum[wave][n] = acc;
+    __syncthreads();
+    const int64_t row = tile * kTileRows + threadIdx.x;
+    if (threadIdx.x < kTileRows && row < N) {
+      uint64_t v = 0;
+#pragma unroll
+      for (int w = 0; w < 8; ++w) v += sum[w][threadIdx.x];
+      out[row] = accumulate ? (int64_t)((uint64_t)out[row] + v) : (int64_t)v;
+    }
+  }
+}
+
+// ------------------------------------------------------------------------------------------------------
+// Two to eight tokens (small-batch decode): the matvec's MFMA arrangement (rows = block x limb of one token, columns =
+// 16 weight rows, one MFMA per bit position), with the slab range's digits of every token resident in LDS and each
+// weight read and bit-expanded once for all tokens. Workgroup = 8 waves; a wave walks groups of R tiles over the
+// workgroup's slab range, the next (group, slab)'s weights in flight. grid.y splits K (64-bit atomics into cleared
+// outputs). Slabs of up to three limbs (|x| < 2^23) recombine in 32 bits; more take the 64-bit form, limbs past the
+// fourth from the global table.
+// Bound by the matrix pipe and VALU (8 MFMAs and about 15 VALU instructions a token, slab and tile, and 64 for a tile's
+// bits); the weights of an 8B layer are 0.5 to 13 MB.
+// Why not the one-token kernel over several tokens: its 48 KB of staging held no limb of four tokens over eight slabs,
+// so every operand came from L2. Measured, that kernel against this one at 2, 4, 7 tokens (us, with the prep launch):
+// 4096 x 4096 10.8, 10.7, 16.6 / 9.9, 10.5, 12.8; 12288 x 4096 12.6, 17.6, 28.5 / 11.9, 13.7, 17.1; the 151,936-row
+// head 59, 299, 522 / 64, 91, 138. At 8 tokens against the GEMM kernels 16.4, 24.2, 176 / 13.6, 18.5, 151; at 10 it
+// would be 17.9, 27.2, 182 against 16.3, 24.8, 176, so the line (kGemmMinT) lies behind 8.
+// ------------------------------------------------------------------------------------------------------
+constexpr int kFewLimbs = 4;
+constexpr int64_t kFewLds = 144 * 1024;   // digits resident in LDS: 2 KB a token and slab
+
+template <bool S64, int R, int TT>
+__global__ __launch_bounds__(512) void q1_few_kernel(Q1Segs sg, const uint4* __restrict__ xq,
+                                                     const int64_t* __restrict__ totals, const int* __restrict__ lslab,
+                                                     int64_t nslabs, int64_t nbp, int T, int frac, int64_t spk,
+                                                     int mode) {
+  extern __shared__ __align__(16) unsigned char smem[];
+  uint4* sA = (uint4*)smem;                                      // [T][spk][kFewLimbs][32]
+  uint4* zslot = sA + (int64_t)T * spk * kFewLimbs * 32;         // 8 zeros
+  int64_t* stot = (int64_t*)(zslot + 8);                         // [T][spk][4]
+  int* sL = (int*)(stot + (int64_t)T * spk * kSlabBlocks);       // [T][spk]
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t s0 = (int64_t)blockIdx.y * spk;
+  const int nsl = (int)(min(nslabs, s0 + spk) - s0);
+  const int g = lane >> 4, n = lane & 15;
+  const bool aact = (n >> 2) == g;
+  const int al = n & 3;                                          // limb of this lane's A row
+
+  using ScT = typename std::conditional<S64, int64_t, int32_t>::type;
+  struct Unit { int64_t t0; int seg; int j; };                   // first tile, segment, slab of the range
+  const int64_t W = (int64_t)gridDim.x * 8, ngroups = sg.gbegin[sg.cnt];
+  const int64_t g0 = (int64_t)blockIdx.x * 8 + wave;
+  const int64_t nu = g0 < ngroups ? ((ngroups - 1 - g0) / W + 1) * nsl : 0;
+  auto unit = [&](int64_t u) {
+    const int64_t gi = g0 + (u / nsl) * W;
+    int seg = 0;
+#pragma unroll
+    for (int z = 1; z < kMaxSegs; ++z)
+      if (z < sg.cnt && gi >= sg.gbegin[z]) seg = z;
+    return Unit{(gi - sg.gbegin[seg]) * R, seg, (int)(u % nsl)};
+  };
+  v4i wb[2][R];
+  ScT sc[2][R];
+  auto load = [&](int buf, const Unit& x) {
+    const v4i* bits = (const v4i*)sg.bits[x.seg];
+    const ScT* scale = (const ScT*)sg.scale[x.seg];
+    const int64_t ntiles = sg.ntiles[x.seg];
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int64_t tl = x.t0 + r < ntiles ? x.t0 + r : x.t0;
+      const int64_t idx = (tl * nslabs + s0 + x.j) * 64 + lane;
+      wb[buf][r] = __builtin_nontemporal_load(&bits[idx]);
+      sc[buf][r] = __builtin_nontemporal_load(&scale[idx]);
+    }
+  };
+  Unit cur = unit(0);
+  if (nu) load(0, cur);                                          // in flight while the digits are staged
+  for (int i = threadIdx.x; i < T * nsl * 32; i += 512) {
+    const int e = i & 31, tj = i >> 5, t = tj / nsl, j = tj - t * nsl;
+    const int L = lslab[t * nslabs + s0 + j];
+#pragma unroll
+    for (int l = 0; l < kFewLimbs; ++l) {
+      uint4 v = uint4{0, 0, 0, 0};
+      if (l < L) v = xq[(((int64_t)t * kMaxLimbs + l) * nbp + (s0 + j) * kSlabBlocks) * 8 + e];
+      sA[((t * spk + j) * kFewLimbs + l) * 32 + e] = v;
+    }
+    if (e < kSlabBlocks) stot[(t * spk + j) * kSlabBlocks + e] = totals[(int64_t)t * nbp + (s0 + j) * kSlabBlocks + e];
+    if (e == 0) sL[t * spk + j] = L;
+  }
+  if (threadIdx.x < 8) zslot[threadIdx.x] = uint4{0, 0, 0, 0};
+  __syncthreads();
+
+  uint64_t acc[TT][R];
+#pragma unroll
+  for (int t = 0; t < TT; ++t)
+#pragma unroll
+    for (int r = 0; r < R; ++r) acc[t][r] = 0;
+  // one (R tiles, slab): every token's digits against the tiles' bit planes
+  auto compute = [&](int buf, int j) {
+    v4i b[R][8];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const v4i w = wb[buf][r];
+        b[r][k] = v4i{(int)(((uint32_t)w[0] >> k) & 0x01010101u), (int)(((uint32_t)w[1] >> k) & 0x01010101u),
+                      (int)(((uint32_t)w[2] >> k) & 0x01010101u), (int)(((uint32_t)w[3] >> k) & 0x01010101u)};
+      }
+#pragma unroll
+    for (int t = 0; t < TT; ++t) {
+      if (t >= T) break;
+      const int L = __builtin_amdgcn_readfirstlane(sL[t * spk + j]);
+      const uint4* src = aact ? sA + ((t * spk + j) * kFewLimbs + al) * 32 + g * 8 : zslot;
+      v4i D[R][2];
+#pragma unroll
+      for (int r = 0; r < R; ++r) D[r][0] = D[r][1] = v4i{0, 0, 0, 0};
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const uint4 a4 = src[k];
+        const v4i A = v4i{(int)a4.x, (int)a4.y, (int)a4.z, (int)a4.w};
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+          D[r][k & 1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A, b[r][k], D[r][k & 1], 0, 0, 0);
+      }
+      const int64_t tot = stot[(t * spk + j) * kSlabBlocks + g];
+      if (L <= 3) {
+        // |D| <= 2^14 a limb: the sum of three limbs and 2 pos - tot stay below 2^31
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          const int pos = (D[r][0][0] + D[r][1][0]) + ((D[r][0][1] + D[r][1][1]) << 8) +
+                          ((D[r][0][2] + D[r][1][2]) << 16);
+          const int S = (pos << 1) - (int)tot;
+          const int64_t prod = (int64_t)((uint64_t)(int64_t)S * (uint64_t)(int64_t)sc[buf][r]);
+          acc[t][r] += (uint64_t)imie_floor_shift(prod, frac);
+        }
+        continue;
+      }
+      uint64_t pos[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        pos[r] = 0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) pos[r] += (uint64_t)(int64_t)(D[r][0][q] + D[r][1][q]) << (8 * q);
+        D[r][0] = D[r][1] = v4i{0, 0, 0, 0};
+      }
+      if (L > kFewLimbs) {
+        const uint4* gsrc = xq + (((int64_t)t * kMaxLimbs + kFewLimbs + al) * nbp + (s0 + j) * kSlabBlocks + g) * 8;
+        const bool on = aact && kFewLimbs + al < L;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+          const uint4 a4 = on ? gsrc[k] : uint4{0, 0, 0, 0};
+          const v4i A = v4i{(int)a4.x, (int)a4.y, (int)a4.z, (int)a4.w};
+#pragma unroll
+          for (int r = 0; r < R; ++r)
+            D[r][k & 1] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A, b[r][k], D[r][k & 1], 0, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) pos[r] += (uint64_t)(int64_t)(D[r][0][q] + D[r][1][q]) << (8 * (kFewLimbs + q));
+      }
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const int64_t prod = (int64_t)((2u * pos[r] - (uint64_t)tot) * (uint64_t)(int64_t)sc[buf][r]);
+        acc[t][r] += (uint64_t)imie_floor_shift(prod, frac);
+      }
+    }
+  };
+  // the group's rows are complete after the range's last slab: sum the four blocks of each row and write
+  auto flush = [&](const Unit& x) {
+    int64_t* out = sg.out[x.seg];
+    const int64_t N = sg.N[x.seg], ntiles = sg.ntiles[x.seg];
+#pragma unroll
+    for (int t = 0; t < TT; ++t) {
+      if (t >= T) break;
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        uint64_t v = acc[t][r];
+        v += (uint64_t)__shfl_xor((int64_t)v, 16, 64);
+        v += (uint64_t)__shfl_xor((int64_t)v, 32, 64);
+        acc[t][r] = 0;
+        const int64_t row = (x.t0 + r) * kTileRows + n;
+        if (g != 0 || x.t0 + r >= ntiles || row >= N) continue;
+        int64_t* dst = out + (int64_t)t * N + row;
+        if (mode == 1) atomicAdd((unsigned long long*)dst, (unsigned long long)v);
+        else *dst = mode == 2 ? (int64_t)((uint64_t)*dst + v) : (int64_t)v;
+      }
+    }
+  };
+  for (int64_t u = 0; u < nu; ++u) {
+    const Unit nx = unit(u + 1 < nu ? u + 1 : u);
+    if (u & 1) {
+      if (u + 1 < nu) load(0, nx);
+      compute(1, cur.j);
+    } else {
+      if (u + 1 < nu) load(1, nx);
+      compute(0, cur.j);
+    }
+    if (cur.j == nsl - 1) flush(cur);
+    cur = nx;
+  }
+}
 
 // ------------------------------------------------------------------------------------------------------
 // GEMM path (T >= kGemmMinT tokens; prefill): int8 MFMA with TOKENS in the MFMA M dimension.
@@ -2156,6 +2428,77 @@ static int q1_gemm_multi(const Q1Weight* const* ws, int cnt, const int64_t* x_de
 // ------------------------------------------------------------------------------------------------------
 // Launch helpers
 // ------------------------------------------------------------------------------------------------------
+// One-token single projections up to this many tiles take q1_row_kernel: its cost grows by 1.7 us a round of 256 tiles
+// (768 tiles 7.6 us, 9496 tiles 68 us), the prep and K-split or streaming launches stay at 10.5 us to about 1024 tiles
+// (the 151,936-row head 35 us).
+constexpr int64_t kRowMaxTiles = 1024;
+// Two to kGemmMinT - 1 tokens (q1_few_kernel). Slab ranges as long as they leave 2048 waves (8 per CU), at most 8 slabs
+// and what LDS holds of the tokens' digits; two tiles per wave share the digit reads once that still leaves 1024 waves.
+static int q1_few_launch(const Q1Weight* const* ws, int cnt, const int64_t* x_dev, int64_t T, int64_t frac,
+                         int64_t* const* outs, int accumulate, Q1Ws& wk, hipStream_t st, int prepped,
+                         int64_t ntiles_all) {
+  const Q1Weight& w0 = *ws[0];
+  const int64_t nslabs = w0.nslabs, nbp = nslabs * kSlabBlocks;
+  int64_t spk = 1;
+  for (int64_t c = 8; c >= 2; c >>= 1)
+    if (ntiles_all * ((nslabs + c - 1) / c) >= 2048 && T * c * (kFewLimbs * 512 + 36) <= kFewLds) { spk = c; break; }
+  if (spk > nslabs) spk = nslabs;
+  const int64_t ksplit = (nslabs + spk - 1) / spk;
+  const int R = ntiles_all * ksplit >= 2048 ? 2 : 1;
+  Q1Segs sg = {};
+  sg.cnt = cnt;
+  int64_t groups = 0;
+  for (int i = 0; i < cnt; ++i) {
+    sg.bits[i] = ws[i]->bits;
+    sg.scale[i] = ws[i]->scale;
+    sg.N[i] = ws[i]->N;
+    sg.ntiles[i] = ws[i]->ntiles;
+    sg.out[i] = outs[i];
+    sg.gbegin[i] = groups;
+    groups += (ws[i]->ntiles + R - 1) / R;
+  }
+  sg.gbegin[cnt] = groups;
+  if (!prepped) {
+    Q1Zero zero = {};                                 // K-split outputs are cleared by the prep kernel
+    if (ksplit > 1 && !accumulate) {
+      zero.cnt = cnt;
+      for (int i = 0; i < cnt; ++i) { zero.p[i] = outs[i]; zero.n[i] = T * ws[i]->N; }
+    }
+    imie_prof_mark(IMIE_K_Q1_PREP, st, true);
+    Q1PrepOut po = {(uint32_t*)wk.xq.p, (int64_t*)wk.totals.p, (int*)wk.lslab.p, w0.nb, nbp, nslabs};
+    hipLaunchKernelGGL(q1_prep_kernel, dim3((unsigned)nslabs, (unsigned)T), dim3(64), 0, st, x_dev, w0.nb * 128, po, zero);
+    imie_prof_mark(IMIE_K_Q1_PREP, st, false);
+    IMIE_HIP(hipGetLastError());
+  }
+  const size_t lds = (size_t)T * spk * (kFewLimbs * 32 * 16 + kSlabBlocks * 8 + 4) + 128;
+  const int mode = ksplit > 1 ? 1 : (accumulate ? 2 : 0);
+  // workgroups of 8 groups; a long walk is cut into equal rounds over what the chip holds at once (two per CU)
+  int64_t wgs = (groups + 7) / 8;
+  const int64_t fit = 512 / ksplit > 0 ? 512 / ksplit : 1;
+  if (wgs > fit) { const int64_t rounds = (wgs + fit - 1) / fit; wgs = (wgs + rounds - 1) / rounds; }
+  const dim3 grid((unsigned)wgs, (unsigned)ksplit);
+  const int fr = (int)(frac > 63 ? 63 : frac);
+  imie_prof_mark(IMIE_K_Q1_GEMV, st, true);
+#define IMIE_Q1_FEW(S64_, R_, TT_)                                                                                    \
+  do {                                                                                                               \
+    static const hipError_t big = hipFuncSetAttribute((const void*)q1_few_kernel<S64_, R_, TT_>,                       \
+                                                      hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);         \
+    (void)big;                                                                                                        \
+    hipLaunchKernelGGL((q1_few_kernel<S64_, R_, TT_>), grid, dim3(512), lds, st, sg, (const uint4*)wk.xq.p,            \
+                       (const int64_t*)wk.totals.p, (const int*)wk.lslab.p, nslabs, nbp, (int)T, fr, spk, mode);        \
+  } while (0)
+#define IMIE_Q1_FEW_R(S64_, TT_) do { if (R == 2) IMIE_Q1_FEW(S64_, 2, TT_); else IMIE_Q1_FEW(S64_, 1, TT_); } while (0)
+  static_assert(kGemmMinT <= 9, "instantiated for up to 8 tokens");
+  if (w0.scale64) { if (T <= 4) IMIE_Q1_FEW_R(true, 4); else IMIE_Q1_FEW_R(true, 8); }
+  else if (T <= 4) IMIE_Q1_FEW_R(false, 4);
+  else IMIE_Q1_FEW_R(false, 8);
+#undef IMIE_Q1_FEW_R
+#undef IMIE_Q1_FEW
+  imie_prof_mark(IMIE_K_Q1_GEMV, st, false);
+  IMIE_HIP(hipGetLastError());
+  return IMIE_OK;
+}
+
 // One prep (digit table of x, shared by every segment) and one matvec launch over up to kMaxSegs weights with
 // the same n_blocks and scale width; outs[i] receives (T, N_i). accumulate != 0 adds into the outputs.
 // prepped != 0: the caller's producer already wrote the digit table into wk (imie_q1_prep_target) and cleared
@@ -2175,12 +2518,34 @@ static int q1_apply_multi(const Q1Weight* const* ws, int cnt, const int64_t* x_d
   if (wk.xq.ensure((size_t)T * kMaxLimbs * nbp * 8 * 16) || wk.totals.ensure((size_t)T * nbp * 8) ||
       wk.lslab.ensure((size_t)T * nslabs * 4))
     return IMIE_EARG;
-  // Work split: waves = tile groups of R tiles; grid.y splits the slabs when there are too few tile groups
-  // to keep ~8 waves per CU busy (decode-sized matvecs).
   int64_t ntiles_all = 0;
   for (int i = 0; i < cnt; ++i) ntiles_all += ws[i]->ntiles;
+  if (T > 1) return q1_few_launch(ws, cnt, x_dev, T, frac, outs, accumulate, wk, st, prepped, ntiles_all);
+  if (!prepped && cnt == 1 && nslabs <= kRowMaxSlabs && ntiles_all <= kRowMaxTiles) {
+    const size_t lds = (size_t)nslabs * (kMaxLimbs * 512 + kSlabBlocks * 8 + 4) + 128;
+    int64_t wgs = ntiles_all;                         // equal rounds of at most 256 workgroups (the digits are per workgroup)
+    if (wgs > 256) { const int64_t rounds = (wgs + 255) / 256; wgs = (wgs + rounds - 1) / rounds; }
+    const int fr1 = (int)(frac > 63 ? 63 : frac);
+    imie_prof_mark(IMIE_K_Q1_GEMV, st, true);
+#define IMIE_Q1_ROW(S64_)                                                                                             \
+  do {                                                                                                                \
+    static const hipError_t big = hipFuncSetAttribute((const void*)q1_row_kernel<S64_>,                                 \
+                                                      hipFuncAttributeMaxDynamicSharedMemorySize, 156 * 1024);          \
+    (void)big;                                                                                                         \
+    hipLaunchKernelGGL(q1_row_kernel<S64_>, dim3((unsigned)wgs), dim3(512), lds, st, (const v4i*)w0.bits, w0.scale, w0.N, \
+                       w0.ntiles, (int)nslabs, w0.nb * 128, x_dev, fr1, accumulate ? 1 : 0, outs[0]);                    \
+  } while (0)
+    if (w0.scale64) IMIE_Q1_ROW(true);
+    else IMIE_Q1_ROW(false);
+#undef IMIE_Q1_ROW
+    imie_prof_mark(IMIE_K_Q1_GEMV, st, false);
+    IMIE_HIP(hipGetLastError());
+    return IMIE_OK;
+  }
+  // Work split: waves = tile groups of R tiles; grid.y splits the slabs when there are too few tile groups
+  // to keep ~8 waves per CU busy (decode-sized matvecs).
   // R = 4 only for single-token launches (four tokens x four tiles would exceed the register budget)
-  const int R = (ntiles_all >= 4 * 16384 && T == 1) ? 4 : (ntiles_all >= 2 * 8192 ? 2 : 1);
+  const int R = ntiles_all >= 4 * 16384 ? 4 : (ntiles_all >= 2 * 8192 ? 2 : 1);
   Q1Segs sg = {};
   sg.cnt = cnt;
   int64_t groups = 0;
@@ -2195,7 +2560,7 @@ static int q1_apply_multi(const Q1Weight* const* ws, int cnt, const int64_t* x_d
   sg.gbegin[cnt] = groups;
   int64_t ksplit = 1, spk = nslabs;
   int pf = 0;
-  if (T == 1 && R == 1 && groups * nslabs <= 64 * 1024) {
+  if (R == 1 && groups * nslabs <= 64 * 1024) {
     // decode-sized: the largest slab range of 4 / 2 / 1 that still gives >= 2048 waves; each wave requests
     // its whole range at once, so one round of resident waves covers the matrix
     pf = 1;
@@ -2209,17 +2574,14 @@ static int q1_apply_multi(const Q1Weight* const* ws, int cnt, const int64_t* x_d
     spk = (nslabs + ksplit - 1) / ksplit;
     ksplit = (nslabs + spk - 1) / spk;
   }
-  const int TT = T <= 1 ? 1 : (T <= 2 ? 2 : 4);
-  if (TT == 4 && R == 4) return IMIE_EARG;
   // large single-token launches on one weight: persistent waves (IMIE_Q1_PERS = workgroups per CU, 0 = off)
   static const int pers_wpc = [] { const char* e = getenv("IMIE_Q1_PERS"); return e ? atoi(e) : 3; }();
-  const bool pers = pers_wpc > 0 && R == 4 && T == 1 && cnt == 1 && ksplit == 1 && pf == 0;            // not instantiated: R is 4 only for T == 1
-  const int Tc = TT;
+  const bool pers = pers_wpc > 0 && R == 4 && cnt == 1 && ksplit == 1 && pf == 0;
   // the prep kernel clears the outputs when the matvec adds into them (K-split) and no residual is kept
   Q1Zero zero = {};
   if (ksplit > 1 && !accumulate) {
     zero.cnt = cnt;
-    for (int i = 0; i < cnt; ++i) { zero.p[i] = outs[i]; zero.n[i] = T * ws[i]->N; }
+    for (int i = 0; i < cnt; ++i) { zero.p[i] = outs[i]; zero.n[i] = ws[i]->N; }
   }
   const int64_t K = w0.nb * 128;
   // the persistent launch on K <= 4096 builds its digit table itself (copy prologue): no prep launch
@@ -2228,17 +2590,17 @@ static int q1_apply_multi(const Q1Weight* const* ws, int cnt, const int64_t* x_d
   if (!prepped && !pers_pro) {
     imie_prof_mark(IMIE_K_Q1_PREP, st, true);
     Q1PrepOut po = {(uint32_t*)wk.xq.p, (int64_t*)wk.totals.p, (int*)wk.lslab.p, w0.nb, nbp, nslabs};
-    hipLaunchKernelGGL(q1_prep_kernel, dim3((unsigned)nslabs, (unsigned)T), dim3(64), 0, st, x_dev, K, po, zero);
+    hipLaunchKernelGGL(q1_prep_kernel, dim3((unsigned)nslabs, 1), dim3(64), 0, st, x_dev, K, po, zero);
     imie_prof_mark(IMIE_K_Q1_PREP, st, false);
   }
   IMIE_HIP(hipGetLastError());
   const size_t budget = 48 * 1024;
   // staged limbs come in whole groups of four (a limb group reads either LDS or the global table)
-  int Lcap = (int)(budget / ((size_t)Tc * spk * 512));
+  int Lcap = (int)(budget / ((size_t)spk * 512));
   Lcap = Lcap >= 8 ? 8 : (Lcap >= 4 ? 4 : 0);
   if (pers_pro) Lcap = 8;                            // the prologue stages every limb (spk <= 8: 32 KB)
   // + the zero slot (8 x 16 B); a prologue also keeps the slab limb counts and block totals
-  const size_t lds = (size_t)Tc * spk * Lcap * 512 + 128 + (pers_pro ? 32 + 256 : 0);
+  const size_t lds = (size_t)spk * Lcap * 512 + 128 + (pers_pro ? 32 + 256 : 0);
   const int fr = (int)(frac > 63 ? 63 : frac);
   const dim3 grid((unsigned)((groups + 3) / 4), (unsigned)ksplit);
   dim3 pgrid = grid;
@@ -2253,49 +2615,40 @@ static int q1_apply_multi(const Q1Weight* const* ws, int cnt, const int64_t* x_d
   }
   const int mode = ksplit > 1 ? 1 : (accumulate ? 2 : 0);
   imie_prof_mark(IMIE_K_Q1_GEMV, st, true);
-  for (int64_t t0 = 0; t0 < T; t0 += Tc) {
-    const int tn = (int)(T - t0 < Tc ? T - t0 : Tc);
-    Q1Segs sgt = sg;
-    for (int i = 0; i < cnt; ++i) sgt.out[i] = outs[i] + t0 * ws[i]->N;
-    const uint4* xq = (const uint4*)wk.xq.p + t0 * kMaxLimbs * nbp * 8;
-    const int64_t* tot = (const int64_t*)wk.totals.p + t0 * nbp;
-    const int* ls = (const int*)wk.lslab.p + t0 * nslabs;
-#define IMIE_Q1_LAUNCH(S64_, R_, TT_)                                                                        \
-  hipLaunchKernelGGL((q1_gemv_mfma_kernel<S64_, R_, TT_>), grid, dim3(256), lds, st, sgt, xq, tot, ls, nslabs,  \
-                     nbp, tn, fr, spk, Lcap, mode, Q1Pro{})
-#define IMIE_Q1_LAUNCH_R(S64_, TT_)                                                                          \
-  if (R == 4) IMIE_Q1_LAUNCH(S64_, 4, TT_); else if (R == 2) IMIE_Q1_LAUNCH(S64_, 2, TT_); else IMIE_Q1_LAUNCH(S64_, 1, TT_)
-#define IMIE_Q1_LAUNCH_T(S64_)                                                                               \
-  if (TT == 1) { IMIE_Q1_LAUNCH_R(S64_, 1); } else if (TT == 2) { IMIE_Q1_LAUNCH_R(S64_, 2); }                 \
-  else if (R == 2) { IMIE_Q1_LAUNCH(S64_, 2, 4); } else { IMIE_Q1_LAUNCH(S64_, 1, 4); }
-#define IMIE_Q1_LAUNCH_PF(S64_, PF_)                                                                         \
-  hipLaunchKernelGGL((q1_gemv_mfma_kernel<S64_, 1, 1, PF_>), grid, dim3(256), lds, st, sgt, xq, tot, ls, nslabs, \
-                     nbp, tn, fr, spk, Lcap, mode, Q1Pro{})
-    if (pers_pro) {
-      Q1Pro pro = {};
-      pro.x = x_dev;
-      pro.cols = K;
-      if (w0.scale64)
-        hipLaunchKernelGGL((q1_gemv_mfma_kernel<true, 4, 1, 0, kProCopy, 256, true>), pgrid, dim3(256), lds, st, sgt,
-                           nullptr, nullptr, nullptr, nslabs, nbp, tn, fr, spk, Lcap, mode, pro);
-      else
-        hipLaunchKernelGGL((q1_gemv_mfma_kernel<false, 4, 1, 0, kProCopy, 256, true>), pgrid, dim3(256), lds, st, sgt,
-                           nullptr, nullptr, nullptr, nslabs, nbp, tn, fr, spk, Lcap, mode, pro);
-    } else if (pers) {
-      if (w0.scale64)
-        hipLaunchKernelGGL((q1_gemv_mfma_kernel<true, 4, 1, 0, kProNone, 256, true>), pgrid, dim3(256), lds, st, sgt,
-                           xq, tot, ls, nslabs, nbp, tn, fr, spk, Lcap, mode, Q1Pro{});
-      else
-        hipLaunchKernelGGL((q1_gemv_mfma_kernel<false, 4, 1, 0, kProNone, 256, true>), pgrid, dim3(256), lds, st, sgt,
-                           xq, tot, ls, nslabs, nbp, tn, fr, spk, Lcap, mode, Q1Pro{});
-    } else if (pf == 4) { if (w0.scale64) IMIE_Q1_LAUNCH_PF(true, 4); else IMIE_Q1_LAUNCH_PF(false, 4); }
-    else if (pf == 2) { if (w0.scale64) IMIE_Q1_LAUNCH_PF(true, 2); else IMIE_Q1_LAUNCH_PF(false, 2); }
-    else if (w0.scale64) { IMIE_Q1_LAUNCH_T(true); } else { IMIE_Q1_LAUNCH_T(false); }
-#undef IMIE_Q1_LAUNCH_PF
-#undef IMIE_Q1_LAUNCH_T
-#undef IMIE_Q1_LAUNCH_R
-#undef IMIE_Q1_LAUNCH
+  for (int i = 0; i < cnt; ++i) sg.out[i] = outs[i];
+  const uint4* xq = (const uint4*)wk.xq.p;
+  const int64_t* tot = (const int64_t*)wk.totals.p;
+  const int* ls = (const int*)wk.lslab.p;
+#define IMIE_Q1_LAUNCH(S64_, R_, PF_)                                                                        \
+  hipLaunchKernelGGL((q1_gemv_mfma_kernel<S64_, R_, PF_>), grid, dim3(256), lds, st, sg, xq, tot, ls, nslabs,  \
+                     nbp, fr, spk, Lcap, mode, Q1Pro{})
+#define IMIE_Q1_LAUNCH_S(S64_)                                                                               \
+  do {                                                                                                       \
+    if (pf == 4) IMIE_Q1_LAUNCH(S64_, 1, 4);                                                                 \
+    else if (pf == 2) IMIE_Q1_LAUNCH(S64_, 1, 2);                                                            \
+    else if (R == 4) IMIE_Q1_LAUNCH(S64_, 4, 0);                                                             \
+    else if (R == 2) IMIE_Q1_LAUNCH(S64_, 2, 0);                                                             \
+    else IMIE_Q1_LAUNCH(S64_, 1, 0);                                                                         \
+  } while (0)
+#define IMIE_Q1_LAUNCH_PERS(S64_, PRO_, ...)                                                                 \
+  hipLaunchKernelGGL((q1_gemv_mfma_kernel<S64_, 4, 0, PRO_, 256, true>), pgrid, dim3(256), lds, st, sg, __VA_ARGS__)
+  if (pers_pro) {
+    Q1Pro pro = {};
+    pro.x = x_dev;
+    pro.cols = K;
+    if (w0.scale64) IMIE_Q1_LAUNCH_PERS(true, kProCopy, nullptr, nullptr, nullptr, nslabs, nbp, fr, spk, Lcap, mode, pro);
+    else IMIE_Q1_LAUNCH_PERS(false, kProCopy, nullptr, nullptr, nullptr, nslabs, nbp, fr, spk, Lcap, mode, pro);
+  } else if (pers) {
+    if (w0.scale64) IMIE_Q1_LAUNCH_PERS(true, kProNone, xq, tot, ls, nslabs, nbp, fr, spk, Lcap, mode, Q1Pro{});
+    else IMIE_Q1_LAUNCH_PERS(false, kProNone, xq, tot, ls, nslabs, nbp, fr, spk, Lcap, mode, Q1Pro{});
+  } else if (w0.scale64) {
+    IMIE_Q1_LAUNCH_S(true);
+  } else {
+    IMIE_Q1_LAUNCH_S(false);
   }
+#undef IMIE_Q1_LAUNCH_PERS
+#undef IMIE_Q1_LAUNCH_S
+#undef IMIE_Q1_LAUNCH
   imie_prof_mark(IMIE_K_Q1_GEMV, st, false);
   IMIE_HIP(hipGetLastError());
   return IMIE_OK;
@@ -2353,8 +2706,8 @@ static int q1_apply_pro(const Q1Weight* const* ws, int cnt, const Q1Pro& pro, in
   const dim3 grid((unsigned)wg_x, (unsigned)ksplit);
   imie_prof_mark(IMIE_K_Q1_GEMV, st, true);
 #define IMIE_Q1_PRO(PF_, PRO_)                                                                                 \
-  hipLaunchKernelGGL((q1_gemv_mfma_kernel<false, 1, 1, PF_, PRO_, NT>), grid, dim3(NT), lds, st, sg, nullptr,   \
-                     nullptr, nullptr, nslabs, nbp, 1, fr, spk, 8, mode, pro)
+  hipLaunchKernelGGL((q1_gemv_mfma_kernel<false, 1, PF_, PRO_, NT>), grid, dim3(NT), lds, st, sg, nullptr,      \
+                     nullptr, nullptr, nslabs, nbp, fr, spk, 8, mode, pro)
 #define IMIE_Q1_PRO_K(PF_)                                                                                     \
   if (kind == kProCopy) IMIE_Q1_PRO(PF_, kProCopy);                                                           \
   else if (kind == kProSiluMul) IMIE_Q1_PRO(PF_, kProSiluMul);                                                \
@@ -2650,7 +3003,7 @@ int imie_q1_apply_dev(int64_t handle, const int64_t* x_dev, int64_t tokens, int6
 // workspace; imie_q1_apply_dev_noalloc takes that workspace from this file-scope array instead of the allocator.
 // Sized for kNaMaxT tokens of up to kNaMaxSlabs 512-column slabs (K <= 32768). Each device holds its own copy for
 // the life of the process; host code reaches it only through the address hipGetSymbolAddress gives on that device.
-constexpr int64_t kNaMaxT = kGemmMinT - 1;
+constexpr int64_t kNaMaxT = 7;
 constexpr int64_t kNaMaxSlabs = 64;
 constexpr size_t kNaXqBytes = (size_t)kNaMaxT * kMaxLimbs * (kNaMaxSlabs * kSlabBlocks) * 8 * 16;
 constexpr size_t kNaTotBytes = (size_t)kNaMaxT * (kNaMaxSlabs * kSlabBlocks) * 8;
