@@ -753,8 +753,30 @@ __global__ __launch_bounds__(256) void dec_final_kernel(AttnDesc d) {
 //   PV    : A = digits of p (limb lp, keys on the K axis), B = V digit plane b (keys x dims)
 // MFMA int32 sums are exact (|D| <= 64 * 128 * 128 per MFMA; partial sums bounded below 2^31 as noted); every
 // recombination into the int64 result wraps mod 2^64 like the oracle's int64 arithmetic.
-// max|K| / max|V| for the fail-loud bounds are the running maxima kept by the cache writes (run_k / run_v).
+// max|K| / max|V| for the fail-loud bounds are the running maxima kept by the cache writes (run_k / run_v). They also
+// say how many digit planes can be nonzero: a cache whose maximum fits three balanced digits (kCap3: every one of an
+// 8B model's, whose normalised keys stay below 2^21) has a zero top plane, which is then neither read nor multiplied --
+// a quarter of the cache's bytes and of the MFMAs. Maxima that a reset clears go on counting in old_k / old_v: slots
+// of an earlier sequence keep their fourth plane for whoever starts behind them. The choice is made per workgroup, as two
+// copies of the loops: a plane loaded under a condition would make the compiler wait for all loads in flight. Decode is
+// bound by the cache's bytes, prefill by MFMA issue; 32 sequences of 512 to 16000 positions: scores 232 -> 183 us, PV
+// 214 -> 170 us a layer; prefill of 2048 rows 362 + 255 -> 326 + 240 us, of 333 rows behind 5000 264 + 194 -> 226 + 167.
 // ---------------------------------------------------------------------------------------------------------
+constexpr uint64_t kCap3 = 127ull * ((256ull * 256 * 256 - 1) / 255);
+// digit planes of a cache with the running maximum `run` and the retired one `old` (nullptr: all four); wave-uniform,
+// by scalar loads (their own counter: no wait for the vector loads in flight)
+__device__ inline uint64_t sload_u64(const uint64_t* p) {
+  const uint64_t a = (uint64_t)p;
+  const uint64_t u = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a) |
+                     ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32)) << 32);
+  return *(const __attribute__((address_space(4))) uint64_t*)u;
+}
+__device__ inline int kv8_planes(const uint64_t* run, const uint64_t* old, int64_t bkv) {
+  if (!run || !old) return 4;
+  const uint64_t a = sload_u64(run + bkv), c = sload_u64(old + bkv);
+  return a <= kCap3 && c <= kCap3 ? 3 : 4;
+}
+
 __device__ inline int64_t bal_digit(int64_t x, int l) {
   for (int i = 0; i < l; ++i) {
     const int64_t dg = ((x + 128) & 255) - 128;
@@ -844,8 +866,10 @@ __global__ __launch_bounds__(256, REP <= 4 ? 3 : 2) void dec_scores8_kernel(Attn
     for (int hb = 0; hb < RBH; ++hb)
       if (pend_i[hb] >= 0) d.scores[pend_i[hb]] = pend_v[hb];
   };
-  auto load_tile = [&](auto pgc, bool live, int64_t t, int64_t lim, v4i (&bk)[4][2]) {   // keys below lim
+  // digit planes D0 .. D1 - 1 of the tile
+  auto load_tile = [&](auto pgc, auto d0c, auto d1c, bool live, int64_t t, int64_t lim, v4i (&bk)[4][2]) {   // keys below lim
     constexpr bool PG = decltype(pgc)::value;
+    constexpr int D0 = decltype(d0c)::value, D1 = decltype(d1c)::value;
     flush();
     const int64_t j = t + m;
     const bool valid = live && j < lim;
@@ -863,7 +887,7 @@ __global__ __launch_bounds__(256, REP <= 4 ? 3 : 2) void dec_scores8_kernel(Attn
     // waits for its load at once. Lanes of keys past `lim` read an in-bounds address (their score columns are
     // never stored); dims at or past hd read dims 0.. of the same slot, which meet zero q digits.
 #pragma unroll
-    for (int db = 0; db < 4; ++db)
+    for (int db = D0; db < D1; ++db)
 #pragma unroll
       for (int h = 0; h < KS; ++h) {
         const int64_t c = 64 * h + 16 * g;
@@ -876,7 +900,8 @@ __global__ __launch_bounds__(256, REP <= 4 ? 3 : 2) void dec_scores8_kernel(Attn
     for (int hb = 0; hb < RBH; ++hb) asm volatile("" ::"v"(pend_v[hb]), "v"(pend_i[hb]));
     __builtin_amdgcn_sched_barrier(0);
   };
-  auto score_tile = [&](int64_t t, const v4i (&bk)[4][2]) {
+  auto score_tile = [&](auto ndc, int64_t t, const v4i (&bk)[4][2]) {
+    constexpr int ND = decltype(ndc)::value;
     const int64_t j = t + m;
     const bool valid = j < jend;
 #pragma unroll
@@ -884,7 +909,7 @@ __global__ __launch_bounds__(256, REP <= 4 ? 3 : 2) void dec_scores8_kernel(Attn
       uint64_t S = 0;
       for (int lb = 0; lb < LB; ++lb)
 #pragma unroll
-        for (int db = 0; db < 4; ++db) {
+        for (int db = 0; db < ND; ++db) {
           v4i D = mfma8(av[hb][lb][0], bk[db][0], v4i{0, 0, 0, 0});
           if constexpr (KS > 1) D = mfma8(av[hb][lb][1], bk[db][1], D);
 #pragma unroll
@@ -906,8 +931,13 @@ __global__ __launch_bounds__(256, REP <= 4 ? 3 : 2) void dec_scores8_kernel(Attn
   // the first K tile in flight during the q setup, bounded by the score row stride rather than the sequence length
   // (no wait for the length): keys past it give scores that are never stored
   const int64_t lim0 = min(j0 + d.chunk, d.Lmax);
-  if (pgreg) load_tile(std::true_type{}, t < lim0, t, lim0, bkA);
-  else load_tile(std::false_type{}, t < lim0, t, lim0, bkA);
+  // three planes; the fourth once the running maximum (a scalar load meanwhile) asks for it
+  using I0 = std::integral_constant<int, 0>;
+  using I3 = std::integral_constant<int, 3>;
+  using I4 = std::integral_constant<int, 4>;
+  if (pgreg) load_tile(std::true_type{}, I0{}, I3{}, t < lim0, t, lim0, bkA);
+  else load_tile(std::false_type{}, I0{}, I3{}, t < lim0, t, lim0, bkA);
+  const int nd = kv8_planes(d.run_k, d.old_k, bkv);
   if (d.qd) {
     // digits prepared by the head stage (all eight limb planes written): A operands straight from memory, loaded
     // together with the limb counts and masked once those arrive
@@ -986,23 +1016,29 @@ __global__ __launch_bounds__(256, REP <= 4 ? 3 : 2) void dec_scores8_kernel(Attn
     for (int lb = 0; lb < 2; ++lb)
 #pragma unroll
       for (int h = 0; h < 2; ++h) asm volatile("" : "+v"(av[hb][lb][h]));
-  auto walk = [&](auto pgc) {
+  auto walk = [&](auto pgc, auto ndc) {
+    if constexpr (decltype(ndc)::value == 4) load_tile(pgc, I3{}, I4{}, t < lim0, t, lim0, bkA);
     // every load so far (the first K tile, the q digits) is complete at the loop's entry: a load still in flight
     // there would make the compiler's wait tracking conservative in every iteration
     __builtin_amdgcn_s_waitcnt(0x0F70);             // vmcnt(0)
     while (t < jend) {
       const int64_t t2 = t + 64;
-      load_tile(pgc, t2 < jend, t2, jend, bkB);
-      score_tile(t, bkA);
+      load_tile(pgc, I0{}, ndc, t2 < jend, t2, jend, bkB);
+      score_tile(ndc, t, bkA);
       if (t2 >= jend) break;
       const int64_t t3 = t2 + 64;
-      load_tile(pgc, t3 < jend, t3, jend, bkA);
-      score_tile(t2, bkB);
+      load_tile(pgc, I0{}, ndc, t3 < jend, t3, jend, bkA);
+      score_tile(ndc, t2, bkB);
       t = t3;
     }
   };
-  if (pgreg) walk(std::true_type{});
-  else walk(std::false_type{});
+  if (nd == 3) {
+    if (pgreg) walk(std::true_type{}, I3{});
+    else walk(std::false_type{}, I3{});
+  } else {
+    if (pgreg) walk(std::true_type{}, I4{});
+    else walk(std::false_type{}, I4{});
+  }
   flush();
 #pragma unroll
   for (int hb = 0; hb < RBH; ++hb) {
@@ -1025,7 +1061,7 @@ __global__ __launch_bounds__(256, REP <= 4 ? 3 : 2) void dec_scores8_kernel(Attn
 // recomputed here from the score and the row maximum (dec_exp_kernel<REP, false> wrote no e); otherwise the
 // scores array holds e_j.
 template <int REP, bool RECOMP>
-__global__ __launch_bounds__(256) void dec_pv8_kernel(AttnDesc d) {
+__global__ __launch_bounds__(256, REP <= 4 ? 3 : 2) void dec_pv8_kernel(AttnDesc d) {
   constexpr int RBH = (REP + 3) / 4;
   __shared__ __align__(16) int8_t sPd[RBH][16][64];
   __shared__ uint64_t s_z[REP], s_mp[4][REP];
@@ -1033,7 +1069,8 @@ __global__ __launch_bounds__(256) void dec_pv8_kernel(AttnDesc d) {
   __shared__ double s_rzd[REP];
   const int64_t bkv = blockIdx.x, b = imie_udiv32(bkv, d.Hkv), kv = imie_umod32(bkv, d.Hkv);
   const int64_t j0 = (int64_t)blockIdx.y * d.chunk;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, m = lane & 15, g = lane >> 4;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), m = lane & 15,
+            g = lane >> 4;
   const int64_t rows = d.B * d.H;
   uint64_t* part = d.part + (int64_t)blockIdx.y * rows * d.hd;
   const int DT = (int)(d.hd / 16);
@@ -1050,30 +1087,38 @@ __global__ __launch_bounds__(256) void dec_pv8_kernel(AttnDesc d) {
   page_split(d, max(j0, min(j0 + d.chunk, d.Lmax) - 1), pi1, pin1);
   const bool pgreg = pi1 - pi0 < 64;
   const int64_t pgl = (pgreg && lane <= pi1 - pi0) ? d.pt[b * d.mp + pi0 + lane] : 0;
-  auto load_step = [&](int64_t t0, int64_t lim, v4i (&bv)[2][4], int64_t (&sc)[RW]) {
+  const int64_t vplane = d.hd * d.P;                  // imie_kv8::v_off(slot, db, c) = db * vplane + c * P + slot
+  const uint32_t voff = (uint32_t)m * (uint32_t)d.P + 16u * (uint32_t)g;   // P < 2^27 (imie_attention_launch)
+  int64_t vtile[2];                                   // a tile past the head dim reads tile 0 (its MFMAs are skipped)
+#pragma unroll
+  for (int tt = 0; tt < 2; ++tt) vtile[tt] = wave + 4 * tt < DT ? 16 * (wave + 4 * tt) * d.P : 0;
+  // digit planes D0 .. D1 - 1 of V; the scores with plane 0
+  auto load_step = [&](auto d0c, auto d1c, int64_t t0, int64_t lim, v4i (&bv)[2][4], int64_t (&sc)[RW]) {
+    constexpr int D0 = decltype(d0c)::value, D1 = decltype(d1c)::value;
     const int64_t tn = min((int64_t)64, lim - t0);
     int64_t pi, slot0;
     page_split(d, t0, pi, slot0);
-    const int64_t pg = pgreg ? (int64_t)imie_readlane_u64((uint64_t)pgl, (int)(pi - pi0)) : d.pt[b * d.mp + pi];
-    const int8_t* vblk = Vb + imie_kv8::block_base(pg, kv, d.Hkv, d.hd, d.P);
+    const int64_t pg = (int64_t)imie_readlane_u64((uint64_t)(pgreg ? pgl : d.pt[b * d.mp + pi]), pgreg ? (int)(pi - pi0) : 0);
+    // a plane is hd * P bytes: scalar addresses and one 32-bit lane offset (no vector address arithmetic)
+    const int8_t* vblk = Vb + imie_kv8::block_base(pg, kv, d.Hkv, d.hd, d.P) + slot0;
 #pragma unroll
-    for (int tt = 0; tt < 2; ++tt) {
-      const int tile = wave + 4 * tt;
+    for (int db = D0; db < D1; ++db)
 #pragma unroll
-      for (int db = 0; db < 4; ++db)
-        bv[tt][db] = tile < DT ? *(const v4i*)(vblk + imie_kv8::v_off(slot0 + 16 * g, db, 16 * tile + m, d.hd, d.P))
-                               : v4i{0, 0, 0, 0};
-    }
+      for (int tt = 0; tt < 2; ++tt) bv[tt][db] = *(const v4i*)(vblk + ((int64_t)db * vplane + vtile[tt]) + voff);
     const int kk = tid & 63;
 #pragma unroll
-    for (int k = 0; k < RW; ++k) {
+    for (int k = 0; k < RW && D0 == 0; ++k) {
       const int r = (tid >> 6) + 4 * k;
       sc[k] = (r < REP && kk < tn) ? d.scores[(b * d.H + kv * REP + r) * d.Lmax + t0 + kk] : 0;
     }
   };
   v4i bvA[2][4], bvB[2][4];
   int64_t scA[RW], scB[RW];
-  load_step(j0, d.Lmax, bvA, scA);
+  using I0 = std::integral_constant<int, 0>;
+  using I3 = std::integral_constant<int, 3>;
+  using I4 = std::integral_constant<int, 4>;
+  load_step(I0{}, I3{}, j0, d.Lmax, bvA, scA);
+  const int nd = kv8_planes(d.run_v, d.old_v, bkv);            // the fourth plane below, if it can be nonzero
   uint64_t cz0[RW];
   int64_t cm0[RW];
 #pragma unroll
@@ -1117,7 +1162,6 @@ __global__ __launch_bounds__(256) void dec_pv8_kernel(AttnDesc d) {
   const bool fx32 = (d.dclip >> 32) == 0 && (d.log2e >> 32) == 0;
   for (int i = tid; i < RBH * 16 * 64; i += 256) (&sPd[0][0][0])[i] = 0;
   __syncthreads();
-  const int Lp = imie_limbs_needed((uint64_t)1 << d.frac);
   uint64_t mp[REP];
 #pragma unroll
   for (int r = 0; r < REP; ++r) mp[r] = 0;
@@ -1126,66 +1170,69 @@ __global__ __launch_bounds__(256) void dec_pv8_kernel(AttnDesc d) {
   for (int hb = 0; hb < RBH; ++hb)
 #pragma unroll
     for (int db = 0; db < 4; ++db) acc[hb][db][0] = acc[hb][db][1] = v4i{0, 0, 0, 0};
-  for (int64_t t0 = j0; t0 < jend; t0 += 64) {
-    const int64_t tn = min((int64_t)64, jend - t0);
-    v4i bv[2][4];
-    int64_t scv[RW];
-#pragma unroll
-    for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-      for (int db = 0; db < 4; ++db) bv[tt][db] = bvA[tt][db];
-#pragma unroll
-    for (int k = 0; k < RW; ++k) scv[k] = scA[k];
-    if (t0 + 64 < jend) {
-      load_step(t0 + 64, jend, bvB, scB);
+  auto walk = [&](auto ndc) {
+  constexpr int ND = decltype(ndc)::value;
+  if constexpr (ND == 4) load_step(I3{}, I4{}, j0, d.Lmax, bvA, scA);
+    for (int64_t t0 = j0; t0 < jend; t0 += 64) {
+      const int64_t tn = min((int64_t)64, jend - t0);
+      v4i bv[2][4];
+      int64_t scv[RW];
 #pragma unroll
       for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
-        for (int db = 0; db < 4; ++db) bvA[tt][db] = bvB[tt][db];
+        for (int db = 0; db < ND; ++db) bv[tt][db] = bvA[tt][db];
 #pragma unroll
-      for (int k = 0; k < RW; ++k) scA[k] = scB[k];
-    }
-    __syncthreads();                                  // previous step's digits consumed
-    {
-      const int kk = tid & 63;
+      for (int k = 0; k < RW; ++k) scv[k] = scA[k];
+      if (t0 + 64 < jend) {
+        load_step(I0{}, ndc, t0 + 64, jend, bvB, scB);
 #pragma unroll
-      for (int k = 0; k < RW; ++k) {
-        const int r = (tid >> 6) + 4 * k;
-        if (r >= REP) break;
-        const uint64_t Z = s_z[r];
-        int64_t p = 0;
-        if (kk < tn && Z != 0) {
-          int64_t e = scv[k];
-          if (RECOMP) {                                  // e_j of dec_exp_kernel from the score and the row maximum
-            int64_t dd = (int64_t)((uint64_t)s_m[r] - (uint64_t)scv[k]);
-            if (dd > d.dclip) dd = d.dclip;
-            e = exp_clipped(dd, d.frac, d.log2e, fx32);
+        for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+          for (int db = 0; db < ND; ++db) bvA[tt][db] = bvB[tt][db];
+#pragma unroll
+        for (int k = 0; k < RW; ++k) scA[k] = scB[k];
+      }
+      __syncthreads();                                  // previous step's digits consumed
+      {
+        const int kk = tid & 63;
+#pragma unroll
+        for (int k = 0; k < RW; ++k) {
+          const int r = (tid >> 6) + 4 * k;
+          if (r >= REP) break;
+          const uint64_t Z = s_z[r];
+          int64_t p = 0;
+          if (kk < tn && Z != 0) {
+            int64_t e = scv[k];
+            if (RECOMP) {                                  // e_j of dec_exp_kernel from the score and the row maximum
+              int64_t dd = (int64_t)((uint64_t)s_m[r] - (uint64_t)scv[k]);
+              if (dd > d.dclip) dd = d.dclip;
+              e = exp_clipped(dd, d.frac, d.log2e, fx32);
+            }
+            p = prob_div(e, d.frac, Z, s_rzd[r]);
           }
-          p = prob_div(e, d.frac, Z, s_rzd[r]);
-        }
-        mp[r] = (uint64_t)p > mp[r] ? (uint64_t)p : mp[r];
-        int64_t x = p;
-        for (int lp = 0; lp < 4; ++lp) {
-          const int64_t dg = ((x + 128) & 255) - 128;
-          x = (int64_t)((uint64_t)x - (uint64_t)dg) >> 8;
-          sPd[r >> 2][4 * (r & 3) + lp][kk] = lp < Lp ? (int8_t)dg : (int8_t)0;
+          mp[r] = (uint64_t)p > mp[r] ? (uint64_t)p : mp[r];
+          const uint32_t dg = imie_digits32((uint32_t)p);       // 0 <= p <= 2^frac, frac <= 29: digits at or above Lp are 0
+#pragma unroll
+          for (int lp = 0; lp < 4; ++lp) sPd[r >> 2][4 * (r & 3) + lp][kk] = (int8_t)(uint8_t)(dg >> (8 * lp));
         }
       }
+      __syncthreads();
+      v4i av[RBH];
+#pragma unroll
+      for (int hb = 0; hb < RBH; ++hb) av[hb] = *(const v4i*)&sPd[hb][m][16 * g];
+#pragma unroll
+      for (int tt = 0; tt < 2; ++tt) {
+        const int tile = wave + 4 * tt;
+        if (tile >= DT) continue;
+#pragma unroll
+        for (int db = 0; db < ND; ++db)
+#pragma unroll
+          for (int hb = 0; hb < RBH; ++hb) acc[hb][db][tt] = mfma8(av[hb], bv[tt][db], acc[hb][db][tt]);
+      }
     }
-    __syncthreads();
-    v4i av[RBH];
-#pragma unroll
-    for (int hb = 0; hb < RBH; ++hb) av[hb] = *(const v4i*)&sPd[hb][m][16 * g];
-#pragma unroll
-    for (int tt = 0; tt < 2; ++tt) {
-      const int tile = wave + 4 * tt;
-      if (tile >= DT) continue;
-#pragma unroll
-      for (int db = 0; db < 4; ++db)
-#pragma unroll
-        for (int hb = 0; hb < RBH; ++hb) acc[hb][db][tt] = mfma8(av[hb], bv[tt][db], acc[hb][db][tt]);
-    }
-  }
+  };
+  if (nd == 3) walk(I3{});
+  else walk(I4{});
 #pragma unroll
   for (int r = 0; r < REP; ++r) {
     const uint64_t mm = imie_wave_max_u64(mp[r]);
@@ -1701,9 +1748,10 @@ struct FfShared {
   int8_t sP[2][4][kFfRows][kFfPad];                            // p digit planes of one key step, double buffer
   uint64_t s_red[8][kFfRows];
   uint64_t s_mq[kFfRows];
+  int hot[2];                                                  // number of the last step with a p beyond two digits
 };
 
-template <int LQ, int HD, bool F32, int PASSES, int NW>
+template <int LQ, int HD, bool F32, int PASSES, int NW, int ND = 4>
 __device__ __forceinline__ void pf_fused8_body(const AttnDesc& d, FfShared& S, int64_t b, int64_t h, int64_t kv, int64_t pt,
                                int64_t row0, int64_t len);
 
@@ -1782,9 +1830,16 @@ __global__ __launch_bounds__(64 * NW) void pf_fused8_kernel(AttnDesc d) {
                       d.dclip >= 0 && d.dclip < ((int64_t)1 << 20) && d.log2e >= 0 && d.log2e < ((int64_t)1 << 17) &&
                       (u128)mqa * d.run_k[bkv] * 128 < ((u128)1 << 47);
     if (tid == 0) d.rowmax[blockIdx.x] = fast ? 0 : 1;
-    if (fast) pf_fused8_body<3, 128, true, 1, NW>(d, S, b, h, kv, pt, row0, len);
+    if (fast) {
+      if (kv8_planes(d.run_k, d.old_k, bkv) == 3)
+        pf_fused8_body<3, 128, true, 1, NW, 3>(d, S, b, h, kv, pt, row0, len);
+      else pf_fused8_body<3, 128, true, 1, NW, 4>(d, S, b, h, kv, pt, row0, len);
+    }
   } else if (MODE == 2) {
-    pf_fused8_body<3, 128, true, 2, NW>(d, S, b, h, kv, pt, row0, len);
+    if (kv8_planes(d.run_k, d.old_k, bkv) == 3 && kv8_planes(d.run_v, d.old_v, bkv) == 3)
+      pf_fused8_body<3, 128, true, 2, NW, 3>(d, S, b, h, kv, pt, row0, len);
+    else
+      pf_fused8_body<3, 128, true, 2, NW, 4>(d, S, b, h, kv, pt, row0, len);
   } else {
     pf_fused8_body<8, 0, false, 3, NW>(d, S, b, h, kv, pt, row0, len);  // any hd (multiple of 16, <= 128), any limbs
   }
@@ -1799,7 +1854,7 @@ __global__ __launch_bounds__(64 * NW) void pf_fused8_kernel(AttnDesc d) {
 // 3 = all three in one launch.
 // NW waves: wave w scores keys 16 w .. 16 w + 15 of every 16 NW-key step and (pass 3) owns 8 / NW of the 16-dim
 // output tiles.
-template <int LQ, int HD, bool F32, int PASSES, int NW>
+template <int LQ, int HD, bool F32, int PASSES, int NW, int ND>
 __device__ __forceinline__ void pf_fused8_body(const AttnDesc& d, FfShared& S, int64_t b, int64_t h, int64_t kv, int64_t pt,
                                int64_t row0, int64_t len) {
   constexpr int STEP = 16 * NW, DPW = 8 / NW, KSP = NW / 4;   // keys per step, dim tiles per wave, 64-key K steps
@@ -1807,13 +1862,13 @@ __device__ __forceinline__ void pf_fused8_body(const AttnDesc& d, FfShared& S, i
   auto& sP = S.sP;
   auto& s_red = S.s_red;
   auto& s_mq = S.s_mq;
-  constexpr int NE = LQ + 3 < 8 ? LQ + 3 : 8;                 // exponents lq + db below 8 (256^8 = 0 mod 2^64)
+  constexpr int NE = LQ + ND - 1 < 8 ? LQ + ND - 1 : 8;       // exponents lq + db below 8 (256^8 = 0 mod 2^64)
   // F32: scores, row maxima, Z (at most 16384 keys: Z < 2^30) and p (<= 2^16) in 32 bits, 3 p limbs
   using ST = std::conditional_t<F32, int32_t, int64_t>;
   using UT = std::conditional_t<F32, uint32_t, uint64_t>;
   constexpr ST SMIN = F32 ? (ST)INT32_MIN : (ST)INT64_MIN;
   constexpr UT SBIT = (UT)1 << (8 * sizeof(UT) - 1);
-  constexpr int NTP = F32 ? 6 : 7;                             // PV exponents lp + db (lp < 3 when F32)
+  constexpr int NTP = (F32 ? 3 : 4) + ND - 1;                  // PV exponents lp + db (lp < 3 when F32)
   const int64_t bkv = b * d.Hkv + kv;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), m = lane & 15, g = lane >> 4;
   auto row_lv = [&](int i) -> int64_t {                         // keys visible to tile row i (0: no row)
@@ -1842,7 +1897,7 @@ __device__ __forceinline__ void pf_fused8_body(const AttnDesc& d, FfShared& S, i
                          imie_kv8::k_off(slot, 0, 0, HDv);
     // keys past the sequence length are loaded from their (allocated) slots and masked where the scores are used
 #pragma unroll
-    for (int db = 0; db < 4; ++db)
+    for (int db = 0; db < ND; ++db)
 #pragma unroll
       for (int hh = 0; hh < 2; ++hh) {
         if (hh >= KS) { bk[db][hh] = v4i{0, 0, 0, 0}; continue; }
@@ -1883,7 +1938,7 @@ __device__ __forceinline__ void pf_fused8_body(const AttnDesc& d, FfShared& S, i
       const v4i a0 = QREG ? qreg[QREG ? lq : 0][0] : q_operand(lq, 0);
       const v4i a1 = QREG ? qreg[QREG ? lq : 0][1] : q_operand(lq, 1);
 #pragma unroll
-      for (int db = 0; db < 4; ++db) {
+      for (int db = 0; db < ND; ++db) {
         if (lq + db >= NE) continue;
         v4i x = TR ? mfma8(bk[db][0], a0, T[lq + db]) : mfma8(a0, bk[db][0], T[lq + db]);
         if (KS > 1) x = TR ? mfma8(bk[db][1], a1, x) : mfma8(a1, bk[db][1], x);
@@ -1894,10 +1949,10 @@ __device__ __forceinline__ void pf_fused8_body(const AttnDesc& d, FfShared& S, i
     for (int i = 0; i < 4; ++i) {
       int64_t s;
       if constexpr (F32) {
-        static_assert(NE == 6, "3 q limbs");
+        static_assert(NE == 6 || NE == 5, "3 q limbs");
         const uint32_t U0 = (uint32_t)T[0][i] + ((uint32_t)T[1][i] << 8);
         const uint32_t U1 = (uint32_t)T[2][i] + ((uint32_t)T[3][i] << 8);
-        const uint32_t U2 = (uint32_t)T[4][i] + ((uint32_t)T[5][i] << 8);
+        const uint32_t U2 = (uint32_t)T[4][i] + (NE > 5 ? (uint32_t)T[NE - 1][i] << 8 : 0u);
         const int32_t V = (int32_t)(U1 + (U2 << 16) + (uint32_t)((int32_t)U0 >> 16));
         s = (int64_t)V * (int32_t)d.inv_sqrt >> 16;
       } else {
@@ -2101,7 +2156,7 @@ __device__ __forceinline__ void pf_fused8_body(const AttnDesc& d, FfShared& S, i
       for (int tt = 0; tt < DPW; ++tt) {
         const int tile = DPW * wave + tt;
 #pragma unroll
-        for (int db = 0; db < 4; ++db) {
+        for (int db = 0; db < ND; ++db) {
           const uint32_t off = ((uint32_t)db * (uint32_t)HDv + (uint32_t)(16 * tile + m)) * (uint32_t)d.P + 16u * g;
           bv[tt][ks][db] = (ALLT || tile < DT) ? ld16u(vs, off, (uint32_t)(4 * HDv * d.P)) : v4i{0, 0, 0, 0};
         }
@@ -2119,32 +2174,37 @@ __device__ __forceinline__ void pf_fused8_body(const AttnDesc& d, FfShared& S, i
     if (t < vis) scores(t, bk, sc, std::true_type{});
     // issued whatever the next step is (past vis: this tile again; see walk)
     load_k(t + STEP < vis ? t + STEP : (t < vis ? t : 16 * wave), bk);
-    uint32_t pk[4] = {0, 0, 0, 0};                              // per limb: the digits of keys 4 g .. 4 g + 3
+    uint32_t pk[4], dg[4];                                      // per limb: the digits of keys 4 g .. 4 g + 3
+    UT pmx = 0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int64_t e = expv(sc[i], i);
       const int64_t p = probv(e, i);
-      mp[0] = (UT)p > mp[0] ? (UT)p : mp[0];
-      // balanced base-256 digits of 0 <= p <= 2^frac < 2^30: the bytes of p + 0x80808080, each less 0x80
-      const uint32_t dg = ((uint32_t)p + 0x80808080u) ^ 0x80808080u;
-#pragma unroll
-      for (int lp = 0; lp < 4; ++lp) pk[lp] |= ((dg >> (8 * lp)) & 0xFFu) << (8 * i);
+      pmx = (UT)p > pmx ? (UT)p : pmx;
+      dg[i] = imie_digits32((uint32_t)p);                       // 0 <= p <= 2^frac < 2^30
     }
+    imie_bytes4x4(dg[0], dg[1], dg[2], dg[3], pk);
+    mp[0] = pmx > mp[0] ? pmx : mp[0];
+    // F32: p beyond two balanced digits (above 32639, about one half at frac 16) is rare; a step that has none skips
+    // the third limb's MFMAs. The flag holds the number of its step, so it needs no clearing (a stale value of an
+    // earlier tile costs only the MFMAs).
+    if (F32 && __any(pmx > 32639) && lane == 0) S.hot[buf] = (int)(t0 / STEP) + 1;
 #pragma unroll
     for (int lp = 0; lp < 4; ++lp)                            // one 4-byte store per limb: row m, 4 keys
       if (lp < Lp) *(uint32_t*)&sP[buf][lp][m][16 * wave + 4 * g] = pk[lp];
     __syncthreads();                                          // the step's p digits are in LDS
+    const bool third = !F32 || __builtin_amdgcn_readfirstlane(S.hot[buf]) == (int)(t0 / STEP) + 1;
 #pragma unroll
     for (int ks = 0; ks < KSP; ++ks)
 #pragma unroll
       for (int lp = 0; lp < 4; ++lp) {
-        if (lp >= Lp) break;
+        if (lp >= Lp || (lp == 2 && !third)) break;
         const v4i a = *(const v4i*)&sP[buf][lp][m][64 * ks + 16 * g];
 #pragma unroll
         for (int tt = 0; tt < DPW; ++tt) {
           if (!ALLT && DPW * wave + tt >= DT) continue;
 #pragma unroll
-          for (int db = 0; db < 4; ++db)
+          for (int db = 0; db < ND; ++db)
             if (lp + db < NTP) Tp[tt][lp + db] = mfma8(a, bv[tt][ks][db], Tp[tt][lp + db]);
         }
       }
@@ -2347,7 +2407,7 @@ int imie_attention_launch(AttnDesc d, hipStream_t st) {
     return IMIE_OK;
   }
   if (d.kv32) {                                      // kv8 prefill: MFMA scores, softmax to p digits, MFMA PV
-    if (d.hd % 16 != 0 || !d.run_k || !d.run_v) return IMIE_EARG;
+    if (d.hd % 16 != 0 || !d.run_k || !d.run_v || d.P >= ((int64_t)1 << 27)) return IMIE_EARG;
     if (d.hd <= 128 && pf_fused()) {
       const int64_t npt = (d.M + kFfRows - 1) / kFfRows;
       if (d.hd == 128) {

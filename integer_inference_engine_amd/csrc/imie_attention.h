@@ -10,6 +10,7 @@ struct AttnDesc {
   const void* V;
   int kv32;                        // 1: kv8 digit-plane cache (imie_kvfmt.h), 0: int64 elements
   const uint64_t *run_k, *run_v;   // kv8: running max|K|, max|V| per (sequence, kv head) [B*Hkv]
+  const uint64_t *old_k, *old_v;   // kv8: the maxima that resets have cleared (nullptr: unknown), same layout
   const int8_t* qd;                // kv8 decode (optional): q digit planes [B*H][8][hd] from the head stage
   const int* qlimbs;               //   and their limb counts [B*H] (maxq then points at the head stage's max|q|)
   const int64_t* pt;               // page table [B][mp]

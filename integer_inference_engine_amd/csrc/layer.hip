@@ -81,6 +81,14 @@ int fill_i64(int64_t* p, int64_t n, int64_t v, hipStream_t st) {
   return IMIE_OK;
 }
 
+// a reset: the running maxima start again at 0, what they were is folded into the maxima of old slots
+__global__ void kv_retire_kernel(uint64_t* __restrict__ run, uint64_t* __restrict__ old, int64_t n) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n) return;
+  if (run[i] > old[i]) old[i] = run[i];
+  run[i] = 0;
+}
+
 // Seeded synthetic cache contents: element i (flattened (kv, j, c) of the (Hkv, len, hd) tensor of one layer,
 // kind 0 = K / 1 = V, and sequence b) is uniform in [lo, lo + span) from the counter-based SplitMix64 stream keyed
 // by (seed, 100000 + 1024 layer + 512 kind + sequence id) -- the same draw as the host generator's uniform_int.
@@ -148,7 +156,8 @@ struct Net {
   // workspace
   DevBuf n, q, k, v, qn, kn, att, gate, up, h, pos, starts, attn, guard, status, x, logits, ids, lastx, amx, stepc;
   DevBuf gtab, gmax;                  // device table of the 2 * nl RMSNorm gains (n1g, n2g per layer), their max |g|
-  DevBuf kvrun;                       // kv8: running max|K|, max|V| per (layer, sequence, kv head): [nl][2][B*Hkv]
+  DevBuf kvrun;                       // kv8: running max|K|, max|V| per (layer, sequence, kv head): [nl][2][B*Hkv],
+                                      // then the maxima that resets have cleared (the slots' old values stay)
   DevBuf kvrow;                       // kv8: appended rows' maxima [2][rows*Hkv]
   DevBuf gpart;                       // many-row head stage: per-(row, head) RoPE envelope maxima [rows][H+Hkv][2]
   Q1Ws q1w;                           // this net's Q1 workspace (graph-stable addresses)
@@ -228,7 +237,7 @@ int net_alloc_kv(Net& n, const std::vector<int64_t>& caps, int64_t P, int kv32) 
   IMIE_HIP(hipMemcpy(n.pt, pt.data(), pt.size() * 8, hipMemcpyHostToDevice));
   n.len.assign((size_t)n.B, 0);
   if (kv32) {
-    const size_t rb = (size_t)(n.nl * 2 * n.B * n.Hkv) * 8;
+    const size_t rb = (size_t)(2 * n.nl * 2 * n.B * n.Hkv) * 8;
     if (n.kvrun.ensure(rb)) return IMIE_EARG;
     IMIE_HIP(hipMemset(n.kvrun.p, 0, rb));
   }
@@ -242,6 +251,8 @@ int64_t pos_cap(const Net& n, int64_t b) { return std::min(seq_cap(n, b), n.rope
 
 uint64_t* run_k(Net& n, int64_t l) { return (uint64_t*)n.kvrun.p + (l * 2) * n.B * n.Hkv; }
 uint64_t* run_v(Net& n, int64_t l) { return (uint64_t*)n.kvrun.p + (l * 2 + 1) * n.B * n.Hkv; }
+uint64_t* old_k(Net& n, int64_t l) { return run_k(n, l) + n.nl * 2 * n.B * n.Hkv; }
+uint64_t* old_v(Net& n, int64_t l) { return run_v(n, l) + n.nl * 2 * n.B * n.Hkv; }
 
 // Workspace for rows = B * M new rows attending over at most lmax keys.
 int net_ensure(Net& n, int64_t M, int64_t lmax) {
@@ -374,7 +385,10 @@ int net_run_core(Net& n, int64_t* x, int64_t M, int64_t lmax, hipStream_t st) {
     d.starts = (const int64_t*)n.starts.p; d.lengths = nullptr;
     d.Lmax = lmax; d.frac = (int)n.frac; d.inv_sqrt = n.inv_sqrt;
     d.out = att; d.status = status; d.rope_guard = guard + 4 * l;
-    if (n.kv32) { d.run_k = run_k(n, l); d.run_v = run_v(n, l); }
+    if (n.kv32) {
+      d.run_k = run_k(n, l); d.run_v = run_v(n, l);
+      d.old_k = old_k(n, l); d.old_v = old_v(n, l);
+    }
     imie_attn_bind_scratch(d, n.attn.p);
     if (n.kv32 && M == 1) imie_attn_qdigit_scratch(d, (int8_t**)&d.qd, (int**)&d.qlimbs);
     {
@@ -936,7 +950,13 @@ int imie_net_reset(int64_t ctx) {
   if (!n) return IMIE_EARG;
   IMIE_HIP(hipDeviceSynchronize());
   n->len.assign((size_t)n->B, 0);
-  if (n->kv32 && n->kvrun.p) IMIE_HIP(hipMemset(n->kvrun.p, 0, (size_t)(n->nl * 2 * n->B * n->Hkv) * 8));
+  const int64_t nr = n->nl * 2 * n->B * n->Hkv;
+  if (n->kv32 && n->kvrun.p && nr > 0) {
+    hipLaunchKernelGGL(kv_retire_kernel, dim3((unsigned)((nr + 255) / 256)), dim3(256), 0, imie_stream(),
+                       (uint64_t*)n->kvrun.p, (uint64_t*)n->kvrun.p + nr, nr);
+    IMIE_HIP(hipGetLastError());
+    IMIE_HIP(hipStreamSynchronize(imie_stream()));
+  }
   return IMIE_OK;
 }
 
