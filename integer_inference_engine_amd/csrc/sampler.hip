@@ -155,71 +155,161 @@ __device__ inline uint64_t smp_sha256_first8(const uint32_t m[16]) {
   return ((uint64_t)(0x6a09e667u + a) << 32) | (uint64_t)(0xbb67ae85u + b);
 }
 
-// One SHA-256 compression of a 64-byte block (w[0..15] big-endian message words) into the running state
-__device__ inline void smp_sha256_compress(uint32_t st[8], uint32_t w[16]) {
-  uint32_t a = st[0], b = st[1], c = st[2], d = st[3], e = st[4], f = st[5], g = st[6], h = st[7];
-#pragma unroll
-  for (int i = 0; i < 64; ++i) {
-    uint32_t wi;
-    if (i < 16) {
-      wi = w[i];
-    } else {                                          // rolling 16-word schedule
-      const uint32_t w15 = w[(i - 15) & 15], w2 = w[(i - 2) & 15];
-      const uint32_t s0 = smp_rotr(w15, 7) ^ smp_rotr(w15, 18) ^ (w15 >> 3);
-      const uint32_t s1 = smp_rotr(w2, 17) ^ smp_rotr(w2, 19) ^ (w2 >> 10);
-      wi = w[i & 15] + s0 + w[(i - 7) & 15] + s1;
-      w[i & 15] = wi;
-    }
-    const uint32_t S1 = smp_rotr(e, 6) ^ smp_rotr(e, 11) ^ smp_rotr(e, 25);
-    const uint32_t ch = (e & f) ^ (~e & g);
-    const uint32_t t1 = h + S1 + ch + kSha256K[i] + wi;
-    const uint32_t S0 = smp_rotr(a, 2) ^ smp_rotr(a, 13) ^ smp_rotr(a, 22);
-    const uint32_t mj = (a & b) ^ (a & c) ^ (b & c);
-    h = g; g = f; f = e; e = d + t1; d = c; c = b; b = a; a = t1 + S0 + mj;
-  }
-  st[0] += a; st[1] += b; st[2] += c; st[3] += d; st[4] += e; st[5] += f; st[6] += g; st[7] += h;
+// logits_digest (sampler.py:421-425): SHA-256 of a row's little-endian int64 bytes. Bound by the serial chain of rounds
+// (64 a block, 18993 blocks for a row of 151936 values) at one instruction per four cycles and more, so what counts is
+// the instructions of a round. Two waves a workgroup of 32 rows:
+// * wave 1 expands the message schedules, W + K, into LDS, two blocks of each row at a time, one phase ahead;
+// * wave 0 runs the rounds with two lanes per row: the even lane holds (a, b, c, d), the odd lane (e, f, g, h), and both
+//   halves of a round are the same nine instructions. The even lane works two rounds behind the odd one, which needs
+//   only a value of three rounds ago from it: the odd lane's e' = S1(e) + ch + h + W + K + d takes d = a of round i - 3
+//   (the even lane's second word), the even lane's a' = S0(a) + maj + T1 takes T1 = e' - d of its own round (the odd
+//   lane's second word less its own fourth). The exchange is one quad_perm add off the critical path.
+// At a block's first two steps the odd lane already runs the next block while the even one ends the last.
+// One lane per row with rounds and schedule in one wave, 25 instructions a round, took 62.6 ms for 256 rows of 151936;
+// this takes 27.1 (22 ns a round, five cycles an instruction: more rows a wave or more waves change nothing).
+constexpr int kDigestRows = 32;
+
+struct DigestLane {                                    // per-lane constants of the two halves
+  uint32_t mA, mB;                                     // all ones in the even / odd lane
+  uint32_t r0, r1, r2;                                 // rotations of S0 / S1
+};
+
+__device__ __forceinline__ uint32_t digest_swap(uint32_t x) {   // the pair's other lane (quad_perm [1, 0, 3, 2])
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0xB1, 0xF, 0xF, true);
 }
 
-// logits_digest (sampler.py:421-425): SHA-256 of a row's little-endian int64 bytes, one lane per row. The
-// message is vocab * 8 bytes, so whole 8-byte values fill the blocks and the tail holds 0..7 values.
-__global__ __launch_bounds__(64) void smp_digest_kernel(const int64_t* __restrict__ x, int64_t rows, int64_t vocab,
-                                                        int64_t ld, uint32_t* __restrict__ out) {
-  const int64_t r = (int64_t)blockIdx.x * 64 + threadIdx.x;
-  if (r >= rows) return;
-  const uint64_t* p = reinterpret_cast<const uint64_t*>(x + r * ld);
-  uint32_t st[8] = {0x6a09e667u, 0xbb67ae85u, 0x3c6ef372u, 0xa54ff53au,
-                    0x510e527fu, 0x9b05688cu, 0x1f83d9abu, 0x5be0cd19u};
-  uint32_t w[16];
-  const int64_t full = vocab / 8;                     // 8 values = one 64-byte block
-  for (int64_t blk = 0; blk < full; ++blk) {
-    uint64_t v[8];
+// one step: the new first word; v: the half's four words, x: what the other lane adds (swapped), kw: W + K (even: 1)
+__device__ __forceinline__ uint32_t digest_step(const DigestLane& c, uint32_t v0, uint32_t v1, uint32_t v2, uint32_t v3,
+                                                uint32_t x, uint32_t kw) {
+  const uint32_t S = (uint32_t)__builtin_amdgcn_bitop3_b32(
+      (int)__builtin_amdgcn_alignbit(v0, v0, c.r0), (int)__builtin_amdgcn_alignbit(v0, v0, c.r1),
+      (int)__builtin_amdgcn_alignbit(v0, v0, c.r2), 0x96);                                    // xor of the three
+  const uint32_t sel = (uint32_t)__builtin_amdgcn_bitop3_b32((int)v0, (int)v1, (int)c.mB, 0x1E);   // v0 ^ (v1 | mB):
+                                                       // even a ^ b, odd ~e
+  const uint32_t F = (sel & v2) | (~sel & v1);         // even maj(a, b, c), odd ch(e, f, g)
+  // even T1 = swap - v3, odd h + W + K + d: one xor-add and one quad_perm add (the empty asm keeps the sums apart)
+  uint32_t pre = (v3 ^ c.mA) + kw;
+  asm("" : "+v"(pre));
+  pre += digest_swap(x);
+  asm("" : "+v"(pre));
+  return S + F + pre;
+}
+
+__global__ __launch_bounds__(128) void smp_digest_kernel(const int64_t* __restrict__ x, int64_t rows, int64_t vocab,
+                                                         int64_t ld, uint32_t* __restrict__ out) {
+  __shared__ uint4 s_kw[2][2][16][64];                 // [buffer][block of the phase][four rounds][lane]
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int64_t row0 = (int64_t)blockIdx.x * kDigestRows;
+  const int64_t full = vocab / 8;                      // 8 values = one 64-byte block
+  const int tail = (int)(vocab - full * 8);            // 0..7 values left, then the pad byte and the length
+  const int64_t nblk = full + (tail >= 7 ? 2 : 1), nph = (nblk + 1) / 2;
+  for (int i = tid; i < 2 * 2 * 16 * 32; i += 128) (&s_kw[0][0][0][0])[2 * i] = uint4{1, 1, 1, 1};   // even lanes
+  // wave 1: lane = (block of the phase, row)
+  const int hb = lane >> 5, lr = lane & 31;
+  const uint64_t* p = (const uint64_t*)(x + min(row0 + lr, rows - 1) * ld);
+  uint64_t v[8];
+  auto fetch = [&](int64_t ph) {                       // the values of block 2 ph + hb, 0 past the row
+    const int64_t k0 = (2 * ph + hb) * 8;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] = __builtin_nontemporal_load(p + blk * 8 + j);
+    for (int j = 0; j < 8; ++j) v[j] = k0 + j < vocab ? p[k0 + j] : 0;
+  };
+  auto expand = [&](int64_t ph) {
+    const int64_t blk = 2 * ph + hb;
+    uint32_t w[16];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       w[2 * j] = __builtin_bswap32((uint32_t)v[j]);
       w[2 * j + 1] = __builtin_bswap32((uint32_t)(v[j] >> 32));
+      if (blk * 8 + j == vocab) w[2 * j] = 0x80000000u;
     }
-    smp_sha256_compress(st, w);
-  }
-  const int tail = (int)(vocab - full * 8);           // 0..7 values left
+    if (blk == nblk - 1) {
+      w[14] = (uint32_t)((uint64_t)vocab * 64 >> 32);
+      w[15] = (uint32_t)((uint64_t)vocab * 64);
+    }
+    fetch(ph + 1);
+    uint4* dst = &s_kw[ph & 1][hb][0][2 * lr + 1];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {                       // static indices keep w in registers
-    const uint64_t v = j < tail ? p[full * 8 + j] : 0;
-    w[2 * j] = j < tail ? __builtin_bswap32((uint32_t)v) : (j == tail ? 0x80000000u : 0u);   // 0x80 pad byte
-    w[2 * j + 1] = j < tail ? __builtin_bswap32((uint32_t)(v >> 32)) : 0u;
-  }
-  const uint64_t bits = (uint64_t)vocab * 64;
-  if (tail >= 7) {                                    // no room for the 8-byte length: one more block
-    smp_sha256_compress(st, w);
+    for (int q = 0; q < 16; ++q) {
+      uint32_t o[4];
 #pragma unroll
-    for (int j = 0; j < 16; ++j) w[j] = 0;
+      for (int k = 0; k < 4; ++k) {
+        const int i = 4 * q + k;
+        if (i >= 16) {                                 // rolling 16-word schedule
+          const uint32_t w15 = w[(i - 15) & 15], w2 = w[(i - 2) & 15];
+          const uint32_t s0 = smp_rotr(w15, 7) ^ smp_rotr(w15, 18) ^ (w15 >> 3);
+          const uint32_t s1 = smp_rotr(w2, 17) ^ smp_rotr(w2, 19) ^ (w2 >> 10);
+          w[i & 15] = w[i & 15] + s0 + w[(i - 7) & 15] + s1;
+        }
+        o[k] = w[i & 15] + kSha256K[i];
+      }
+      dst[q * 64] = uint4{o[0], o[1], o[2], o[3]};
+    }
+  };
+  // wave 0
+  const bool odd = lane & 1;
+  DigestLane c;
+  c.mB = odd ? 0xFFFFFFFFu : 0u;
+  c.mA = ~c.mB;
+  c.r0 = odd ? 6 : 2; c.r1 = odd ? 11 : 13; c.r2 = odd ? 25 : 22;
+  const uint32_t i0 = 0x6a09e667u, i1 = 0xbb67ae85u, i2 = 0x3c6ef372u, i3 = 0xa54ff53au;
+  // hA: the hash's a..d in even lanes (0 in odd), hB: e..h in odd lanes (0 in even); v: the running words
+  uint32_t hA[4] = {i0 & c.mA, i1 & c.mA, i2 & c.mA, i3 & c.mA};
+  uint32_t hB[4] = {0x510e527fu & c.mB, 0x9b05688cu & c.mB, 0x1f83d9abu & c.mB, 0x5be0cd19u & c.mB};
+  uint32_t v0 = 0, v1 = 0, v2 = 0, v3 = 0;
+  // steps 0 and 1 of a block: the odd lanes add the hash and begin it; the even lanes end the last block and add theirs
+  // (first: there is none, they take the initial hash)
+  auto begin = [&](uint32_t kw0, uint32_t kw1, bool first) {
+    const uint32_t r0 = v0, r1 = v1;
+    v0 += hB[0]; v1 += hB[1]; v2 += hB[2]; v3 += hB[3];
+    hB[0] = v0 & c.mB; hB[1] = v1 & c.mB; hB[2] = v2 & c.mB; hB[3] = v3 & c.mB;
+    const uint32_t n0 = digest_step(c, v0, v1, v2, v3, r1, kw0 + digest_swap(hA[3]));
+    const uint32_t n1 = digest_step(c, n0, v0, v1, v2, r0, kw1 + digest_swap(hA[2]));
+    v3 = v1; v2 = v0; v1 = n0; v0 = n1;
+    if (first) {
+      v0 = odd ? v0 : i0; v1 = odd ? v1 : i1; v2 = odd ? v2 : i2; v3 = odd ? v3 : i3;
+    } else {
+      v0 += hA[0]; v1 += hA[1]; v2 += hA[2]; v3 += hA[3];
+    }
+    hA[0] = v0 & c.mA; hA[1] = v1 & c.mA; hA[2] = v2 & c.mA; hA[3] = v3 & c.mA;
+  };
+  if (wave == 1) {
+    fetch(0);
+    expand(0);
   }
-  w[14] = (uint32_t)(bits >> 32);
-  w[15] = (uint32_t)bits;
-  smp_sha256_compress(st, w);
+  __syncthreads();
+  for (int64_t ph = 0; ph < nph; ++ph) {
+    if (wave == 1) {
+      if (ph + 1 < nph) expand(ph + 1);
+    } else {
+      for (int h = 0; h < 2; ++h) {
+        const int64_t blk = 2 * ph + h;
+        if (blk >= nblk) break;
+        const uint4* src = &s_kw[ph & 1][h][0][lane];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) out[r * 8 + j] = __builtin_bswap32(st[j]);   // digest bytes in order
+        for (int q = 0; q < 16; ++q) {
+          const uint4 kq = src[q * 64];
+          if (q == 0) {
+            begin(kq.x, kq.y, blk == 0);
+          } else {
+            const uint32_t n0 = digest_step(c, v0, v1, v2, v3, v1, kq.x);
+            const uint32_t n1 = digest_step(c, n0, v0, v1, v2, v0, kq.y);
+            v3 = v1; v2 = v0; v1 = n0; v0 = n1;
+          }
+          const uint32_t n2 = digest_step(c, v0, v1, v2, v3, v1, kq.z);
+          const uint32_t n3 = digest_step(c, n2, v0, v1, v2, v0, kq.w);
+          v3 = v1; v2 = v0; v1 = n2; v0 = n3;
+        }
+      }
+    }
+    __syncthreads();                                   // the next phase is in LDS, this one's buffer is free
+  }
+  if (wave != 0) return;
+  begin(1, 1, false);                                  // the even lanes' last two rounds
+  const int64_t r = row0 + (lane >> 1);
+  if (r >= rows) return;
+#pragma unroll
+  for (int j = 0; j < 4; ++j)                          // digest bytes in order
+    out[r * 8 + (odd ? 4 : 0) + j] = __builtin_bswap32(odd ? hB[j] : hA[j]);
 }
 
 // "trinote-sampler-draw/v1" || seed || position || counter (8 bytes each, big-endian), SHA-256, first 8 bytes
@@ -755,7 +845,7 @@ int imie_logits_digest_dev(const int64_t* logits_dev, int64_t rows, int64_t voca
   if (!logits_dev || !digest_dev || rows <= 0 || vocab <= 0 || ld < vocab || imie_device_ready() != 0)
     return IMIE_EARG;
   if ((reinterpret_cast<uintptr_t>(digest_dev) & 3) != 0) return IMIE_EARG;
-  hipLaunchKernelGGL(smp_digest_kernel, dim3((unsigned)((rows + 63) / 64)), dim3(64), 0,
+  hipLaunchKernelGGL(smp_digest_kernel, dim3((unsigned)((rows + kDigestRows - 1) / kDigestRows)), dim3(128), 0,
                      (hipStream_t)stream, logits_dev, rows, vocab, ld, (uint32_t*)digest_dev);
   IMIE_HIP(hipGetLastError());
   return IMIE_OK;
