@@ -364,21 +364,24 @@ __global__ __launch_bounds__(256) void qk_prep_kernel(const int64_t* __restrict_
       int64_t v[8];
 #pragma unroll
       for (int e = 0; e < 8; ++e) v[e] = X[r * K + c0 + e];
+      // the digits of a value are the bytes of one add and one xor; limbs 0..3 by byte transposes, limb 4 gathered
       uint64_t pk[kQkLimbs];
-#pragma unroll
-      for (int l = 0; l < kQkLimbs; ++l) pk[l] = 0;
+      uint32_t lo[8], hi[8], ta[4], tb[4];
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        const uint64_t a = imie_absu64(v[e]);
+        const uint64_t a = imie_absu64(v[e]), dg = imie_digits64((uint64_t)v[e]);
         mx = a > mx ? a : mx;
-        int64_t x = v[e];
-#pragma unroll
-        for (int l = 0; l < kQkLimbs; ++l) {
-          const int64_t dg = ((x + 128) & 255) - 128;
-          x = (int64_t)((uint64_t)x - (uint64_t)dg) >> 8;
-          pk[l] |= (uint64_t)(uint8_t)dg << (8 * e);
-        }
+        lo[e] = (uint32_t)dg;
+        hi[e] = (uint32_t)(dg >> 32);
       }
+      imie_bytes4x4(lo[0], lo[1], lo[2], lo[3], ta);
+      imie_bytes4x4(lo[4], lo[5], lo[6], lo[7], tb);
+#pragma unroll
+      for (int l = 0; l < 4; ++l) pk[l] = ((uint64_t)tb[l] << 32) | ta[l];
+      imie_bytes4x4(hi[0], hi[1], hi[2], hi[3], ta);
+      imie_bytes4x4(hi[4], hi[5], hi[6], hi[7], tb);
+      pk[4] = ((uint64_t)tb[0] << 32) | ta[0];
+      static_assert(kQkLimbs == 5, "limb 4 is the first of the high halves");
 #pragma unroll
       for (int l = 0; l < kQkLimbs; ++l) *(uint64_t*)&xd[((int64_t)l * rows + r) * K + c0] = pk[l];
     } else {
@@ -721,28 +724,42 @@ __global__ __launch_bounds__(256) void qk_dot4_kernel(const Item* __restrict__ i
 // four balanced base-256 limbs per MFMA (a second MFMA takes limbs 4..7), weight rows in N, one sub-block (Q4_K:
 // 32 positions; Q6_K: 16, the other half of the K groups zeroed in A) per K = 32 step. D lane (t, n) then holds
 // the limb partial sums of token t for weight row n, recombined in place (no cross-lane traffic) into the
-// sub-block dot q.x per limb; S1 = sum_j sc_j q.x_j and S2 = sum_j m_j xsum_j are summed per limb in int32 and
-// recombined once per block into int64 (|x| < 127 (256^5-1)/255: |S1| < 2^57, |S2| < 2^53), and each 256-block
-// adds dq S1 - dmq S2 into a 128-bit (hi, lo) accumulator with one 64 x 64 -> 128 multiply per term. MFMA sums are
-// exact: |D| <= 32 * 128 * 32 < 2^31.
-// gate/up: workgroup = (64 weight rows, item), wave = 16 rows. Up to eight tokens share one walk over the weights:
-// with at most four limbs, two token groups of four are staged (32 digit rows, K in two halves, one barrier each)
-// and every block's decode (scales, mins, nibbles) feeds both groups' MFMAs; otherwise one group of four at a time
-// stages its rows over the whole K (limbs 0..3, then 4..7 in a second pass when there are more than four). The
-// block loop has no barrier; the next block's weights are in flight while a block computes.
-// down (K of a few blocks): workgroup = (64 weight rows, item); the block loop is software-pipelined, the next
-// block's digits going to the other half of an LDS double buffer while a block computes. The buffer's second
-// 16-row group holds tokens 4..7 (up to eight tokens of at most four limbs share each block's unpacked weights)
-// or limbs 4..7 of up to four tokens.
+// sub-block dot q.x per limb. Per block and limb T = sum_j sc_j D_j and M = sum_j m_j xsum_j stay in int32, and the
+// limb's 64-bit sum takes dq T - dmq M by two 32 x 32 + 64 multiply-adds; the four limbs meet in 128 bits once a row.
+// That needs |dq|, |dmq| within a bound that keeps the sums below 2^63 (moe_dq_max: 2^31 - 1 up to 129 blocks of Q4_K,
+// 17 of Q6_K); a block beyond it adds its products to a 128-bit sum instead. MFMA sums are exact: |D| <= 32 * 128 * 128.
+// Up to eight tokens share one walk over the weights: two 16-row groups hold tokens 0..3 and 4..7 (at most four limbs)
+// or limbs 0..3 and 4..7 of four tokens, and every block's decode (scales, mins, quants) feeds both groups' MFMAs. A
+// group's digits are staged in LDS kMoeChunk blocks at a time; the block loop between has
+// no barrier, and the next block's weights are in flight while a block computes.
+// Bound by VALU issue, most of it the block decode: about four tokens meet an expert in a batch of 64.
+// gate/up: workgroup = (64 weight rows, item), wave = 16 rows. down, whose rows are a few blocks long: workgroup =
+// (one or two times 64 weight rows, item), the digits staged once for all of them.
+// The kernels run a few rounds of workgroups, so their code is kept short and in one copy (group count at run time): a
+// cold workgroup waits on instruction fetches (the same walk with a copy per group count and two blocks ahead: 113 us).
+// Measured, 64 tokens, 8 of 128 experts, 2048 -> 768 -> 2048, against 64 x 64 -> 128 products a block, scales decoded
+// one by one and 64 rows a workgroup: gate / up 98 -> 89 us, down 93 -> 83 us (the weights alone: 31 and 23 us).
 // ---------------------------------------------------------------------------------------------------------
 constexpr int kMoeTok = 4;         // tokens per MFMA row group (4 tokens x 4 limbs = 16 rows)
-// LDS row stride of the staged digits: K + 16 bytes (K a multiple of 256). A lane of row r (of the 16 (token, limb)
-// rows) and K group kg reads 8 bytes at r (K + 16) + 8 kg + 32 j, i.e. 8-byte slot 2 r + kg (mod 32): the 32 lanes
-// of a half-wave hit 32 distinct slots (with a K-byte stride all 16 rows of a K group shared one slot: 16-way bank
-// conflicts).
-__host__ __device__ inline int64_t moe_kp(int64_t K) { return K + 16; }
-// gate/up staging: 16 rows x (K + 16) (one token group) or 32 rows x (K / 2 + 16) (two groups, K in halves)
-__host__ __device__ inline size_t moe_lds_bytes(int64_t K) { return (size_t)16 * (size_t)K + 512; }
+constexpr int kMoeChunk = 8;       // blocks staged at a time
+// 16-row tiles of a down wave: two share a workgroup's start and staging where that leaves eight workgroups a CU (64
+// tokens: 92.8 us before, 82.5 with two, 84.9 with four), else one (5 tokens, 36 experts: two cost 3 us a call)
+constexpr int kMoeDownWgs = 2048;
+// LDS row stride of the staged digits: the staged length + 16 bytes (a multiple of 256, + 16). A lane of row r (of the
+// 16 (token, limb) rows) and K group kg reads 8 bytes at r stride + 8 kg + 32 j, i.e. 8-byte slot 2 r + kg (mod 32): the
+// 32 lanes of a half-wave hit 32 distinct slots (without the 16 bytes all 16 rows of a K group shared one slot: 16-way
+// bank conflicts).
+// staging for rows of nb blocks: 32 rows x a chunk, and 256 zero bytes
+__host__ __device__ inline int moe_chunk(int nb) { return nb < kMoeChunk ? nb : kMoeChunk; }
+__host__ __device__ inline size_t moe_lds_bytes(int nb) { return (size_t)32 * (256 * moe_chunk(nb) + 16) + 256; }
+// the largest |dq|, |dmq| for which nb blocks' |dq T| + |dmq M| stay below 2^63 (tmax >= |T| + |M|, resp. |T|) and the
+// factor fits int32
+constexpr int64_t kMoeT4 = (int64_t)8 * 63 * (32 * 128 * 15 + 32 * 128);
+constexpr int64_t kMoeT6 = (int64_t)16 * 128 * (16 * 128 * 128);
+__host__ __device__ inline int64_t moe_dq_max(int64_t nb, int64_t tmax) {
+  const int64_t m = INT64_MAX / (nb * tmax);
+  return m < INT32_MAX ? m : INT32_MAX;
+}
 
 struct MoeItem {
   const uint8_t* wg;        // gate (Q4_K), up (Q4_K), down (Q6_K) of the expert
@@ -783,109 +800,114 @@ __device__ inline int64_t nmc_silu_mul(int64_t x, int64_t u, int fa, int64_t log
   return (int64_t)gu;
 }
 
-// Per-block staging (the down kernel, whose K of a few blocks is walked with the next block's digits fetched while a
-// block computes): up to 8 limbs x kMoeTok tokens x 256 bytes per block, rows of 272 bytes (moe_kp(256)), double
-// buffered.
-constexpr int kMoeLimbs = 8;
-constexpr int kMoeRow = 272;
-constexpr int kMoeBuf = kMoeLimbs * kMoeTok * kMoeRow;
-
-// Staging of one block's digits (L limbs x kMoeTok tokens x 256 bytes) as a register fetch issued before the
-// current block's compute and an LDS store after it. At most 8 x 4 x 16 = 512 uint4: two per thread. The thread's
-// two (source row, LDS slot) pairs are fixed for a token group (MoePlan); a block only adds its offset.
-struct MoePlan {
-  const int8_t* src[2];     // digits of (limb, token) row at 16-byte chunk c, block 0
-  int dst[2];               // LDS byte offset of [l][t][16 c]
-  bool on[2];
+// the rows of one walk: up to eight tokens' activation rows, absent ones repeating the last
+struct MoeRows {
+  int row[2 * kMoeTok];
+  int tn, L;                // tokens taken, limbs of the widest
+  bool two, hi;             // two 16-row groups; the second holds limbs 4..7 (else tokens 4..7)
 };
-__device__ inline MoePlan moe_plan(const int* rowsel, int tn, int L, const int8_t* __restrict__ xd, int64_t rows,
-                                   int64_t K, int tid) {
-  MoePlan p;
-  const int n = L * tn * 16, nt = (int)blockDim.x;    // 256 or 512 threads: two or one chunks each
+// the walk that begins at sel[0] with n pairs left: eight tokens of at most four limbs, or four
+__device__ inline MoeRows moe_rows(const int* __restrict__ sel, const int* __restrict__ Lrow, int n) {
+  MoeRows r;
+  int lr[2 * kMoeTok];
 #pragma unroll
-  for (int k = 0; k < 2; ++k) {
-    const int i = tid + nt * k;
-    p.on[k] = i < n;
-    const int l = p.on[k] ? i / (tn * 16) : 0, rem = i - l * (tn * 16), t = p.on[k] ? rem >> 4 : 0, c = rem & 15;
-    p.src[k] = xd + ((int64_t)l * rows + rowsel[t]) * K + 16 * c;
-    // row 16 gi + 4 (l mod 4) + (t mod 4): the second 16-row group holds limbs 4..7 (tn <= 4) or tokens 4..7 (L <= 4)
-    const int gi = (l >= 4 || t >= kMoeTok) ? 1 : 0;
-    p.dst[k] = (16 * gi + 4 * (l & 3) + (t & 3)) * kMoeRow + 16 * c;
+  for (int i = 0; i < 2 * kMoeTok; ++i) r.row[i] = sel[i < n ? i : n - 1];   // two load rounds, all issued at once
+#pragma unroll
+  for (int i = 0; i < 2 * kMoeTok; ++i) lr[i] = Lrow[r.row[i]];
+  int l4 = 1, l8 = 1;
+#pragma unroll
+  for (int i = 0; i < 2 * kMoeTok; ++i) {
+    l8 = lr[i] > l8 ? lr[i] : l8;
+    if (i < kMoeTok) l4 = l8;
   }
-  return p;
-}
-struct MoeStage {
-  uint4 v[2];
-};
-__device__ inline MoeStage moe_fetch(const MoePlan& p, int64_t b) {
-  MoeStage r;
-#pragma unroll
-  for (int k = 0; k < 2; ++k) r.v[k] = p.on[k] ? *(const uint4*)(p.src[k] + b * 256) : uint4{0, 0, 0, 0};
+  r.tn = min(n, l8 <= 4 ? 2 * kMoeTok : kMoeTok);
+  r.L = r.tn > kMoeTok ? l8 : l4;
+  r.hi = r.L > 4;
+  r.two = r.hi || r.tn > kMoeTok;
   return r;
 }
-__device__ inline void moe_store(const MoeStage& r, const MoePlan& p, int8_t* buf) {
-#pragma unroll
-  for (int k = 0; k < 2; ++k)
-    if (p.on[k]) *(uint4*)(buf + p.dst[k]) = r.v[k];
-}
 
-// both staging buffers to zero (threads tid of nt; the caller synchronizes before and after)
-__device__ inline void moe_clear(int8_t* sx, int tid, int nt) {
-  for (int i = tid; i < 2 * kMoeBuf / 16; i += nt) ((uint4*)sx)[i] = uint4{0, 0, 0, 0};
-}
-
-// Stage limbs 4 p .. 4 p + 3 of up to 8 tokens' activation rows, K positions kbeg .. kbeg + klen, into LDS row
-// r = 16 grp + 4 l + t (token 4 grp + t, limb 4 p + l) at stride kp: 16 ngrp rows x klen / 16 chunks of 16 bytes, the
-// loads of four chunks per thread issued before their stores. Rows of absent tokens (>= tn) or limbs (>= L) are
-// written as zeros, so the MFMA A operands need no selects. The caller synchronizes before (buffer free) and after
-// (rows visible).
-__device__ inline void moe_stage(int8_t* sx, const int (&prow)[2 * kMoeTok], int tn, int L, int p, int ngrp,
-                                 int64_t kbeg, int64_t klen, int64_t kp, const int8_t* __restrict__ xd, int64_t rows,
-                                 int64_t K, int tid, int nt) {
-  const int cpr = (int)(klen >> 4), total = 16 * ngrp * cpr;
-  for (int i0 = tid; i0 < total; i0 += 4 * nt) {
+// Stage the digits of blocks b0 .. b0 + cn into LDS rows at stride kp: row 16 g + 4 l + t holds token 4 g + t, limb l (hi:
+// token t, limb 4 g + l), in chunks of 16 bytes (thread: chunk tid % 16 of a (block, row)), the loads of four per thread
+// issued before their stores. Rows of absent tokens or limbs are written as zeros, so the MFMA A operands need no
+// selects. The caller synchronizes before (buffer free) and after (rows visible).
+__device__ inline void moe_stage(int8_t* sx, const MoeRows& w, int b0, int cn, int kp, const int8_t* __restrict__ xd,
+                                 int64_t rows, int64_t K, int tid, int nt) {
+  const int lgr = w.two ? 5 : 4, total = cn << lgr, c = 16 * (tid & 15);
+  for (int j0 = tid >> 4; j0 < total; j0 += 4 * (nt >> 4)) {
     uint4 v[4];
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const int i = i0 + u * nt;
-      const int r = i / cpr, c = i - r * cpr, l = (r >> 2) & 3, tok = 4 * (r >> 4) + (r & 3);
-      const bool on = i < total && tok < tn && 4 * p + l < L;
-      int pr = prow[0];
+      const int j = j0 + u * (nt >> 4);
+      const int r = j & ((1 << lgr) - 1), b = j >> lgr;
+      const int l = ((r >> 2) & 3) + (w.hi ? 4 * (r >> 4) : 0), tok = (r & 3) + (w.hi ? 0 : 4 * (r >> 4));
+      const bool on = j < total && tok < w.tn && l < w.L;
+      int pr = w.row[0];
 #pragma unroll
-      for (int q = 1; q < 2 * kMoeTok; ++q) pr = tok == q ? prow[q] : pr;
-      v[u] = on ? *(const uint4*)(xd + ((int64_t)(4 * p + l) * rows + pr) * K + kbeg + 16 * c) : uint4{0, 0, 0, 0};
+      for (int q = 1; q < 2 * kMoeTok; ++q) pr = tok == q ? w.row[q] : pr;
+      v[u] = on ? *(const uint4*)(xd + ((int64_t)l * rows + pr) * K + 256 * (int64_t)(b0 + b) + c) : uint4{0, 0, 0, 0};
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
-      const int i = i0 + u * nt;
-      if (i < total) {
-        const int r = i / cpr, c = i - r * cpr;
-        *(uint4*)(sx + r * kp + 16 * c) = v[u];
-      }
+      const int j = j0 + u * (nt >> 4);
+      if (j < total) *(uint4*)(sx + (j & ((1 << lgr) - 1)) * kp + 256 * (j >> lgr) + c) = v[u];
     }
   }
 }
 
-// The lane's A operand source: limb l (of the staged pass) of token t (row m = 4 t + l of the MFMA), K group kg.
-struct MoeA {
-  int off;                  // byte offset of [l][t][8 kg]
+// A (token, row)'s sums: per limb in 64 bits; what blocks beyond moe_dq_max add, in 128 bits in memory (rare, and not
+// touched before the wave meets such a block: a scratch load would wait for the weights in flight)
+struct MoeSum {
+  int64_t v[4];
 };
-__device__ inline MoeA moe_a_lane(int lane, int64_t kp) {
-  const int m = lane & 15, kg = lane >> 4, t = m >> 2, l = m & 3;
-  MoeA r;
-  r.off = (l * kMoeTok + t) * (int)kp + 8 * kg;
-  return r;
+struct MoeFactor {          // a block's dq or dmq: exact where ok, else fp16_fixed_fast has it in 64 bits
+  int f;
+  bool ok;
+};
+// fp16_fixed_fast in 32 bits (m 2^sh with sh <= 20: single precision holds it exactly either way, so one ldexp and rint
+// serve both directions of the shift), without a branch
+__device__ inline MoeFactor moe_factor(uint32_t h, int fw, int64_t dqmax) {
+  const uint32_t e = (h >> 10) & 31, mant = h & 0x3FF;
+  const int sh = (e == 0 ? 1 : (int)e) - 25 + fw;
+  const float m = (float)(e == 0 ? mant : (mant | 0x400));
+  const int r = (int)__builtin_rintf(__builtin_ldexpf(m, sh < 20 ? sh : 20));
+  return {((h >> 15) & 1) ? -r : r, sh <= 20 && r <= (int)dqmax};
 }
-// A operand at K position p0 (buf points at the block's first position)
-__device__ inline int64_t moe_a(const int8_t* buf, const MoeA& a, int p0) {
-  return *(const int64_t*)(buf + a.off + p0);
+__device__ inline int64_t limb_sum(v4i d) {           // sum_r d[r] 256^r
+  return (int64_t)d[0] + ((int64_t)d[1] << 8) + ((int64_t)d[2] << 16) + ((int64_t)d[3] << 24);
+}
+__device__ inline void moe_wide_begin(Acc128 (&w)[2], bool& any) {
+  if (any) return;                                    // wave-uniform
+  w[0] = w[1] = Acc128{0, 0};
+  any = true;
+}
+__device__ __attribute__((noinline)) void moe_wide_add(Acc128* w, uint32_t h, int fw, bool neg, v4i t) {
+  const int64_t f = fp16_fixed_fast(h, fw);
+  acc_madd(*w, neg ? -f : f, limb_sum(t));
+}
+__device__ inline i128 moe_total(const MoeSum& s, const Acc128& w, bool any) {
+  i128 t = 0;
+#pragma unroll
+  for (int l = 3; l >= 0; --l) t = (i128)((unsigned __int128)t << 8) + s.v[l];
+  if (any) t += (i128)(((unsigned __int128)(uint64_t)w.hi << 64) | w.lo);
+  return t;
+}
+__device__ inline int64_t moe_result(i128 t, int fw, bool* fits) {
+  const i128 y = t >> fw;
+  *fits = y <= (i128)INT64_MAX && y >= (i128)INT64_MIN;
+  return (int64_t)y;
 }
 
-// sum_r T[r] << 8 (4 lg + r): a token's value from its per-limb partial sums (int32 per limb)
-__device__ inline int64_t limb_sum(v4i d, int lg) {
-  const int64_t v = (int64_t)d[0] + ((int64_t)d[1] << 8) + ((int64_t)d[2] << 16) + ((int64_t)d[3] << 24);
-  return lg ? (int64_t)((uint64_t)v << 32) : v;
+// No load in flight (after a staging there is none): the compiler's count of them at a block loop's entry is then the
+// loop's own, and its waits for one weight slot leave the other slot's loads in flight.
+__device__ inline void moe_settle() { __builtin_amdgcn_s_waitcnt(0x0F70); }   // vmcnt(0)
+
+// The lane's A operand: limb l of token t (row m = 4 t + l of the MFMA), K group kg: byte offset of [l][t][8 kg].
+__device__ inline int moe_a_lane(int lane, int kp) {
+  const int m = lane & 15, kg = lane >> 4, t = m >> 2, l = m & 3;
+  return (l * kMoeTok + t) * kp + 8 * kg;
 }
+__device__ inline int64_t moe_a(const int8_t* p, int p0) { return *(const int64_t*)(p + p0); }
 
 // Q4_K weights of one block for B lanes (row n, K group kg): the 16-byte header (d, dmin, 12 scale bytes) and the
 // qs bytes 32 g + 8 kg .. + 7 for g = 0..3 (sub-blocks 2 g (low nibbles), 2 g + 1 (high nibbles))
@@ -914,6 +936,10 @@ template <>
 __device__ inline uint8_t gload<uint8_t>(const uint8_t* p) {
   return *(__attribute__((address_space(1))) const uint8_t*)p;
 }
+template <>
+__device__ inline uint16_t gload<uint16_t>(const uint8_t* p) {
+  return *(__attribute__((address_space(1))) const uint16_t*)p;
+}
 __device__ inline Q4Lane q4_lane_load(const uint8_t* blk, int kg) {
   Q4Lane r;
   r.h = gload<uint4>(blk);
@@ -922,22 +948,17 @@ __device__ inline Q4Lane q4_lane_load(const uint8_t* blk, int kg) {
   return r;
 }
 
-// One Q4_K block: acc += dq S1 - dmq S2 for the lane's (token, row). Per limb r, S1's part sum_j sc_j D_j[r] stays
-// in int32 (|D| <= 32 * 128 * 15, 8 sub-blocks x 63: < 2^25) and S2's part sum_j m_j (sum of the sub-block's
-// digits) is an MFMA accumulation with B = m_j in every byte (|.| <= 8 * 63 * 32 * 128 < 2^21).
-template <int NG>
-__device__ inline void q4_block_mfma(const Q4Lane& w, const int8_t* buf, int gstride, const MoeA& a, int lg, int fw,
-                                     Acc128 (&acc)[NG], bool two) {
-  const uint32_t hb = w.h.x;
-  const int64_t dq = fp16_fixed_fast(hb & 0xFFFF, fw), dmq = fp16_fixed_fast(hb >> 16, fw);
-  const uint32_t scw[3] = {w.h.y, w.h.z, w.h.w};
-  auto scb = [&](int i) { return (int)((scw[i >> 2] >> (8 * (i & 3))) & 0xFF); };
-  int sc[8], mn[8];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    if (j < 4) { sc[j] = scb(j) & 63; mn[j] = scb(j + 4) & 63; }
-    else { sc[j] = (scb(j + 4) & 0xF) | ((scb(j - 4) >> 6) << 4); mn[j] = (scb(j + 4) >> 4) | ((scb(j) >> 6) << 4); }
-  }
+// One Q4_K block for the lane's (token, row) of up to two groups (gstride bytes apart in LDS; a: the lane's A pointer at
+// the block). T[r] = sum_j sc_j D_j[r] (|D| <= 32 * 128 * 15, 8 sub-blocks x 63: < 2^25); M = sum_j m_j (sum of the
+// sub-block's digits) is an MFMA accumulation with B = m_j in every byte (|.| <= 8 * 63 * 32 * 128 < 2^21).
+__device__ inline void q4_block_mfma(const Q4Lane& w, const int8_t* a, int gstride, bool two, int fw, int64_t dqmax,
+                                     MoeSum (&acc)[2], Acc128 (&accw)[2], bool& any) {
+  const MoeFactor dq = moe_factor(w.h.x & 0xFFFF, fw, dqmax), dmq = moe_factor(w.h.x >> 16, fw, dqmax);
+  const bool wide = __any(!(dq.ok && dmq.ok));
+  if (wide) moe_wide_begin(accw, any);
+  // the twelve 6-bit scales and mins, four to a dword: bytes j of sc0 / mn0 (sub-blocks 0..3), of sc1 / mn1 (4..7)
+  const uint32_t sc[2] = {w.h.y & 0x3F3F3F3Fu, (w.h.w & 0x0F0F0F0Fu) | ((w.h.y >> 2) & 0x30303030u)};
+  const uint32_t mn[2] = {w.h.z & 0x3F3F3F3Fu, ((w.h.w >> 4) & 0x0F0F0F0Fu) | ((w.h.z >> 2) & 0x30303030u)};
   // sub-block j's weights: the low / high nibbles of q bytes 32 (j / 2) + 8 kg ..; the min term's B operand has
   // m_j in every byte
   auto bq = [&](int j) {
@@ -947,14 +968,13 @@ __device__ inline void q4_block_mfma(const Q4Lane& w, const int8_t* buf, int gst
     return (int64_t)(((uint64_t)b1 << 32) | b0);
   };
   auto bm = [&](int j) {
-    const uint32_t mb = __builtin_amdgcn_perm(0u, (uint32_t)mn[j], 0u);   // byte 0 in all four bytes
+    const uint32_t mb = __builtin_amdgcn_perm(0u, mn[j >> 2], 0x01010101u * (uint32_t)(j & 3));
     return (int64_t)(((uint64_t)mb << 32) | mb);
   };
-  // the weight decode above is shared by the NG token groups (16 MFMA rows each, gstride bytes apart in LDS)
 #pragma unroll
-  for (int gi = 0; gi < NG; ++gi) {
-    if (gi > 0 && !two) break;                        // wave-uniform
-    const int8_t* gb = buf + gi * gstride;
+  for (int gi = 0; gi < 2; ++gi) {
+    if (gi == 1 && !two) break;                       // wave-uniform
+    const int8_t* gb = a + gi * gstride;
     v4i M = {0, 0, 0, 0}, T = {0, 0, 0, 0};
     // two halves of four sub-blocks: four independent MFMAs issued back to back, their results consumed after
 #pragma unroll
@@ -963,122 +983,90 @@ __device__ inline void q4_block_mfma(const Q4Lane& w, const int8_t* buf, int gst
 #pragma unroll
       for (int jj = 0; jj < 4; ++jj) {
         const int j = 4 * hh + jj;
-        const int64_t av = moe_a(gb, a, 32 * j);
+        const int64_t av = moe_a(gb, 32 * j);
         d[jj] = mfma32(av, bq(j), v4i{0, 0, 0, 0});
         M = mfma32(av, bm(j), M);
       }
 #pragma unroll
-      for (int jj = 0; jj < 4; ++jj)
+      for (int jj = 0; jj < 4; ++jj) {
+        const int sj = (int)((sc[hh] >> (8 * jj)) & 0xFF);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) T[r] += __mul24(sc[4 * hh + jj], d[jj][r]);   // 24-bit: |sc| < 2^6, |D| < 2^17
+        for (int r = 0; r < 4; ++r) T[r] += __mul24(sj, d[jj][r]);   // 24-bit: |sc| < 2^6, |D| < 2^17
+      }
     }
-    acc_madd(acc[gi], dq, limb_sum(T, lg));
-    acc_madd(acc[gi], -dmq, limb_sum(M, lg));
+    if (!wide) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        acc[gi].v[r] += (int64_t)dq.f * T[r];
+        acc[gi].v[r] += (int64_t)-dmq.f * M[r];
+      }
+    } else {
+      moe_wide_add(&accw[gi], w.h.x & 0xFFFF, fw, false, T);
+      moe_wide_add(&accw[gi], w.h.x >> 16, fw, true, M);
+    }
   }
 }
 
-// The token groups' activation rows (sel[first + t], absent tokens repeat the last one) and their limb counts
-// (two load rounds, all issued at once); returns the largest
-__device__ inline int moe_group_rows(const int* __restrict__ sel, const int* __restrict__ Lrow, int first, int tn,
-                                     int (&prow)[2 * kMoeTok], int (&lr)[2 * kMoeTok]) {
-#pragma unroll
-  for (int i = 0; i < 2 * kMoeTok; ++i) prow[i] = sel[first + (i < tn ? i : tn - 1)];
-  int L = 1;
-#pragma unroll
-  for (int i = 0; i < 2 * kMoeTok; ++i) { lr[i] = Lrow[prow[i]]; L = lr[i] > L ? lr[i] : L; }
-  return L;
-}
-
-__global__ __launch_bounds__(256, 2) void moe_gateup_kernel(const MoeItem* __restrict__ items, const int* __restrict__ ptok,
+// Waves 0..3 walk the gate rows and 4..7 the up rows of the same 64 rows, two blocks ahead each; their results meet in
+// LDS for the SiLU pass, a thread per (token, row).
+__global__ __launch_bounds__(512, 4) void moe_gateup_kernel(const MoeItem* __restrict__ items, const int* __restrict__ ptok,
                                                          const int* __restrict__ ppair, const int8_t* __restrict__ xd,
                                                          const int* __restrict__ Lrow, int64_t rows, int64_t K,
                                                          int64_t e_ffn, int fw, int fa, int64_t log2e, int64_t dclip,
-                                                         int64_t* __restrict__ gu, int* __restrict__ status,
-                                                         const int* __restrict__ wide) {
-  extern __shared__ __align__(16) int8_t sx[];       // moe_lds_bytes(K)
+                                                         int64_t dqmax, int64_t* __restrict__ gu,
+                                                         int* __restrict__ status, const int* __restrict__ wide) {
+  extern __shared__ __align__(16) int8_t sx[];       // moe_lds_bytes(nb)
+  __shared__ int64_t s_y[2][2 * kMoeTok][64];         // [gate, up][token][row]
   if (*wide) return;                                  // the VALU fallback takes this call
   const MoeItem it = items[blockIdx.y];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  if ((int64_t)blockIdx.x * 64 >= e_ffn) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), proj = wave >> 2;
   const int n = lane & 15, kg = lane >> 4, t = lane >> 4;
   const int nb = (int)(K / 256);
-  const int64_t o = (int64_t)blockIdx.x * 64 + wave * 16 + n;
-  const bool orow = o < e_ffn;
-  const uint8_t* grow = it.wg + (orow ? o : 0) * nb * 144;
-  const uint8_t* urow = it.wu + (orow ? o : 0) * nb * 144;
-  auto emit = [&](const Acc128& ag, const Acc128& au, int tok) {
-    bool f1, f2, f3;
-    const int64_t gy = acc_shift(ag, fw, &f1), uy = acc_shift(au, fw, &f2);
-    const int64_t v = nmc_silu_mul(gy, uy, fa, log2e, dclip, &f3);
-    if (!(f1 && f2 && f3)) atomicOr(status, IMIE_EOVF);
-    gu[(int64_t)ppair[it.first + tok] * e_ffn + o] = v;
-  };
-  for (int t0 = 0; t0 < it.count; t0 += 2 * kMoeTok) {
-    const int tn8 = min(2 * kMoeTok, it.count - t0);
-    int prow[2 * kMoeTok], lr[2 * kMoeTok];
-    const int L8 = moe_group_rows(ptok, Lrow, it.first + t0, tn8, prow, lr);
-    // one weight slot per projection, the first requested before the staging: block b + 1 is requested as soon as
-    // block b has consumed the slot (the other waves of the SIMD cover the latency)
-    Q4Lane gw = q4_lane_load(grow, kg), uw = q4_lane_load(urow, kg);
-    if (tn8 > kMoeTok && L8 <= 4 && (nb & 1) == 0) {
-      // two token groups of four in one walk over the weights (the block decode shared): K staged in halves of
-      // 32 rows x (K / 2 + 16)
-      const int64_t kp = K / 2 + 16;
-      const MoeA al = moe_a_lane(lane, kp);
-      Acc128 ag[2] = {{0, 0}, {0, 0}}, au[2] = {{0, 0}, {0, 0}};
-      for (int h = 0; h < 2; ++h) {
-        __syncthreads();                              // the buffer is free
-        moe_stage(sx, prow, tn8, L8, 0, 2, h * (K / 2), K / 2, kp, xd, rows, K, tid, blockDim.x);
-        __syncthreads();
-        for (int bb = 0; bb < nb / 2; ++bb) {
-          const int b = h * (nb / 2) + bb, bn = b + 1 < nb ? b + 1 : b;
-          const int8_t* buf = sx + 256 * bb;
-          q4_block_mfma<2>(gw, buf, (int)(16 * kp), al, 0, fw, ag, true);
-          gw = q4_lane_load(grow + bn * 144, kg);
-          q4_block_mfma<2>(uw, buf, (int)(16 * kp), al, 0, fw, au, true);
-          uw = q4_lane_load(urow + bn * 144, kg);
-        }
+  const int row = 16 * (wave & 3) + n;
+  const int64_t ob = (int64_t)blockIdx.x * 64;
+  const bool orow = ob + row < e_ffn;
+  const uint8_t* wrow = (proj ? it.wu : it.wg) + (orow ? ob + row : 0) * nb * 144;
+  for (int t0 = 0; t0 < it.count;) {
+    Q4Lane wq = q4_lane_load(wrow, kg);
+    const MoeRows w = moe_rows(ptok + it.first + t0, Lrow, it.count - t0);
+    const int64_t pair = ppair[it.first + min(t0 + wave, it.count - 1)];   // the SiLU pass's token is the wave
+    const int ch = moe_chunk(nb), kp = 256 * ch + 16;
+    const int8_t* a0 = sx + moe_a_lane(lane, kp);
+    MoeSum acc[2] = {};
+    Acc128 accw[2];
+    bool any = false;
+    for (int c0 = 0; c0 < nb; c0 += ch) {
+      const int cn = min(ch, nb - c0);
+      __syncthreads();                                // the buffer is free
+      moe_stage(sx, w, c0, cn, kp, xd, rows, K, tid, 512);
+      __syncthreads();
+      moe_settle();
+      for (int bb = 0; bb < cn; ++bb) {               // the next block is requested as soon as this one is decoded
+        const Q4Lane cur = wq;
+        wq = q4_lane_load(wrow + (int64_t)min(c0 + bb + 1, nb - 1) * 144, kg);
+        q4_block_mfma(cur, a0 + 256 * bb, 16 * kp, w.two, fw, dqmax, acc, accw, any);
       }
-      if (orow) {
-        emit(ag[0], au[0], t0 + t);
-        if (kMoeTok + t < tn8) emit(ag[1], au[1], t0 + kMoeTok + t);
-      }
-      continue;
     }
-    // one token group of four at a time; more than four limbs take two passes per group (limbs 0..3, 4..7)
-    const int64_t kp = K + 16;
-    const MoeA al = moe_a_lane(lane, kp);
-    for (int s0 = 0; s0 < tn8; s0 += kMoeTok) {
-      const int tn = min(kMoeTok, tn8 - s0);
-      int pr4[2 * kMoeTok];
-      int L = 1;
-#pragma unroll
-      for (int i = 0; i < 2 * kMoeTok; ++i) {
-        const int q = s0 + (i < tn ? i : tn - 1);
-        int v = prow[0], lv = lr[0];
-#pragma unroll
-        for (int z = 1; z < 2 * kMoeTok; ++z) { v = q == z ? prow[z] : v; lv = q == z ? lr[z] : lv; }
-        pr4[i] = v;
-        L = i < tn && lv > L ? lv : L;
-      }
-      const int np = L > 4 ? 2 : 1;
-      Acc128 ag[1] = {{0, 0}}, au[1] = {{0, 0}};
-      for (int p = 0; p < np; ++p) {
-        __syncthreads();                              // the buffer is free
-        moe_stage(sx, pr4, tn, L, p, 1, 0, K, kp, xd, rows, K, tid, blockDim.x);
-        __syncthreads();
-        for (int b = 0; b < nb; ++b) {
-          // the next block of this walk: this group's next pass or the following group start again at block 0
-          const int bn = b + 1 < nb ? b + 1 : 0;
-          const int8_t* buf = sx + 256 * b;
-          q4_block_mfma<1>(gw, buf, 0, al, p, fw, ag, false);
-          gw = q4_lane_load(grow + bn * 144, kg);
-          q4_block_mfma<1>(uw, buf, 0, al, p, fw, au, false);
-          uw = q4_lane_load(urow + bn * 144, kg);
-        }
-      }
-      if (orow && t < tn) emit(ag[0], au[0], t0 + s0 + t);
+    auto put = [&](i128 v, int tok) {
+      bool f;
+      s_y[proj][tok][row] = moe_result(v, fw, &f);
+      if (!f && orow && tok < w.tn) atomicOr(status, IMIE_EOVF);
+    };
+    i128 y = moe_total(acc[0], accw[0], any);
+    if (w.two) {
+      const i128 y1 = moe_total(acc[1], accw[1], any);
+      if (w.hi) y += (i128)((unsigned __int128)y1 << 32);
+      else put(y1, kMoeTok + t);
     }
+    put(y, t);
+    __syncthreads();
+    if (wave < w.tn && ob + lane < e_ffn) {
+      bool f;
+      const int64_t v = nmc_silu_mul(s_y[0][wave][lane], s_y[1][wave][lane], fa, log2e, dclip, &f);
+      if (!f) atomicOr(status, IMIE_EOVF);
+      gu[pair * e_ffn + ob + lane] = v;
+    }
+    t0 += w.tn;
   }
 }
 
@@ -1100,37 +1088,37 @@ __device__ inline Q6Lane q6_lane_load(const uint8_t* blk, int kg) {
     r.h[half] = gload<uint2>(blk + 128 + 32 * half + 8 * kg);
   }
   r.sc = gload<uint4>(blk + 192);
-  r.d = (uint32_t)gload<uint8_t>(blk + 208) | ((uint32_t)gload<uint8_t>(blk + 209) << 8);
+  r.d = gload<uint16_t>(blk + 208);                   // blocks are 210 bytes apart: 2-byte aligned
   return r;
 }
 
-// One Q6_K block: acc += dq S1; per limb r, sum_j sc_j D_j[r] in int32 (|D| <= 32 * 128 * 32 = 2^17, 16
-// sub-blocks x 128: < 2^28)
-// The second group (gstride bytes further in LDS) is either limbs 4..7 of the same tokens (added into acc0 with
-// lg1 = 1) or limbs 0..3 of four more tokens (acc1, lg1 = 0); the block's unpacked weights and scales serve both.
-__device__ inline void q6_block_mfma(const Q6Lane& w, const int8_t* buf, int gstride, const MoeA& a, int kg, int fw,
-                                     Acc128& acc0, Acc128& acc1, int lg1, bool two) {
-  const int64_t dq = fp16_fixed_fast(w.d, fw);
+// One Q6_K block: T[r] = sum_j sc_j D_j[r] with the weights as bytewise 4 (q6 - 32) (the six bits at the top of the byte,
+// sign bit flipped: five instructions a dword), so the row's total is a multiple of 4 and shifted back once (|D| <= 16 *
+// 128 * 128 = 2^18, 16 sub-blocks x 128: 2^29). A 32-position K step spans two sub-blocks (K groups 0, 1 and 2, 3): two
+// MFMAs, whose A pointers (a0, a1; s0, s1: bytes between the groups) lead the other one's lanes to zeros in LDS.
+__device__ inline void q6_block_mfma(const Q6Lane& w, const int8_t* a0, const int8_t* a1, int s0, int s1, bool two,
+                                     int fw, int64_t dqmax, MoeSum (&acc)[2], Acc128 (&accw)[2], bool& any) {
+  const MoeFactor dq = moe_factor(w.d, fw, dqmax);
+  const bool wide = __any(!dq.ok);
+  if (wide) moe_wide_begin(accw, any);
   const uint32_t scw[4] = {w.sc.x, w.sc.y, w.sc.z, w.sc.w};
-  auto scs = [&](int i) { return (int)(int8_t)((scw[i >> 2] >> (8 * (i & 3))) & 0xFF); };
-  const bool klo = kg < 2;
+  auto scs = [&](int i) { return (int)(int8_t)(uint8_t)(scw[i >> 2] >> (8 * (i & 3))); };
+  auto wq = [](uint32_t lv, uint32_t hv, int qq) {
+    const uint32_t lo = qq >= 2 ? lv >> 2 : lv << 2, hi = hv << (6 - 2 * qq);
+    return (((lo & 0x3C3C3C3Cu) | (hi & ~0x3C3C3C3Cu)) & 0xFCFCFCFCu) ^ 0x80808080u;
+  };
   int64_t bq[2][4];
 #pragma unroll
   for (int half = 0; half < 2; ++half)
 #pragma unroll
     for (int qq = 0; qq < 4; ++qq) {
       const uint2 lv = w.l[half][qq & 1], hv = w.h[half];
-      const int sl = qq >= 2 ? 4 : 0, sh = 2 * qq;
-      uint32_t v0 = ((lv.x >> sl) & 0x0F0F0F0Fu) | (((hv.x >> sh) & 0x03030303u) << 4);
-      uint32_t v1 = ((lv.y >> sl) & 0x0F0F0F0Fu) | (((hv.y >> sh) & 0x03030303u) << 4);
-      v0 = ((v0 | 0x80808080u) - 0x20202020u) ^ 0x80808080u;   // bytewise q6 - 32 as int8
-      v1 = ((v1 | 0x80808080u) - 0x20202020u) ^ 0x80808080u;
-      bq[half][qq] = (int64_t)(((uint64_t)v1 << 32) | v0);
+      bq[half][qq] = (int64_t)(((uint64_t)wq(lv.y, hv.y, qq) << 32) | wq(lv.x, hv.x, qq));
     }
 #pragma unroll
   for (int gi = 0; gi < 2; ++gi) {
     if (gi == 1 && !two) break;                       // wave-uniform
-    const int8_t* gb = buf + gi * gstride;
+    const int8_t *g0 = a0 + gi * s0, *g1 = a1 + gi * s1;
     v4i T = {0, 0, 0, 0};
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
@@ -1138,94 +1126,87 @@ __device__ inline void q6_block_mfma(const Q6Lane& w, const int8_t* buf, int gst
       v4i d[4][2];
 #pragma unroll
       for (int qq = 0; qq < 4; ++qq) {
-        // the K step spans sub-blocks 8 half + 2 qq (K groups 0, 1) and + 1 (K groups 2, 3)
-        const int64_t av = moe_a(gb, a, 128 * half + 32 * qq);
-        d[qq][0] = mfma32(klo ? av : 0, bq[half][qq], v4i{0, 0, 0, 0});
-        d[qq][1] = mfma32(klo ? 0 : av, bq[half][qq], v4i{0, 0, 0, 0});
+        d[qq][0] = mfma32(moe_a(g0, 128 * half + 32 * qq), bq[half][qq], v4i{0, 0, 0, 0});
+        d[qq][1] = mfma32(moe_a(g1, 128 * half + 32 * qq), bq[half][qq], v4i{0, 0, 0, 0});
       }
 #pragma unroll
       for (int qq = 0; qq < 4; ++qq) {
-        const int s0 = scs(8 * half + 2 * qq), s1 = scs(8 * half + 2 * qq + 1);
+        const int c0 = scs(8 * half + 2 * qq), c1 = scs(8 * half + 2 * qq + 1);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) T[r] += __mul24(s0, d[qq][0][r]) + __mul24(s1, d[qq][1][r]);   // |s| < 2^8, |D| < 2^18
+        for (int r = 0; r < 4; ++r) T[r] += __mul24(c0, d[qq][0][r]) + __mul24(c1, d[qq][1][r]);   // |s| < 2^8, |D| <= 2^18
       }
     }
-    if (gi == 0) acc_madd(acc0, dq, limb_sum(T, 0));
-    else acc_madd(acc1, dq, limb_sum(T, lg1));
+    if (!wide) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) acc[gi].v[r] += (int64_t)dq.f * T[r];
+    } else {
+      moe_wide_add(&accw[gi], w.d, fw, false, T);
+    }
   }
 }
 
-__global__ __launch_bounds__(256) void moe_down_kernel(const MoeItem* __restrict__ items, const int* __restrict__ ppair,
-                                                       const int8_t* __restrict__ xd, const int64_t* __restrict__ xs16,
-                                                       const int* __restrict__ Lrow, int64_t rows, int64_t K,
-                                                       int64_t d_model, int fw, int64_t* __restrict__ dout,
-                                                       int* __restrict__ status, const int* __restrict__ wide) {
-  __shared__ __align__(16) int8_t sx[2][kMoeBuf];
-  __shared__ int s_rows[2 * kMoeTok];
+__global__ __launch_bounds__(256, 4) void moe_down_kernel(const MoeItem* __restrict__ items, const int* __restrict__ ppair,
+                                                       const int8_t* __restrict__ xd, const int* __restrict__ Lrow,
+                                                       int64_t rows, int64_t K, int64_t d_model, int wtiles, int fw, int64_t dqmax,
+                                                       int64_t* __restrict__ dout, int* __restrict__ status,
+                                                       const int* __restrict__ wide) {
+  extern __shared__ __align__(16) int8_t sx[];       // moe_lds_bytes(nb): 256 zero bytes, the staged digits
   if (*wide) return;
   const MoeItem it = items[blockIdx.y];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  if ((int64_t)blockIdx.x * 64 >= d_model) return;
   const int n = lane & 15, kg = lane >> 4, t = lane >> 4;
-  const int64_t o = (int64_t)blockIdx.x * 64 + wave * 16 + n;
-  const bool orow = o < d_model;
-  const int64_t nb = K / 256;
-  const uint8_t* drow = it.wd + (orow ? o : 0) * nb * 210;
+  const int nb = (int)(K / 256);
+  // the wave's tiles: rows o0 + 64 rt
+  const int64_t o0 = (int64_t)blockIdx.x * (64 * wtiles) + wave * 16 + n;
+  const int tiles = (int)min((int64_t)wtiles, (d_model - (int64_t)blockIdx.x * (64 * wtiles) + 63) / 64);
+  auto wrow = [&](int rt) {
+    const int64_t o = o0 + 64 * rt;
+    return it.wd + (o < d_model ? o : 0) * nb * 210;
+  };
+  if (tid < 16) ((uint4*)sx)[tid] = uint4{0, 0, 0, 0};   // visible with the first staging
   for (int t0 = 0; t0 < it.count;) {
-    // up to eight tokens with at most four limbs (the second 16-row group holds tokens 4..7), else up to four
-    // tokens (the second group holds limbs 4..7 when there are more than four)
-    const int tn8 = min(2 * kMoeTok, it.count - t0);
-    int L4 = 1, L8 = 1;
-    for (int i = 0; i < tn8; ++i) {
-      const int lr = Lrow[ppair[it.first + t0 + i]];
-      L8 = lr > L8 ? lr : L8;
-      if (i < kMoeTok) L4 = L8;
+    Q6Lane wq = q6_lane_load(wrow(0), kg);
+    const MoeRows w = moe_rows(ppair + it.first + t0, Lrow, it.count - t0);
+    const int ch = moe_chunk(nb), kp = 256 * ch + 16;
+    const int al = 256 + moe_a_lane(lane, kp), z = 8 * kg;
+    for (int rt = 0; rt < tiles; ++rt) {
+      const uint8_t *row = wrow(rt), *next = wrow(min(rt + 1, tiles - 1));
+      MoeSum ad[2] = {};
+      Acc128 adw[2];
+      bool any = false;
+      for (int c0 = 0; c0 < nb; c0 += ch) {
+        const int cn = min(ch, nb - c0);
+        if (rt == 0 || ch < nb) {                     // whole rows that fit are staged once for all tiles
+          __syncthreads();                            // the buffer is free
+          moe_stage(sx + 256, w, c0, cn, kp, xd, rows, K, tid, 256);
+          __syncthreads();
+          moe_settle();
+        }
+        for (int bb = 0; bb < cn; ++bb) {
+          const int b = c0 + bb + 1, a = al + 256 * bb;
+          const Q6Lane cur = wq;
+          wq = q6_lane_load(b < nb ? row + (int64_t)b * 210 : next, kg);
+          q6_block_mfma(cur, sx + (kg < 2 ? a : z), sx + (kg < 2 ? z : a), kg < 2 ? 16 * kp : 0, kg < 2 ? 0 : 16 * kp,
+                        w.two, fw, dqmax, ad, adw, any);
+        }
+      }
+      const int64_t o = o0 + 64 * rt;
+      auto emit = [&](i128 y, int tok) {
+        if (o >= d_model || tok >= w.tn) return;
+        bool f;
+        const int64_t v = moe_result(y >> 2, fw, &f);
+        if (!f) atomicOr(status, IMIE_EOVF);
+        dout[(int64_t)ppair[it.first + t0 + tok] * d_model + o] = v;
+      };
+      i128 y = moe_total(ad[0], adw[0], any);
+      if (w.two) {
+        const i128 y1 = moe_total(ad[1], adw[1], any);
+        if (w.hi) y += (i128)((unsigned __int128)y1 << 32);
+        else emit(y1, kMoeTok + t);
+      }
+      emit(y, t);
     }
-    const bool tok2 = tn8 > kMoeTok && L8 <= 4;
-    const int tn = tok2 ? tn8 : min(kMoeTok, tn8), L = tok2 ? L8 : L4;
-    __syncthreads();                                  // the previous token group is done with the buffers
-    moe_clear(&sx[0][0], tid, blockDim.x);
-    if (tid < tn) s_rows[tid] = ppair[it.first + t0 + tid];
-    __syncthreads();
-    const MoeA al = moe_a_lane(lane, kMoeRow);
-    Q6Lane w0 = q6_lane_load(drow, kg), w1 = w0;
-    if (nb > 1) w1 = q6_lane_load(drow + 210, kg);
-    const MoePlan pl = moe_plan(s_rows, tn, L, xd, rows, K, tid);
-    moe_store(moe_fetch(pl, 0), pl, &sx[0][0]);
-    __syncthreads();
-    Acc128 ad{0, 0}, ad1{0, 0};
-    Acc128& a2 = tok2 ? ad1 : ad;
-    const int lg1 = tok2 ? 0 : 1;
-    const bool two = tok2 || L > 4;
-    constexpr int gstride = 4 * kMoeTok * kMoeRow;
-    for (int64_t b = 0; b < nb; b += 2) {
-      MoeStage nx{};
-      if (b + 1 < nb) nx = moe_fetch(pl, b + 1);
-      q6_block_mfma(w0, &sx[0][0], gstride, al, kg, fw, ad, a2, lg1, two);
-      if (b + 2 < nb) w0 = q6_lane_load(drow + (b + 2) * 210, kg);
-      if (b + 1 >= nb) break;
-      moe_store(nx, pl, &sx[1][0]);
-      __syncthreads();
-      if (b + 2 < nb) nx = moe_fetch(pl, b + 2);
-      q6_block_mfma(w1, &sx[1][0], gstride, al, kg, fw, ad, a2, lg1, two);
-      if (b + 3 < nb) w1 = q6_lane_load(drow + (b + 3) * 210, kg);
-      if (b + 2 >= nb) break;
-      moe_store(nx, pl, &sx[0][0]);
-      __syncthreads();
-    }
-    if (orow && t < tn) {
-      bool f;
-      const int64_t y = acc_shift(ad, fw, &f);
-      if (!f) atomicOr(status, IMIE_EOVF);
-      dout[(int64_t)ppair[it.first + t0 + t] * d_model + o] = y;
-    }
-    if (orow && tok2 && kMoeTok + t < tn) {
-      bool f;
-      const int64_t y = acc_shift(ad1, fw, &f);
-      if (!f) atomicOr(status, IMIE_EOVF);
-      dout[(int64_t)ppair[it.first + t0 + kMoeTok + t] * d_model + o] = y;
-    }
-    t0 += tn;
+    t0 += w.tn;
   }
 }
 
@@ -1954,13 +1935,12 @@ int moe_batched(const long long* gate_h, const long long* up_h, const long long*
   const Item *d_ig = (const Item*)(mb + o_ig), *d_iu = (const Item*)(mb + o_iu), *d_id = (const Item*)(mb + o_id);
   const int *d_pt = (const int*)(mb + o_pt), *d_pp = (const int*)(mb + o_pp);
   const int64_t prow = P > m ? P : m, pk = d_model > e_ffn ? d_model : e_ffn;
-  if (g_qprep.xd.ensure((size_t)(kQkLimbs * prow * pk)) || g_qprep.xs.ensure((size_t)(prow * (pk / 16)) * 8) ||
-      g_qprep.lr.ensure((size_t)prow * 4) || g_qprep.flag.ensure(64))
+  if (g_qprep.xd.ensure((size_t)(kQkLimbs * prow * pk)) || g_qprep.lr.ensure((size_t)prow * 4) ||
+      g_qprep.flag.ensure(64))
     return IMIE_EARG;
   int* flagA = (int*)g_qprep.flag.p;
   int* flagB = flagA + 1;
   int8_t* xdp = (int8_t*)g_qprep.xd.p;
-  int64_t* xsp = (int64_t*)g_qprep.xs.p;
   int* lrp = (int*)g_qprep.lr.p;
   int64_t log2e, dclip;
   silu_consts_nmc(fa, &log2e, &dclip);
@@ -1971,16 +1951,19 @@ int moe_batched(const long long* gate_h, const long long* up_h, const long long*
   hipLaunchKernelGGL(qk_prep_kernel, dim3((unsigned)m), dim3(256), 0, st, h_dev, (int64_t)m, d_model, xdp, nullptr, lrp,
                      flagA);
   hipLaunchKernelGGL(moe_gateup_kernel, dim3((unsigned)((e_ffn + 63) / 64),
-                     (unsigned)ne), dim3(256), moe_lds_bytes(d_model), st, d_items,
-                     d_pt, d_pp, xdp, lrp, (int64_t)m, d_model, e_ffn, fw, fa, log2e, dclip, gb, status, flagA);
+                     (unsigned)ne), dim3(512), moe_lds_bytes((int)(d_model / 256)), st, d_items,
+                     d_pt, d_pp, xdp, lrp, (int64_t)m, d_model, e_ffn, fw, fa, log2e, dclip,
+                     moe_dq_max(d_model / 256, kMoeT4), gb, status, flagA);
   // exact VALU fallback of the gate/up stage (runs only when the prep flagged a wide activation row)
   const int64_t ntg = (e_ffn + kRows - 1) / kRows;
   hipLaunchKernelGGL(qk_gateup_gated_kernel, dim3(kGatedWgs2), dim3(256), 0, st, d_ig, d_iu, d_pt, d_pp, h_dev,
                      d_model, gb, ub, e_ffn, fw, fa, log2e, dclip, status, flagA, ntg, (int64_t)ne);
   // down over the P rows of gu
   hipLaunchKernelGGL(qk_prep_kernel, dim3((unsigned)P), dim3(256), 0, st, gb, P, e_ffn, xdp, nullptr, lrp, flagB);
-  hipLaunchKernelGGL(moe_down_kernel, dim3((unsigned)((d_model + 63) / 64), (unsigned)ne), dim3(256), 0, st, d_items,
-                     d_pp, xdp, xsp, lrp, P, e_ffn, d_model, fw, db, status, flagB);
+  const int wtiles = (int64_t)ne * ((d_model + 63) / 64) >= kMoeDownWgs ? 2 : 1;
+  hipLaunchKernelGGL(moe_down_kernel, dim3((unsigned)((d_model + 64 * wtiles - 1) / (64 * wtiles)), (unsigned)ne),
+                     dim3(256), moe_lds_bytes((int)(e_ffn / 256)), st, d_items, d_pp, xdp, lrp, P, e_ffn, d_model,
+                     wtiles, fw, moe_dq_max(e_ffn / 256, kMoeT6), db, status, flagB);
   hipLaunchKernelGGL(qk_group_gated_kernel, dim3(kGatedWgs), dim3(256), 0, st, d_id, d_pp, d_pp, gb, e_ffn, db,
                      d_model, fw, status, flagB, (int64_t)((d_model + kRows - 1) / kRows), (int64_t)ne);
   hipLaunchKernelGGL(qk_combine_kernel, dim3((unsigned)(((int64_t)m * d_model + 255) / 256)), dim3(256), 0, st, db,

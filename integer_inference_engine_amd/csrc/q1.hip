@@ -6,7 +6,7 @@
 // Reference semantics: bonsai/src/trinote/infer_int/reference_bonsai.py:149-219 (q1_linear_ref) and the C
 // producer bonsai/tools/bonsai_q1_kernel.c:85-106. Bit i of byte j of a block is weight 8j+i.
 //
-// Matvec design (T < 8): int8 MFMA v_mfma_i32_16x16x64_i8 over 16-row tiles and 512-column slabs:
+// Matvec design (T <= 8): int8 MFMA v_mfma_i32_16x16x64_i8 over 16-row tiles and 512-column slabs:
 //   * B operand = one bit position s of the weight bytes of 16 output rows as 0/1 bytes
 //       B_s dword = (word >> s) & 0x01010101                            (2 VALU per 4 dwords of weights)
 //   * A operand = balanced base-256 digits ("limbs") of x from the prepared digit table, rows = (block g of the
@@ -17,7 +17,7 @@
 //   * Epilogue per (row, block): pos = sum_r D[r] << 8r, 2*pos - total, * scale, floor shift, add (wrapping
 //     int64, as the reference's C producer).
 // MFMA int32 accumulation is exact: each D entry is at most 8 * 16 * 128 = 2^14 in magnitude.
-// Prefill (T >= 8) uses the tiled GEMM further down.
+// Prefill (T >= 9) uses the tiled GEMM further down.
 #include "imie_common.h"
 #include <vector>
 #include "imie_kernels.h"
