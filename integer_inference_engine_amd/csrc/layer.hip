@@ -17,6 +17,7 @@
 #include "imie_kvfmt.h"
 #include <string.h>
 #include <algorithm>
+#include <thread>
 
 namespace {
 
@@ -152,6 +153,7 @@ struct Net {
   std::vector<int64_t> pg0, npg;      // per sequence: first pool page and page count (its pages are contiguous)
   std::vector<void*> kpool, vpool;    // per layer
   int64_t* pt = nullptr;              // device [B][mp]
+  DevBuf* arena = nullptr;            // set: the pools and pt lie in this buffer, which outlives the net
   std::vector<int64_t> len;           // host lengths per sequence
   // workspace
   DevBuf n, q, k, v, qn, kn, att, gate, up, h, pos, starts, attn, guard, status, x, logits, ids, lastx, amx, stepc;
@@ -180,12 +182,59 @@ Net* net_get(int64_t h) {
 }
 
 void net_free_kv(Net& n) {
-  for (auto p : n.kpool) if (p) imie_free(p);
-  for (auto p : n.vpool) if (p) imie_free(p);
+  if (!n.arena) {
+    for (auto p : n.kpool) if (p) imie_free(p);
+    for (auto p : n.vpool) if (p) imie_free(p);
+    if (n.pt) imie_free(n.pt);
+  }
   n.kpool.clear();
   n.vpool.clear();
-  if (n.pt) imie_free(n.pt);
   n.pt = nullptr;
+}
+
+// a net's workspaces
+constexpr int kNetBufs = 30;
+struct NetBufs { DevBuf* b[kNetBufs]; };
+NetBufs net_bufs(Net& n) {
+  return {{&n.n, &n.q, &n.k, &n.v, &n.qn, &n.kn, &n.att, &n.gate, &n.up, &n.h, &n.pos, &n.starts, &n.attn, &n.guard,
+           &n.status, &n.x, &n.logits, &n.ids, &n.lastx, &n.amx, &n.stepc, &n.q1w.xq, &n.q1w.totals, &n.q1w.lslab,
+           &n.q1w.wide, &n.kvrun, &n.kvrow, &n.gpart, &n.gtab, &n.gmax}};
+}
+
+// What whole prefills (bonsai_prefill_forward_gpu) keep between calls: the workspaces, the cache's memory and a pinned
+// buffer for its export, handed to one call at a time under the library lock and idle when it returns (the call
+// synchronizes). Allocating and freeing some fifty buffers a call and exporting through pageable memory was half of a
+// 256-row, 12-layer call. Only sizes within the bounds stay; imie_buf_free_all gives them back.
+constexpr size_t kKeepDevice = (size_t)2 << 30, kKeepPinned = (size_t)256 << 20;
+struct Kept {
+  DevBuf ws[kNetBufs], arena;
+  char* pin = nullptr;
+  size_t pin_cap = 0;
+  void give_back() {
+    for (auto& b : ws) b.release();
+    arena.release();
+    if (pin) (void)hipHostFree(pin);
+    pin = nullptr;
+    pin_cap = 0;
+  }
+};
+Kept& kept() {
+  static Kept k;
+  return k;
+}
+void kept_take(Net& n) {
+  const NetBufs nb = net_bufs(n);
+  for (int i = 0; i < kNetBufs; ++i) std::swap(*nb.b[i], kept().ws[i]);
+}
+void kept_return(Net& n) {
+  const NetBufs nb = net_bufs(n);
+  size_t total = kept().arena.cap;
+  for (auto b : nb.b) total += b->cap;
+  if (total > kKeepDevice) {                           // too large to hold on to
+    kept().arena.release();
+    return;                                            // net_free releases the workspaces
+  }
+  for (int i = 0; i < kNetBufs; ++i) std::swap(*nb.b[i], kept().ws[i]);
 }
 
 void net_free(Net* n) {
@@ -193,11 +242,7 @@ void net_free(Net* n) {
   (void)hipStreamSynchronize(imie_stream());
   net_free_kv(*n);
   if (n->gexec) { (void)hipGraphExecDestroy(n->gexec); n->gexec = nullptr; }
-  DevBuf* bs[] = {&n->n, &n->q, &n->k, &n->v, &n->qn, &n->kn, &n->att, &n->gate, &n->up, &n->h, &n->pos,
-                  &n->starts, &n->attn, &n->guard, &n->status, &n->x, &n->logits, &n->ids, &n->lastx, &n->amx,
-                  &n->stepc, &n->q1w.xq, &n->q1w.totals, &n->q1w.lslab, &n->q1w.wide, &n->kvrun, &n->kvrow, &n->gpart,
-                  &n->gtab, &n->gmax};
-  for (auto b : bs) b->release();
+  for (auto b : net_bufs(*n).b) b->release();
   n->live = false;
 }
 
@@ -225,7 +270,16 @@ int net_alloc_kv(Net& n, const std::vector<int64_t>& caps, int64_t P, int kv32) 
   const size_t bytes = (size_t)(n.npages * n.Hkv * P * n.hd) * esz;
   n.kpool.assign((size_t)n.nl, nullptr);
   n.vpool.assign((size_t)n.nl, nullptr);
-  for (int64_t l = 0; l < n.nl; ++l) {
+  const size_t ptb = ((size_t)(n.B * mp) * 8 + 255) & ~(size_t)255;
+  if (n.arena) {                                       // [page table][K of every layer][V of every layer]
+    if (n.arena->ensure(ptb + 2 * (size_t)n.nl * bytes)) return IMIE_EARG;
+    n.pt = (int64_t*)n.arena->p;
+    for (int64_t l = 0; l < n.nl; ++l) {
+      n.kpool[(size_t)l] = (char*)n.arena->p + ptb + (size_t)l * bytes;
+      n.vpool[(size_t)l] = (char*)n.arena->p + ptb + (size_t)(n.nl + l) * bytes;
+    }
+  }
+  for (int64_t l = 0; l < n.nl && !n.arena; ++l) {
     if (hipMalloc(&n.kpool[(size_t)l], bytes) != hipSuccess) return IMIE_EARG;
     if (hipMalloc(&n.vpool[(size_t)l], bytes) != hipSuccess) return IMIE_EARG;
   }
@@ -233,7 +287,7 @@ int net_alloc_kv(Net& n, const std::vector<int64_t>& caps, int64_t P, int kv32) 
   for (int64_t b = 0; b < n.B; ++b)
     for (int64_t i = 0; i < mp; ++i)
       pt[(size_t)(b * mp + i)] = n.pg0[(size_t)b] + (i < n.npg[(size_t)b] ? i : 0);
-  IMIE_HIP(hipMalloc((void**)&n.pt, pt.size() * 8));
+  if (!n.arena) IMIE_HIP(hipMalloc((void**)&n.pt, pt.size() * 8));
   IMIE_HIP(hipMemcpy(n.pt, pt.data(), pt.size() * 8, hipMemcpyHostToDevice));
   n.len.assign((size_t)n.B, 0);
   if (kv32) {
@@ -527,7 +581,8 @@ int64_t net_create(int64_t B, int64_t n_layers, int64_t H, int64_t Hkv, int64_t 
                    int64_t cap, int64_t vocab, int64_t frac, int64_t eps, int64_t inv_sqrt, const int64_t* wq,
                    const int64_t* wk, const int64_t* wv, const int64_t* wo, const int64_t* w1, const int64_t* wu,
                    const int64_t* w2, const int64_t* n1g, const int64_t* n2g, const int64_t* qng, const int64_t* kng,
-                   int64_t finalg, int64_t out_head, int64_t cos_h, int64_t sin_h, int64_t page, int kv32) {
+                   int64_t finalg, int64_t out_head, int64_t cos_h, int64_t sin_h, int64_t page, int kv32,
+                   bool keep = false) {
   if (B <= 0 || n_layers <= 0 || H <= 0 || Hkv <= 0 || H % Hkv || hd <= 0 || hd > 128 || (hd & 1) || d <= 0 ||
       dff <= 0 || cap <= 0 || frac < 1 || frac > 29 || eps < 0 || imie_device_ready() != 0)
     return -1;
@@ -559,12 +614,16 @@ int64_t net_create(int64_t B, int64_t n_layers, int64_t H, int64_t Hkv, int64_t 
   n->sin = buf_get(sin_h, cap * (hd / 2));
   if (!n->cos || !n->sin) { delete n; return -1; }
   n->rope_rows = std::min(bufs()[(size_t)cos_h].n, bufs()[(size_t)sin_h].n) / (hd / 2);
+  if (keep) {                                          // workspaces and cache memory of the last such net
+    kept_take(*n);
+    n->arena = &kept().arena;
+  }
   {
     std::vector<const int64_t*> gt;
     for (const LayerW& L : n->layers) { gt.push_back(L.n1g); gt.push_back(L.n2g); }
     if (n->gtab.ensure(gt.size() * sizeof(void*)) || n->gmax.ensure(gt.size() * 8) ||
         hipMemcpy(n->gtab.p, gt.data(), gt.size() * sizeof(void*), hipMemcpyHostToDevice) != hipSuccess) {
-      n->gtab.release(); n->gmax.release(); delete n; return -1;
+      net_free(n); delete n; return -1;
     }
   }
   n->live = true;
@@ -600,6 +659,7 @@ void imie_buf_free_all(void) {
   (void)hipStreamSynchronize(imie_stream());
   for (auto& e : bufs()) if (e.p) imie_free(e.p);
   bufs().clear();
+  kept().give_back();
 }
 
 // gpu_native.py:559-595 / bonsai_q1_gpu.cu:3694-3819 `bonsai_prefill_forward_gpu`: whole prefill on the device,
@@ -616,7 +676,7 @@ int bonsai_prefill_forward_gpu(const int64_t* x_embed, int64_t T, int64_t d, int
       !kng)
     return IMIE_EARG;
   const int64_t h = net_create(1, n_layers, H, Hkv, hd, d, dff, T, 0, frac, eps, inv_sqrt, wq, wk, wv, wo, w1, wu,
-                               w2, n1g, n2g, qng, kng, finalg, out_head, cos_h, sin_h, T, 0);
+                               w2, n1g, n2g, qng, kng, finalg, out_head, cos_h, sin_h, T, 0, true);
   if (h < 0) return IMIE_EARG;
   Net& n = *nets()[(size_t)h];
   hipStream_t st = imie_stream();
@@ -628,22 +688,58 @@ int bonsai_prefill_forward_gpu(const int64_t* x_embed, int64_t T, int64_t d, int
     const int64_t start = 0;
     if ((rc = net_run(n, (int64_t*)n.x.p, &start, T, st))) break;
     if ((rc = net_head(n, (const int64_t*)n.x.p, {T - 1}, (int64_t*)n.logits.p, nullptr, st))) break;
+    // the cache's export: dense int64 with P = T, layer pools exactly (Hkv, T, hd), all K then all V in the arena. It goes
+    // to pinned memory behind the forward; the caller's arrays (usually fresh, so unmapped) are faulted in meanwhile,
+    // unchanged, and filled once the call is known to be good.
+    const size_t half = (size_t)n_layers * (size_t)(Hkv * T * hd) * 8;
+    const bool exp = out_k && out_v, pinned = exp && 2 * half <= kKeepPinned;
+    if (pinned) {
+      if (kept().pin_cap < 2 * half) {
+        if (kept().pin) (void)hipHostFree(kept().pin);
+        kept().pin_cap = 0;
+        if (hipHostMalloc((void**)&kept().pin, 2 * half) != hipSuccess) { kept().pin = nullptr; rc = IMIE_EARG; break; }
+        kept().pin_cap = 2 * half;
+      }
+      if (hipMemcpyAsync(kept().pin, n.kpool[0], 2 * half, hipMemcpyDeviceToHost, st) != hipSuccess) { rc = IMIE_EARG; break; }
+      for (int64_t* a : {out_k, out_v})
+        for (size_t o = 0; o < half; o += 4096) {
+          volatile char* c = (volatile char*)a + o;
+          *c = *c;
+        }
+    }
     int stat = 0;
     if ((rc = read_status(n, st, &stat))) break;
     if (stat) { rc = stat & IMIE_ERMS ? IMIE_ERMS : IMIE_EOVF; break; }
     if (hipMemcpy(out_logits, n.logits.p, (size_t)n.vocab * 8, hipMemcpyDeviceToHost) != hipSuccess) { rc = IMIE_EARG; break; }
-    if (out_k && out_v) {
-      // dense int64 cache with P = T: layer pool is exactly (Hkv, T, hd)
-      const size_t lb = (size_t)(Hkv * T * hd) * 8;
-      for (int64_t l = 0; l < n_layers; ++l) {
-        if (hipMemcpy((char*)out_k + l * lb, n.kpool[(size_t)l], lb, hipMemcpyDeviceToHost) != hipSuccess ||
-            hipMemcpy((char*)out_v + l * lb, n.vpool[(size_t)l], lb, hipMemcpyDeviceToHost) != hipSuccess) {
-          rc = IMIE_EARG;
-          break;
+    if (pinned) {
+      const char* src = kept().pin;
+      auto copy = [&](int part, int parts) {           // part of K and of V
+        const size_t a = half / (size_t)parts * (size_t)part, e = part + 1 == parts ? half : half / (size_t)parts * (size_t)(part + 1);
+        memcpy((char*)out_k + a, src + a, e - a);
+        memcpy((char*)out_v + a, src + half + a, e - a);
+      };
+      // one core copies about 10 GB/s: four of them above 8 MB (a thread that cannot start leaves its part to this one)
+      const int parts = 2 * half >= ((size_t)8 << 20) ? 4 : 1;
+      std::thread th[3];
+      for (int i = 1; i < parts; ++i) {
+        try {
+          th[i - 1] = std::thread(copy, i, parts);
+        } catch (const std::exception&) {
+          copy(i, parts);
         }
+      }
+      copy(0, parts);
+      for (auto& t : th) if (t.joinable()) t.join();
+    } else if (exp) {
+      if (hipMemcpy(out_k, n.kpool[0], half, hipMemcpyDeviceToHost) != hipSuccess ||
+          hipMemcpy(out_v, n.vpool[0], half, hipMemcpyDeviceToHost) != hipSuccess) {
+        rc = IMIE_EARG;
+        break;
       }
     }
   } while (0);
+  (void)hipStreamSynchronize(st);                      // also on refusal: the kept memory is idle
+  kept_return(n);
   net_free(&n);
   delete nets()[(size_t)h];
   nets()[(size_t)h] = nullptr;
