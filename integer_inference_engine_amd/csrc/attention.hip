@@ -116,6 +116,7 @@ __device__ inline int64_t qoff(const AttnDesc& d, int64_t r) {
 
 template <typename KT>
 __global__ __launch_bounds__(256) void attn_scores_kernel(AttnDesc d) {
+  if (d.gate && *d.gate == 0) return;
   __shared__ int64_t sq[kRowTile][129];
   __shared__ int64_t sk[kKeyTile][129];
   const int64_t rep = d.H / d.Hkv;
@@ -188,6 +189,7 @@ __global__ __launch_bounds__(256) void attn_scores_kernel(AttnDesc d) {
 }
 
 __global__ __launch_bounds__(256) void attn_softmax_kernel(AttnDesc d) {
+  if (d.gate && *d.gate == 0) return;
   __shared__ uint64_t red[256];
   const int64_t r = blockIdx.x;
   const RowInfo ri = row_info(d, r);
@@ -232,6 +234,7 @@ __global__ __launch_bounds__(256) void attn_softmax_kernel(AttnDesc d) {
 
 template <typename KT>
 __global__ __launch_bounds__(256) void attn_pv_kernel(AttnDesc d) {
+  if (d.gate && *d.gate == 0) return;
   __shared__ int64_t sp[kRowTile][kKeyTile + 1];
   __shared__ int64_t sv[kKeyTile][129];
   const int64_t rep = d.H / d.Hkv;
@@ -282,6 +285,7 @@ __global__ __launch_bounds__(256) void attn_pv_kernel(AttnDesc d) {
 }
 
 __global__ void attn_final_kernel(AttnDesc d) {
+  if (d.gate && *d.gate == 0) return;
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t rows = d.B * d.H * d.M;
   if (i >= rows * d.hd) return;
@@ -298,6 +302,7 @@ __global__ void attn_final_kernel(AttnDesc d) {
 }
 
 __global__ void attn_init_kernel(AttnDesc d) {
+  if (d.gate && *d.gate == 0) return;
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   const int64_t rows = d.B * d.H * d.M;
   if (i < rows * d.hd) d.acc[i] = 0;
@@ -1760,6 +1765,7 @@ __device__ __forceinline__ void pf_fused8_body(const AttnDesc& d, FfShared& S, i
 // follows, which does only those tiles (or every tile when the head dim is not 128) in general int64 arithmetic.
 template <int MODE, int NW>
 __global__ __launch_bounds__(64 * NW) void pf_fused8_kernel(AttnDesc d) {
+  if (d.gate && *d.gate != 0) return;                 // uniform over the launch
   __shared__ __align__(16) FfShared S;
   if (MODE == 1 && d.hd == 128 && d.rowmax[blockIdx.x] == 0) return;
   if (MODE == 2 && d.rowmax[blockIdx.x] != 0) return;
@@ -2286,6 +2292,96 @@ static void attn_set_pshift(AttnDesc& d) {
   if (d.P > 0 && (d.P & (d.P - 1)) == 0) { d.pshift = 0; while (((int64_t)1 << d.pshift) < d.P) ++d.pshift; }
 }
 
+namespace {
+// ---------------------------------------------------------------------------------------------------------
+// Prefill over an int64 cache through the kv8 kernels. The int64 kernels form 64-bit products one by one in the VALU;
+// the digit kernels do the same dot products on the matrix cores, exactly, for any cache whose values fit four balanced
+// digits (|v| <= 2139062143: any real one). So the launch first writes the cache's digit planes and maxima to scratch, as
+// one page of Lp = 64-rounded length per sequence, and runs the fused kernel on them; a value that does not fit sets the
+// gate, which turns the fused launches off and the int64 kernels behind them on. Both leave the same bits and check the
+// same bounds. The planes lie where the scores would (only the int64 kernels write those, after the planes are done
+// with), so the path is taken where they fit: rep * M * Lmax >= about hd * Lp, i.e. from 32 rows at 4 heads per kv head.
+// Fewer rows are a few key tiles of the int64 kernels.
+// 256 rows, 32 heads over 8 kv heads of 128: 372 us (scores 227, softmax 25, PV 109, ends 11) -> 70 (planes 17 + 2, fused
+// 38, idle launches 13).
+// ---------------------------------------------------------------------------------------------------------
+struct Kv8Copy {
+  uint64_t *run, *old, *gate;      // [2][B * Hkv] maxima, zeros, flag
+  int64_t* pt;                     // page b of sequence b
+  int8_t *k, *v;
+  int64_t Lp;
+};
+// the layout in the scores' space, or k == nullptr where it does not fit
+Kv8Copy kv8_copy(const AttnDesc& d) {
+  Kv8Copy c{};
+  c.Lp = (d.Lmax + 63) / 64 * 64;
+  const size_t n = (size_t)(d.B * d.Hkv), plane = n * (size_t)(c.Lp * d.hd) * 4;
+  if (d.M == 1 || 2 * plane > (size_t)(d.B * d.H * d.M * d.Lmax) * 8 || 4 * d.hd * c.Lp >= ((int64_t)1 << 31) ||
+      4 * n + 1 + (size_t)d.B > (size_t)(d.B * d.H * d.M))
+    return c;
+  c.run = (uint64_t*)d.pmax;                           // at least a word per row, unused by the int64 kernels
+  c.old = c.run + 2 * n;
+  c.gate = c.old + 2 * n;
+  c.pt = (int64_t*)(c.gate + 1);
+  c.k = (int8_t*)d.scores;
+  c.v = c.k + plane;
+  return c;
+}
+__global__ void kv8_copy_init_kernel(Kv8Copy c, int64_t n, int64_t B) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < 4 * n + 1) c.run[i] = 0;                     // maxima, zeros, gate
+  if (i < B) c.pt[i] = i;
+}
+// workgroup = 64 keys of a (sequence, kv head), blockIdx.z: K or V. A thread takes one dim of 16 consecutive keys (loads
+// of consecutive dims, coalesced); V's slots are consecutive: 16-byte stores a plane; K's 16-dim pieces: byte stores,
+// the 16 lanes of a piece and the 16 keys filling 256 consecutive bytes between them.
+__global__ __launch_bounds__(256) void kv8_copy_kernel(AttnDesc d, Kv8Copy c) {
+  const int64_t bkv = blockIdx.x, b = imie_udiv32(bkv, d.Hkv), kv = imie_umod32(bkv, d.Hkv);
+  const int64_t len = d.starts ? d.starts[b] + d.M : d.lengths[b];
+  const int64_t j0 = (int64_t)blockIdx.y * 64;
+  if (j0 >= len) return;
+  const bool isv = blockIdx.z != 0;
+  const void* pool = isv ? d.V : d.K;
+  int8_t* blk = (isv ? c.v : c.k) + imie_kv8::block_base(b, kv, d.Hkv, d.hd, c.Lp);
+  uint64_t mx = 0;
+  for (int i = threadIdx.x; i < 4 * d.hd; i += 256) {
+    const int c0 = (int)imie_umod32(i, d.hd);
+    const int64_t j = j0 + 16 * imie_udiv32(i, d.hd);
+    uint32_t pl[4][4];                                 // [plane][four keys]
+#pragma unroll
+    for (int h = 0; h < 4; ++h) {
+      uint32_t dg[4], t[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int64_t jj = j + 4 * h + u;
+        const int64_t v = jj < len ? key_ptr<int64_t>(d, pool, b, kv, jj)[c0] : 0;
+        const uint64_t a = imie_absu64(v);
+        mx = a > mx ? a : mx;
+        dg[u] = imie_digits32((uint32_t)(uint64_t)v);
+      }
+      imie_bytes4x4(dg[0], dg[1], dg[2], dg[3], t);
+#pragma unroll
+      for (int db = 0; db < 4; ++db) pl[db][h] = t[db];
+    }
+#pragma unroll
+    for (int db = 0; db < 4; ++db) {
+      if (isv) {
+        *(uint4*)(blk + imie_kv8::v_off(j, db, c0, d.hd, c.Lp)) = uint4{pl[db][0], pl[db][1], pl[db][2], pl[db][3]};
+      } else {
+        int8_t* q = blk + imie_kv8::k_off(j, db, c0, d.hd);
+#pragma unroll
+        for (int u = 0; u < 16; ++u) q[16 * u] = (int8_t)(uint8_t)(pl[db][u >> 2] >> (8 * (u & 3)));
+      }
+    }
+  }
+  mx = imie_wave_max_u64(mx);
+  if ((threadIdx.x & 63) == 0) {
+    amax_u64(&c.run[(isv ? d.B * d.Hkv : 0) + bkv], mx);
+    if (mx > (uint64_t)imie_kv8::kCap) atomicOr((unsigned long long*)c.gate, 1ull);
+  }
+}
+}  // namespace
+
 size_t imie_attn_scratch_bytes(int64_t B, int64_t H, int64_t Hkv, int64_t M, int64_t hd, int64_t Lmax) {
   const int64_t rows = B * H * M;
   int64_t chunk = 0, nch = 0;
@@ -2332,6 +2428,15 @@ void imie_attn_qdigit_scratch(const AttnDesc& d, int8_t** qd, int** qlimbs) {
   int64_t* p = (int64_t*)d.cvm + nch * d.B * d.Hkv;
   *qd = (int8_t*)(((uintptr_t)p + 15) & ~(uintptr_t)15);
   *qlimbs = (int*)(*qd + rows * 8 * d.hd);
+}
+
+static void pf_fused8_launch(const AttnDesc& d, hipStream_t st) {
+  const int64_t npt = (d.M + kFfRows - 1) / kFfRows;
+  if (d.hd == 128) {
+    hipLaunchKernelGGL((pf_fused8_kernel<0, 4>), dim3((unsigned)(d.B * d.H * npt)), dim3(256), 0, st, d);
+    hipLaunchKernelGGL((pf_fused8_kernel<2, 4>), dim3((unsigned)(d.B * d.H * npt)), dim3(256), 0, st, d);
+  }
+  hipLaunchKernelGGL((pf_fused8_kernel<1, 4>), dim3((unsigned)(d.B * d.H * npt)), dim3(256), 0, st, d);
 }
 
 int imie_attention_launch(AttnDesc d, hipStream_t st) {
@@ -2409,12 +2514,7 @@ int imie_attention_launch(AttnDesc d, hipStream_t st) {
   if (d.kv32) {                                      // kv8 prefill: MFMA scores, softmax to p digits, MFMA PV
     if (d.hd % 16 != 0 || !d.run_k || !d.run_v || d.P >= ((int64_t)1 << 27)) return IMIE_EARG;
     if (d.hd <= 128 && pf_fused()) {
-      const int64_t npt = (d.M + kFfRows - 1) / kFfRows;
-      if (d.hd == 128) {
-        hipLaunchKernelGGL((pf_fused8_kernel<0, 4>), dim3((unsigned)(d.B * d.H * npt)), dim3(256), 0, st, d);
-        hipLaunchKernelGGL((pf_fused8_kernel<2, 4>), dim3((unsigned)(d.B * d.H * npt)), dim3(256), 0, st, d);
-      }
-      hipLaunchKernelGGL((pf_fused8_kernel<1, 4>), dim3((unsigned)(d.B * d.H * npt)), dim3(256), 0, st, d);
+      pf_fused8_launch(d, st);
       IMIE_HIP(hipGetLastError());
       imie_prof_mark(IMIE_K_ATTN, st, false);
       return IMIE_OK;
@@ -2436,6 +2536,23 @@ int imie_attention_launch(AttnDesc d, hipStream_t st) {
     IMIE_HIP(hipGetLastError());
     imie_prof_mark(IMIE_K_ATTN, st, false);
     return IMIE_OK;
+  }
+  if (d.hd % 16 == 0 && d.hd <= 128 && pf_fused()) {
+    const Kv8Copy c = kv8_copy(d);
+    if (c.k) {
+      const int64_t n = d.B * d.Hkv;
+      hipLaunchKernelGGL(kv8_copy_init_kernel, dim3((unsigned)((4 * n + 1 + d.B + 255) / 256)), dim3(256), 0, st, c, n, d.B);
+      hipLaunchKernelGGL(kv8_copy_kernel, dim3((unsigned)n, (unsigned)(c.Lp / 64), 2), dim3(256), 0, st, d, c);
+      IMIE_HIP(hipGetLastError());
+      d.gate = c.gate;
+      AttnDesc f = d;
+      f.kv32 = 1; f.K = c.k; f.V = c.v;
+      f.run_k = c.run; f.run_v = c.run + n; f.old_k = c.old; f.old_v = c.old + n;
+      f.pt = c.pt; f.P = c.Lp; f.mp = 1;
+      attn_set_pshift(f);
+      pf_fused8_launch(f, st);
+      IMIE_HIP(hipGetLastError());
+    }
   }
   hipLaunchKernelGGL(attn_init_kernel, dim3((unsigned)((ninit + 255) / 256)), dim3(256), 0, st, d);
   IMIE_HIP(hipGetLastError());

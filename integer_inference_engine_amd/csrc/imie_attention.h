@@ -24,6 +24,7 @@ struct AttnDesc {
   int64_t* out;
   int* status;
   const uint64_t* rope_guard;      // optional: q/k RoPE envelope maxima (4 x u64), checked by the final kernel
+  const uint64_t* gate;            // int64 prefill: nonzero where a key or value does not fit the kv8 digits (nullptr: none)
   // scratch (imie_attn_bind_scratch)
   int64_t* scores;
   uint64_t* acc;
