@@ -963,6 +963,7 @@ struct GemmArgs {
   int64_t ntiles16;                // 16 * tiles: rows of the tiled scale layout
   int frac, accumulate;
   int kfold;                       // > 0: high-dword epilogue (narrow kernel), folded every kfold blocks
+  int split64;                     // 64-bit scales: the narrow kernel takes them in two 32-bit parts
   int rlen;                        // q1_gemm_ps_kernel<.., 2>: first block of the second int32 partial sum
   int ksplit;                      // narrow kernel: blocks split over gridDim.y ranges, outputs added atomically
   int64_t* out;
@@ -1033,8 +1034,14 @@ __device__ inline void gemm_slab_limbs(const GemmArgs& a, int64_t t0g, int* s_lw
 // + H with H = A * 2^32, so the high dword of p is A + floor(S * scale / 2^frac) exactly; clearing p's low dword
 // gives the next H (one v_mad_i64_i32 and one clear). A is folded into the int64 sum every kfold blocks, chosen
 // on the host so |A| + max|q| stays below 2^31 (|S| < 2^30 on <= 3 limbs).
+// S64 and FE (64-bit scales up to 2^33, 4 <= frac <= 31, the host's split64: the codec's whole fp16 range at 16 fraction
+// bits is below 2^32): a scale is a 2^frac + b with b in [-2^(frac-1), 2^(frac-1)), and since S * scale stays below 2^63
+// the floor is S a + floor(S b / 2^frac) exactly: one v_mad_i64_i32 into the sum, one v_mul_hi_i32 by b << (32 - frac) and
+// one add instead of a 64 x 64 product, a 64-bit shift and an add.
+// The kernel is bound by VALU issue: a call of 93 rows, 12288 -> 4096, 60.2 -> 55.5 us; of 200 rows 92 -> 83.
 template <bool S64, int NBUF, bool FE>
 __global__ __launch_bounds__(256) void q1_gemm_narrow_kernel(GemmArgs a) {
+  constexpr bool SP = S64 && FE;
   constexpr int MT = 2, NT = 4;
   __shared__ int s_lw[kGemmMaxSlabs];
   // [buffer][limb][token][shift], tokens padded to 9 x 16 B: the 16 lanes of a quarter-wave read tokens
@@ -1091,11 +1098,16 @@ __global__ __launch_bounds__(256) void q1_gemm_narrow_kernel(GemmArgs a) {
     for (int l = 0; l < kNarrowLimbs; ++l)
 #pragma unroll
       for (int u = 0; u < 2; ++u) sA[buf][l][st_tok][st_s + u] = pa[l][u];
+    if (SP) {                                         // the scale's parts: a above, b << (32 - frac) below
+      const int64_t b = (int64_t)((uint64_t)ps << (64 - a.frac)) >> (64 - a.frac);
+      ps = (ST)((uint64_t)(((int64_t)ps - b) >> a.frac) << 32 | (uint32_t)((uint64_t)b << (32 - a.frac)));
+    }
     if (tid < 128) { sB[buf][tid] = pb; sS[buf][tid] = ps; }
     if (tid < 64) sT[buf][tid] = 0 - pt;             // negated block totals: S = (D << 1) + sT, one v_lshl_add
   };
   int64_t acc[MT][NT][4];
-  int64_t accH[FE ? MT : 1][FE ? NT : 1][4];
+  constexpr bool HI = FE && !S64;                     // the high-dword epilogue and its fold
+  int64_t accH[HI ? MT : 1][HI ? NT : 1][4];
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
@@ -1103,7 +1115,7 @@ __global__ __launch_bounds__(256) void q1_gemm_narrow_kernel(GemmArgs a) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         acc[i][jj][r] = 0;
-        if (FE) accH[FE ? i : 0][FE ? jj : 0][r] = 0;
+        if (HI) accH[HI ? i : 0][HI ? jj : 0][r] = 0;
       }
   int fcount = 0;
   auto fold = [&]() {
@@ -1113,8 +1125,8 @@ __global__ __launch_bounds__(256) void q1_gemm_narrow_kernel(GemmArgs a) {
       for (int jj = 0; jj < NT; ++jj)
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          acc[i][jj][r] = (int64_t)((uint64_t)acc[i][jj][r] + (uint64_t)(accH[FE ? i : 0][FE ? jj : 0][r] >> 32));
-          accH[FE ? i : 0][FE ? jj : 0][r] = 0;
+          acc[i][jj][r] = (int64_t)((uint64_t)acc[i][jj][r] + (uint64_t)(accH[HI ? i : 0][HI ? jj : 0][r] >> 32));
+          accH[HI ? i : 0][HI ? jj : 0][r] = 0;
         }
   };
   // this workgroup's block range (the whole K unless the launch splits it for a small token count)
@@ -1172,7 +1184,27 @@ __global__ __launch_bounds__(256) void q1_gemm_narrow_kernel(GemmArgs a) {
             D[i][jj] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[i][1], bx[jj][1], c, 0, 0, 0);
           }
       }
-      if (FE) {
+      if constexpr (SP) {
+        int32_t sa[NT], sb[NT];
+#pragma unroll
+        for (int jj = 0; jj < NT; ++jj) {
+          const int64_t sc = (int64_t)sS[buf][ob + 16 * jj + m];
+          sa[jj] = (int32_t)(sc >> 32);
+          sb[jj] = (int32_t)sc;
+        }
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const uint32_t ntot = (uint32_t)sT[buf][tb + 16 * i + 4 * g + r];
+#pragma unroll
+            for (int jj = 0; jj < NT; ++jj) {
+              const int32_t S = (int32_t)(((uint32_t)D[i][jj][r] << 1) + ntot);
+              const int64_t lo = (int64_t)(int32_t)(((int64_t)S * (int64_t)sb[jj]) >> 32);
+              acc[i][jj][r] = (int64_t)((uint64_t)acc[i][jj][r] + (uint64_t)lo + (uint64_t)((int64_t)S * (int64_t)sa[jj]));
+            }
+          }
+      } else if constexpr (FE) {
         int32_t scp[NT];
 #pragma unroll
         for (int jj = 0; jj < NT; ++jj) scp[jj] = (int32_t)((uint32_t)sS[buf][ob + 16 * jj + m] << (32 - a.frac));
@@ -1184,8 +1216,8 @@ __global__ __launch_bounds__(256) void q1_gemm_narrow_kernel(GemmArgs a) {
 #pragma unroll
             for (int jj = 0; jj < NT; ++jj) {
               const int32_t S = (int32_t)(((uint32_t)D[i][jj][r] << 1) + ntot);
-              const int64_t p = (int64_t)S * (int64_t)scp[jj] + accH[FE ? i : 0][FE ? jj : 0][r];
-              accH[FE ? i : 0][FE ? jj : 0][r] = p & (int64_t)0xFFFFFFFF00000000ll;
+              const int64_t p = (int64_t)S * (int64_t)scp[jj] + accH[HI ? i : 0][HI ? jj : 0][r];
+              accH[HI ? i : 0][HI ? jj : 0][r] = p & (int64_t)0xFFFFFFFF00000000ll;
             }
           }
         if (++fcount == a.kfold) { fold(); fcount = 0; }
@@ -1215,7 +1247,7 @@ __global__ __launch_bounds__(256) void q1_gemm_narrow_kernel(GemmArgs a) {
       __syncthreads();
     }
   }
-  if (FE) fold();
+  if (HI) fold();
 #pragma unroll
   for (int i = 0; i < MT; ++i)
 #pragma unroll
@@ -2251,6 +2283,7 @@ static int q1_gemm_multi(const Q1Weight* const* ws, int cnt, const int64_t* x_de
     // high-dword epilogue: int32 scales below 2^(frac-1); |q| = |floor(S * scale / 2^frac)| <= max_q with
     // |S| < 2^30 (narrow blocks); fold before |A| + max_q could reach 2^31
     ga.kfold = 0;
+    ga.split64 = w.scale64 && ga.frac >= 4 && ga.frac <= 31 && w.maxsc <= ((int64_t)1 << 33) && gemm_fast_epi();
     if (!w.scale64 && ga.frac >= 1 && ga.frac <= 31 && w.maxsc < ((int64_t)1 << (ga.frac - 1)) && gemm_fast_epi()) {
       const int64_t max_q = (((int64_t)w.maxsc << 30) >> ga.frac) + 2;
       const int64_t k = (((int64_t)1 << 31) - 1) / max_q - 1;
@@ -2395,7 +2428,10 @@ static int q1_gemm_multi(const Q1Weight* const* ws, int cnt, const int64_t* x_de
           hipLaunchKernelGGL(q1_zero_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, outs[i], n);
         }
         if (w.scale64) {
-          if (nbuf == 1) hipLaunchKernelGGL((q1_gemm_narrow_kernel<true, 1, false>), ngrid, dim3(256), 0, st, ga);
+          if (ga.split64) {
+            if (nbuf == 1) hipLaunchKernelGGL((q1_gemm_narrow_kernel<true, 1, true>), ngrid, dim3(256), 0, st, ga);
+            else hipLaunchKernelGGL((q1_gemm_narrow_kernel<true, 2, true>), ngrid, dim3(256), 0, st, ga);
+          } else if (nbuf == 1) hipLaunchKernelGGL((q1_gemm_narrow_kernel<true, 1, false>), ngrid, dim3(256), 0, st, ga);
           else hipLaunchKernelGGL((q1_gemm_narrow_kernel<true, 2, false>), ngrid, dim3(256), 0, st, ga);
           hipLaunchKernelGGL(q1_gemm_wide_kernel<true>, grid, dim3(256), 0, st, ga);
         } else {

@@ -223,3 +223,27 @@ def test_gemm_batched_decode_epilogue_extremes(gpu, frac, T):
     x[T - 1, 5 * 128 + 3] = cap3 + 1                  # slab 1 needs 4 limbs for every token of the tile
     got = gpu.q1_apply_gpu(x, bits, scale, frac)
     assert got is not None and np.array_equal(got, q1_linear(x, bits, scale, frac))
+
+
+@pytest.mark.parametrize("frac", [3, 4, 16, 31, 32])
+@pytest.mark.parametrize("top", [1 << 33, (1 << 33) + 1])
+def test_gemm_split_scales(gpu, frac, top):
+    """64-bit scales in two 32-bit parts (up to 2^33 and 4 <= frac <= 31) and just beyond: scales at the limit, at the
+    edges of the lower part's range and beyond int32, with activations at the 3-limb cap and beyond it (wide blocks)."""
+    cap3 = 127 * (1 + 256 + 65536)
+    N, nb, T = 48, 9, 20
+    rng = np.random.default_rng(frac)
+    bits = rng.integers(0, 256, size=(N, nb, 16), dtype=np.uint8)
+    bits[:8] = 0xFF
+    bits[8:16] = 0
+    half = 1 << (frac - 1)
+    edges = [top, -top, half, half - 1, -half, -half - 1, (1 << 32) + half, -(1 << 32) - half, 1 << 31, 0, 1]
+    scale = rng.choice(np.array(edges, dtype=np.int64), size=(N, nb))
+    scale[:4] = top
+    scale[8:12] = -top
+    x = rng.choice(np.array([cap3, -cap3, cap3 - 1, 0], dtype=np.int64), size=(T, nb * 128))
+    x[:4] = cap3
+    x[4:8] = -cap3
+    x[16, :512] = 1 << 40
+    got = gpu.q1_apply_gpu(x, bits, scale, frac)
+    assert got is not None and np.array_equal(got, q1_linear(x, bits, scale, frac))
