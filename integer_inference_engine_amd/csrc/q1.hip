@@ -1041,7 +1041,7 @@ __device__ inline void gemm_slab_limbs(const GemmArgs& a, int64_t t0g, int* s_lw
 // The kernel is bound by VALU issue: a call of 93 rows, 12288 -> 4096, 60.2 -> 55.5 us; of 200 rows 92 -> 83.
 template <bool S64, int NBUF, bool FE>
 __global__ __launch_bounds__(256) void q1_gemm_narrow_kernel(GemmArgs a) {
-  constexpr bool SP = S64 && FE;
+  constexpr bool SP = S64 && FE, HI = FE && !S64;     // split scales; the high-dword epilogue and its fold
   constexpr int MT = 2, NT = 4;
   __shared__ int s_lw[kGemmMaxSlabs];
   // [buffer][limb][token][shift], tokens padded to 9 x 16 B: the 16 lanes of a quarter-wave read tokens
@@ -1059,9 +1059,15 @@ __global__ __launch_bounds__(256) void q1_gemm_narrow_kernel(GemmArgs a) {
   if (!live) return;
   gemm_slab_limbs(a, t0g, s_lw);
   const int m = lane & 15, g = lane >> 4;
-  const int tb = (wave >> 1) * 32;                    // this wave's first token within the workgroup tile
-  const int ob = (wave & 1) * 64;                     // this wave's first output within the workgroup tile
-  const int64_t o0g = o0 - ob;
+  // a tile whose upper 32 tokens are absent (T mod 64 in 1..32): the four waves split the outputs, 32 each, instead of
+  // two of them working on padding. Not with the high-dword epilogue, whose sums leave no registers for a second copy of
+  // the block (it spilled 240 bytes). 64-bit scales, 12288 outputs of 4096: 9 rows 34.2 -> 28.2 us, 65 60.5 -> 47.2.
+  const bool half = !HI && t0g + 32 >= a.T;
+  const int64_t o0g = o0 - (wave & 1) * 64;
+  const int tb = half ? 0 : (wave >> 1) * 32;         // this wave's first token within the workgroup tile
+  const int ob = half ? wave * 32 : (wave & 1) * 64;  // this wave's first output within the workgroup tile
+  t0 = t0g + tb;
+  o0 = o0g + ob;
   // cooperative stage: thread -> token tid >> 2, shifts 2 (tid & 3) + {0, 1} of every limb; threads < 128 also
   // one output's bits + scale, threads < 64 one token's total
   const int st_tok = tid >> 2, st_s = 2 * (tid & 3);
@@ -1106,7 +1112,6 @@ __global__ __launch_bounds__(256) void q1_gemm_narrow_kernel(GemmArgs a) {
     if (tid < 64) sT[buf][tid] = 0 - pt;             // negated block totals: S = (D << 1) + sT, one v_lshl_add
   };
   int64_t acc[MT][NT][4];
-  constexpr bool HI = FE && !S64;                     // the high-dword epilogue and its fold
   int64_t accH[HI ? MT : 1][HI ? NT : 1][4];
 #pragma unroll
   for (int i = 0; i < MT; ++i)
@@ -1129,6 +1134,106 @@ __global__ __launch_bounds__(256) void q1_gemm_narrow_kernel(GemmArgs a) {
           accH[HI ? i : 0][HI ? jj : 0][r] = 0;
         }
   };
+  // one block: NJ 16-output tiles of this wave
+  auto compute = [&](auto njc, int buf, int lw) {
+    constexpr int NJ = decltype(njc)::value;
+    v4i bx[NJ][2];
+#pragma unroll
+    for (int jj = 0; jj < NJ; ++jj) {
+      const uint4 w = sB[buf][ob + 16 * jj + m];
+      bx[jj][0] = expand_bits(w, g);
+      bx[jj][1] = expand_bits(w, 4 + g);
+    }
+    // pos = sum_l D_l 256^l by Horner from the top limb: acc = (acc << 8) + MFMA(limb l); one shift per
+    // element per limb, exact in int32 (every partial is bounded by |pos| <= 2^30)
+    v4i D[MT][NJ];
+    {
+      // top limb from a zero accumulator (no shift), then Horner down to limb 0
+      const int l = lw - 1;
+      v4i av[MT][2];
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) av[i][h] = sA[buf][l][tb + 16 * i + m][4 * h + g];
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int jj = 0; jj < NJ; ++jj) {
+          const v4i c = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[i][0], bx[jj][0], v4i{0, 0, 0, 0}, 0, 0, 0);
+          D[i][jj] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[i][1], bx[jj][1], c, 0, 0, 0);
+        }
+    }
+    for (int l = lw - 2; l >= 0; --l) {
+      v4i av[MT][2];
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) av[i][h] = sA[buf][l][tb + 16 * i + m][4 * h + g];
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int jj = 0; jj < NJ; ++jj) {
+          v4i c = D[i][jj];
+          c = v4i{(int)((uint32_t)c[0] << 8), (int)((uint32_t)c[1] << 8), (int)((uint32_t)c[2] << 8),
+                  (int)((uint32_t)c[3] << 8)};
+          c = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[i][0], bx[jj][0], c, 0, 0, 0);
+          D[i][jj] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[i][1], bx[jj][1], c, 0, 0, 0);
+        }
+    }
+    if constexpr (SP) {
+      int32_t sa[NJ], sb[NJ];
+#pragma unroll
+      for (int jj = 0; jj < NJ; ++jj) {
+        const int64_t sc = (int64_t)sS[buf][ob + 16 * jj + m];
+        sa[jj] = (int32_t)(sc >> 32);
+        sb[jj] = (int32_t)sc;
+      }
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const uint32_t ntot = (uint32_t)sT[buf][tb + 16 * i + 4 * g + r];
+#pragma unroll
+          for (int jj = 0; jj < NJ; ++jj) {
+            const int32_t S = (int32_t)(((uint32_t)D[i][jj][r] << 1) + ntot);
+            const int64_t lo = (int64_t)(int32_t)(((int64_t)S * (int64_t)sb[jj]) >> 32);
+            acc[i][jj][r] = (int64_t)((uint64_t)acc[i][jj][r] + (uint64_t)lo + (uint64_t)((int64_t)S * (int64_t)sa[jj]));
+          }
+        }
+    } else if constexpr (FE) {
+      int32_t scp[NJ];
+#pragma unroll
+      for (int jj = 0; jj < NJ; ++jj) scp[jj] = (int32_t)((uint32_t)sS[buf][ob + 16 * jj + m] << (32 - a.frac));
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const uint32_t ntot = (uint32_t)sT[buf][tb + 16 * i + 4 * g + r];
+#pragma unroll
+          for (int jj = 0; jj < NJ; ++jj) {
+            const int32_t S = (int32_t)(((uint32_t)D[i][jj][r] << 1) + ntot);
+            const int64_t p = (int64_t)S * (int64_t)scp[jj] + accH[HI ? i : 0][HI ? jj : 0][r];
+            accH[HI ? i : 0][HI ? jj : 0][r] = p & (int64_t)0xFFFFFFFF00000000ll;
+          }
+        }
+      if (++fcount == a.kfold) { fold(); fcount = 0; }
+    } else {
+#pragma unroll
+      for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const uint32_t ntot = (uint32_t)sT[buf][tb + 16 * i + 4 * g + r];
+#pragma unroll
+          for (int jj = 0; jj < NJ; ++jj) {
+            const int32_t S = (int32_t)(((uint32_t)D[i][jj][r] << 1) + ntot);
+            const ST sc = sS[buf][ob + 16 * jj + m];
+            const int64_t prod = S64 ? (int64_t)((uint64_t)(int64_t)S * (uint64_t)(int64_t)sc)
+                                     : (int64_t)S * (int64_t)(int32_t)sc;   // one v_mad_i64_i32
+            acc[i][jj][r] = (int64_t)((uint64_t)acc[i][jj][r] + (uint64_t)imie_floor_shift(prod, a.frac));
+          }
+        }
+    }
+  };
   // this workgroup's block range (the whole K unless the launch splits it for a small token count)
   const int64_t b0 = (int64_t)blockIdx.y * a.nb / a.ksplit, b1 = ((int64_t)blockIdx.y + 1) * a.nb / a.ksplit;
   if (b0 >= b1) return;
@@ -1141,102 +1246,9 @@ __global__ __launch_bounds__(256) void q1_gemm_narrow_kernel(GemmArgs a) {
     if (more) stage_load(b + 1);                      // next block's operands in flight during this block
     const int lw = s_lw[b >> 2];
     if (lw <= kNarrowLimbs) {
-      v4i bx[NT][2];
-#pragma unroll
-      for (int jj = 0; jj < NT; ++jj) {
-        const uint4 w = sB[buf][ob + 16 * jj + m];
-        bx[jj][0] = expand_bits(w, g);
-        bx[jj][1] = expand_bits(w, 4 + g);
-      }
-      // pos = sum_l D_l 256^l by Horner from the top limb: acc = (acc << 8) + MFMA(limb l); one shift per
-      // element per limb, exact in int32 (every partial is bounded by |pos| <= 2^30)
-      v4i D[MT][NT];
-      {
-        // top limb from a zero accumulator (no shift), then Horner down to limb 0
-        const int l = lw - 1;
-        v4i av[MT][2];
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-#pragma unroll
-          for (int h = 0; h < 2; ++h) av[i][h] = sA[buf][l][tb + 16 * i + m][4 * h + g];
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-#pragma unroll
-          for (int jj = 0; jj < NT; ++jj) {
-            const v4i c = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[i][0], bx[jj][0], v4i{0, 0, 0, 0}, 0, 0, 0);
-            D[i][jj] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[i][1], bx[jj][1], c, 0, 0, 0);
-          }
-      }
-      for (int l = lw - 2; l >= 0; --l) {
-        v4i av[MT][2];
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-#pragma unroll
-          for (int h = 0; h < 2; ++h) av[i][h] = sA[buf][l][tb + 16 * i + m][4 * h + g];
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-#pragma unroll
-          for (int jj = 0; jj < NT; ++jj) {
-            v4i c = D[i][jj];
-            c = v4i{(int)((uint32_t)c[0] << 8), (int)((uint32_t)c[1] << 8), (int)((uint32_t)c[2] << 8),
-                    (int)((uint32_t)c[3] << 8)};
-            c = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[i][0], bx[jj][0], c, 0, 0, 0);
-            D[i][jj] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[i][1], bx[jj][1], c, 0, 0, 0);
-          }
-      }
-      if constexpr (SP) {
-        int32_t sa[NT], sb[NT];
-#pragma unroll
-        for (int jj = 0; jj < NT; ++jj) {
-          const int64_t sc = (int64_t)sS[buf][ob + 16 * jj + m];
-          sa[jj] = (int32_t)(sc >> 32);
-          sb[jj] = (int32_t)sc;
-        }
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const uint32_t ntot = (uint32_t)sT[buf][tb + 16 * i + 4 * g + r];
-#pragma unroll
-            for (int jj = 0; jj < NT; ++jj) {
-              const int32_t S = (int32_t)(((uint32_t)D[i][jj][r] << 1) + ntot);
-              const int64_t lo = (int64_t)(int32_t)(((int64_t)S * (int64_t)sb[jj]) >> 32);
-              acc[i][jj][r] = (int64_t)((uint64_t)acc[i][jj][r] + (uint64_t)lo + (uint64_t)((int64_t)S * (int64_t)sa[jj]));
-            }
-          }
-      } else if constexpr (FE) {
-        int32_t scp[NT];
-#pragma unroll
-        for (int jj = 0; jj < NT; ++jj) scp[jj] = (int32_t)((uint32_t)sS[buf][ob + 16 * jj + m] << (32 - a.frac));
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const uint32_t ntot = (uint32_t)sT[buf][tb + 16 * i + 4 * g + r];
-#pragma unroll
-            for (int jj = 0; jj < NT; ++jj) {
-              const int32_t S = (int32_t)(((uint32_t)D[i][jj][r] << 1) + ntot);
-              const int64_t p = (int64_t)S * (int64_t)scp[jj] + accH[HI ? i : 0][HI ? jj : 0][r];
-              accH[HI ? i : 0][HI ? jj : 0][r] = p & (int64_t)0xFFFFFFFF00000000ll;
-            }
-          }
-        if (++fcount == a.kfold) { fold(); fcount = 0; }
-      } else {
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const uint32_t ntot = (uint32_t)sT[buf][tb + 16 * i + 4 * g + r];
-#pragma unroll
-            for (int jj = 0; jj < NT; ++jj) {
-              const int32_t S = (int32_t)(((uint32_t)D[i][jj][r] << 1) + ntot);
-              const ST sc = sS[buf][ob + 16 * jj + m];
-              const int64_t prod = S64 ? (int64_t)((uint64_t)(int64_t)S * (uint64_t)(int64_t)sc)
-                                       : (int64_t)S * (int64_t)(int32_t)sc;   // one v_mad_i64_i32
-              acc[i][jj][r] = (int64_t)((uint64_t)acc[i][jj][r] + (uint64_t)imie_floor_shift(prod, a.frac));
-            }
-          }
-      }
+      if constexpr (HI) compute(std::integral_constant<int, NT>{}, buf, lw);
+      else if (half) compute(std::integral_constant<int, 2>{}, buf, lw);
+      else compute(std::integral_constant<int, NT>{}, buf, lw);
     }
     if (NBUF == 2) {
       if (more) stage_store(buf ^ 1);
@@ -1253,7 +1265,7 @@ __global__ __launch_bounds__(256) void q1_gemm_narrow_kernel(GemmArgs a) {
 #pragma unroll
     for (int jj = 0; jj < NT; ++jj) {
       const int64_t o = o0 + 16 * jj + m;
-      if (o >= a.N) continue;
+      if (o >= a.N || (half && jj >= 2)) continue;
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int64_t t = t0 + 16 * i + 4 * g + r;

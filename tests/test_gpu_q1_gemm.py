@@ -247,3 +247,17 @@ def test_gemm_split_scales(gpu, frac, top):
     x[16, :512] = 1 << 40
     got = gpu.q1_apply_gpu(x, bits, scale, frac)
     assert got is not None and np.array_equal(got, q1_linear(x, bits, scale, frac))
+
+
+@pytest.mark.parametrize("T", [9, 31, 32, 33, 65, 96, 97])
+@pytest.mark.parametrize("smax", [1 << 11, 1 << 15, 1 << 20, 1 << 32, 1 << 40])
+def test_gemm_half_token_tiles(gpu, T, smax):
+    """Token counts on both sides of a tile's half (a tile without its upper 32 tokens splits the outputs over all waves),
+    over every epilogue: int32 scales with and without the high-dword form, 64-bit scales split and whole."""
+    N, nb = 200, 6
+    seed = T + smax.bit_length()
+    bits = prng.uniform_bytes(seed, 1, (N, nb, 16))
+    scale = prng.uniform_int(seed, 2, (N, nb), -smax, smax)
+    x = prng.uniform_int(seed, 3, (T, nb * 128), -(1 << 22), 1 << 22)
+    got = gpu.q1_apply_gpu(x, bits, scale, 16)
+    assert got is not None and np.array_equal(got, q1_linear(x, bits, scale, 16))
