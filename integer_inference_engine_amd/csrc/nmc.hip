@@ -898,8 +898,8 @@ __device__ inline int64_t moe_result(i128 t, int fw, bool* fits) {
   return (int64_t)y;
 }
 
-// No load in flight (after a staging there is none): the compiler's count of them at a block loop's entry is then the
-// loop's own, and its waits for one weight slot leave the other slot's loads in flight.
+// No load in flight (after a staging there is none anyway): the compiler's count of them at a block loop's entry is then
+// the loop's own, so it waits for a block's weights and not for whatever the staging may have left.
 __device__ inline void moe_settle() { __builtin_amdgcn_s_waitcnt(0x0F70); }   // vmcnt(0)
 
 // The lane's A operand: limb l of token t (row m = 4 t + l of the MFMA), K group kg: byte offset of [l][t][8 kg].
