@@ -739,9 +739,9 @@ __global__ __launch_bounds__(512) void q1_row_kernel(const v4i* __restrict__ bit
 // bits); the weights of an 8B layer are 0.5 to 13 MB.
 // Why not the one-token kernel over several tokens: its 48 KB of staging held no limb of four tokens over eight slabs,
 // so every operand came from L2. Measured, that kernel against this one at 2, 4, 7 tokens (us, with the prep launch):
-// 4096 x 4096 10.8, 10.7, 16.6 / 9.9, 10.5, 12.8; 12288 x 4096 12.6, 17.6, 28.5 / 11.9, 13.7, 17.1; the 151,936-row
-// head 59, 299, 522 / 64, 91, 138. At 8 tokens against the GEMM kernels 16.4, 24.2, 176 / 13.6, 18.5, 151; at 10 it
-// would be 17.9, 27.2, 182 against 16.3, 24.8, 176, so the line (kGemmMinT) lies behind 8.
+// 4096 x 4096 10.7, 11.0, 17.7 / 10.6, 10.9, 11.4; 12288 x 4096 12.5, 17.3, 28.2 / 11.5, 13.5, 16.7; the 151,936-row
+// head 59, 299, 523 / 48, 68, 102. At 8 tokens against the GEMM kernels 16.3, 24.3, 176 / 11.9, 17.8, 112; the GEMM takes
+// 16.1, 24.0, 176 at 9, where the line (kGemmMinT) lies: this kernel is instantiated for up to 8.
 // ------------------------------------------------------------------------------------------------------
 constexpr int kFewLimbs = 4;
 constexpr int64_t kFewLds = 144 * 1024;   // digits resident in LDS: 2 KB a token and slab
@@ -796,12 +796,13 @@ __global__ __launch_bounds__(512) void q1_few_kernel(Q1Segs sg, const uint4* __r
   for (int i = threadIdx.x; i < T * nsl * 32; i += 512) {
     const int e = i & 31, tj = i >> 5, t = tj / nsl, j = tj - t * nsl;
     const int L = lslab[t * nslabs + s0 + j];
+    uint4 v[kFewLimbs];                                          // requested with the limb count: absent limbs' rows are
+#pragma unroll                                                   // in the table too, whatever they hold
+    for (int l = 0; l < kFewLimbs; ++l)
+      v[l] = xq[(((int64_t)t * kMaxLimbs + l) * nbp + (s0 + j) * kSlabBlocks) * 8 + e];
 #pragma unroll
-    for (int l = 0; l < kFewLimbs; ++l) {
-      uint4 v = uint4{0, 0, 0, 0};
-      if (l < L) v = xq[(((int64_t)t * kMaxLimbs + l) * nbp + (s0 + j) * kSlabBlocks) * 8 + e];
-      sA[((t * spk + j) * kFewLimbs + l) * 32 + e] = v;
-    }
+    for (int l = 0; l < kFewLimbs; ++l)
+      sA[((t * spk + j) * kFewLimbs + l) * 32 + e] = l < L ? v[l] : uint4{0, 0, 0, 0};
     if (e < kSlabBlocks) stot[(t * spk + j) * kSlabBlocks + e] = totals[(int64_t)t * nbp + (s0 + j) * kSlabBlocks + e];
     if (e == 0) sL[t * spk + j] = L;
   }
@@ -2481,7 +2482,9 @@ static int q1_gemm_multi(const Q1Weight* const* ws, int cnt, const int64_t* x_de
 // (the 151,936-row head 35 us).
 constexpr int64_t kRowMaxTiles = 1024;
 // Two to kGemmMinT - 1 tokens (q1_few_kernel). Slab ranges as long as they leave 2048 waves (8 per CU), at most 8 slabs
-// and what LDS holds of the tokens' digits; two tiles per wave share the digit reads once that still leaves 1024 waves.
+// and what LDS holds of the tokens' digits; a wave takes two tiles, which share the digit reads, once one each would be
+// more than those 2048 waves (4 rows, 4096 / 4400 outputs of 4096, one tile against two: 10.7, 12.7 / 11.3, 11.3 us; 8
+// rows, 32768 / 34000 outputs: 38.0, 62.8 / 45.4, 45.2).
 static int q1_few_launch(const Q1Weight* const* ws, int cnt, const int64_t* x_dev, int64_t T, int64_t frac,
                          int64_t* const* outs, int accumulate, Q1Ws& wk, hipStream_t st, int prepped,
                          int64_t ntiles_all) {
@@ -2492,7 +2495,7 @@ static int q1_few_launch(const Q1Weight* const* ws, int cnt, const int64_t* x_de
     if (ntiles_all * ((nslabs + c - 1) / c) >= 2048 && T * c * (kFewLimbs * 512 + 36) <= kFewLds) { spk = c; break; }
   if (spk > nslabs) spk = nslabs;
   const int64_t ksplit = (nslabs + spk - 1) / spk;
-  const int R = ntiles_all * ksplit >= 2048 ? 2 : 1;
+  const int R = ntiles_all * ksplit > 2048 ? 2 : 1;
   Q1Segs sg = {};
   sg.cnt = cnt;
   int64_t groups = 0;
@@ -2520,10 +2523,12 @@ static int q1_few_launch(const Q1Weight* const* ws, int cnt, const int64_t* x_de
   }
   const size_t lds = (size_t)T * spk * (kFewLimbs * 32 * 16 + kSlabBlocks * 8 + 4) + 128;
   const int mode = ksplit > 1 ? 1 : (accumulate ? 2 : 0);
-  // workgroups of 8 groups; a long walk is cut into equal rounds over what the chip holds at once (two per CU)
+  // workgroups of 8 groups; a long walk runs on as many as the chip holds at once: one per CU (only R = 2 comes this far,
+  // and its 200 VGPRs leave two waves per SIMD). Cut into equal rounds of up to 512 (297 at the 151,936-row head), some
+  // CUs had two workgroups and the rest one: 62, 91, 151 us at 2, 4, 8 rows against 48, 68, 112.
   int64_t wgs = (groups + 7) / 8;
-  const int64_t fit = 512 / ksplit > 0 ? 512 / ksplit : 1;
-  if (wgs > fit) { const int64_t rounds = (wgs + fit - 1) / fit; wgs = (wgs + rounds - 1) / rounds; }
+  const int64_t fit = 256 / ksplit > 0 ? 256 / ksplit : 1;
+  if (wgs > fit) wgs = fit;
   const dim3 grid((unsigned)wgs, (unsigned)ksplit);
   const int fr = (int)(frac > 63 ? 63 : frac);
   imie_prof_mark(IMIE_K_Q1_GEMV, st, true);

@@ -31,6 +31,7 @@ def _case(seed, T, N, nb, wide):
     (1, 1, 1), (1, 16, 4), (1, 333, 11), (1, 4097, 32), (1, 40, 33), (1, 70, 128), (1, 48, 130),
     (2, 17, 1), (3, 333, 5), (4, 4096, 8), (5, 100, 33), (7, 64, 96), (8, 16, 9), (8, 2000, 32), (9, 33, 8),
     (3, 32784, 4),                                      # an odd number of tiles, two per wave
+    (2, 32768, 4), (2, 65552, 4), (5, 65552, 4),        # the last count of one tile per wave; the first beyond one round
 ])
 def test_few_rows(gpu, T, N, nb, wide):
     bits, scale, x = _case(T * 1000 + nb, T, N, nb, wide)
