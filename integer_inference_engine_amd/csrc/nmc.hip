@@ -1773,22 +1773,27 @@ int read_status_and(hipStream_t st, int* stat) {
   return IMIE_OK;
 }
 
-// Batched MoE: P = m*k pairs (token-major, pair p belongs to token p / k). Pairs sharing a weight run in one
-// item, so each expert's gate/up/down are read once per call. This form runs each projection as its own item list
-// (any quantisation types); moe_batched below takes the fused expert kernels when the layout allows.
-int moe_batched_items(const long long* gate_h, const long long* up_h, const long long* down_h, int m, int k,
-                      const int64_t* h_dev, const int64_t* gates_dev, int64_t d_model, int64_t e_ffn, int fa, int fw,
-                      int64_t* out_dev, hipStream_t st) {
-  const int64_t P = (int64_t)m * k;
-  if (m <= 0 || k <= 0 || d_model <= 0 || e_ffn <= 0 || d_model % 256 || e_ffn % 256 || fa < 1 || fa > 28 || fw < 0 ||
-      fw > 62)
-    return IMIE_EARG;
+// every pair's three weights exist with the shapes of the call; checked on each call, since a handle's number can come to
+// name another matrix (qk_free_all and new registrations)
+bool moe_shapes_ok(const long long* gate_h, const long long* up_h, const long long* down_h, int64_t P, int64_t d_model,
+                   int64_t e_ffn) {
   for (int64_t p = 0; p < P; ++p) {
     const QKWeight *g = qk_get(gate_h[p]), *u = qk_get(up_h[p]), *d = qk_get(down_h[p]);
     if (!g || !u || !d || g->out_f != e_ffn || g->nb * 256 != d_model || u->out_f != e_ffn || u->nb * 256 != d_model ||
         d->out_f != d_model || d->nb * 256 != e_ffn)
-      return IMIE_EARG;
+      return false;
   }
+  return true;
+}
+
+// Batched MoE: P = m*k pairs (token-major, pair p belongs to token p / k). Pairs sharing a weight run in one
+// item, so each expert's gate/up/down are read once per call. This form runs each projection as its own item list
+// (any quantisation types); moe_batched below, which has checked the arguments, takes the fused expert kernels when the
+// layout allows.
+int moe_batched_items(const long long* gate_h, const long long* up_h, const long long* down_h, int m, int k,
+                      const int64_t* h_dev, const int64_t* gates_dev, int64_t d_model, int64_t e_ffn, int fa, int fw,
+                      int64_t* out_dev, hipStream_t st) {
+  const int64_t P = (int64_t)m * k;
   if (g_mws.g.ensure((size_t)(P * e_ffn) * 8) || g_mws.u.ensure((size_t)(P * e_ffn) * 8) ||
       g_mws.d.ensure((size_t)(P * d_model) * 8) || g_mws.status.ensure(64))
     return IMIE_EARG;
@@ -1827,6 +1832,14 @@ int moe_batched_items(const long long* gate_h, const long long* up_h, const long
                      m, k, d_model, gates_dev, fa, out_dev, status);
   IMIE_HIP(hipGetLastError());
   return IMIE_OK;
+}
+
+// whether the fused kernels (Q4_K gate / up, Q6_K down) take the pairs
+bool moe_fused_ok(const long long* gate_h, const long long* up_h, const long long* down_h, int64_t P, int fw) {
+  bool fused = fw <= kMaxFw && qk_mfma_enabled();
+  for (int64_t p = 0; p < P && fused; ++p)
+    fused = qk_get(gate_h[p])->qtype == 0 && qk_get(up_h[p])->qtype == 0 && qk_get(down_h[p])->qtype == 1;
+  return fused;
 }
 
 // A few tokens take moe1_gateup_kernel / moe1_down_kernel (every pair reads its expert's weights, no item lists, two
@@ -1872,20 +1885,9 @@ int moe_batched(const long long* gate_h, const long long* up_h, const long long*
   if (m <= 0 || k <= 0 || d_model <= 0 || e_ffn <= 0 || d_model % 256 || e_ffn % 256 || fa < 1 || fa > 28 || fw < 0 ||
       fw > 62)
     return IMIE_EARG;
-  bool fused = fw <= kMaxFw && qk_mfma_enabled();
-  for (int64_t p = 0; p < P && fused; ++p) {
-    const QKWeight *g = qk_get(gate_h[p]), *u = qk_get(up_h[p]), *d = qk_get(down_h[p]);
-    if (!g || !u || !d) return IMIE_EARG;
-    fused = g->qtype == 0 && u->qtype == 0 && d->qtype == 1;
-  }
-  if (!fused)
+  if (!moe_shapes_ok(gate_h, up_h, down_h, P, d_model, e_ffn)) return IMIE_EARG;
+  if (!moe_fused_ok(gate_h, up_h, down_h, P, fw))
     return moe_batched_items(gate_h, up_h, down_h, m, k, h_dev, gates_dev, d_model, e_ffn, fa, fw, out_dev, st);
-  for (int64_t p = 0; p < P; ++p) {
-    const QKWeight *g = qk_get(gate_h[p]), *u = qk_get(up_h[p]), *d = qk_get(down_h[p]);
-    if (g->out_f != e_ffn || g->nb * 256 != d_model || u->out_f != e_ffn || u->nb * 256 != d_model ||
-        d->out_f != d_model || d->nb * 256 != e_ffn)
-      return IMIE_EARG;
-  }
   if (moe1_ok(m, k, d_model, e_ffn)) {
     if (g_mws.g.ensure((size_t)(P * e_ffn) * 8) || g_mws.status.ensure(64)) return IMIE_EARG;
     return moe1_launch(gate_h, up_h, down_h, m, k, h_dev, gates_dev, d_model, e_ffn, fa, fw, out_dev, nullptr, nullptr,
@@ -2098,14 +2100,8 @@ int imie_qk_moe_dev(const long long* gate_h, const long long* up_h, const long l
                     const int64_t* h_dev, const int64_t* gates_dev, int64_t d_model, int64_t e_ffn, int fa, int fw,
                     const int64_t* res, const int64_t* ao, int64_t* moe, int64_t* out_dev, int* status_dev,
                     hipStream_t st) {
-  bool small = fw <= kMaxFw && qk_mfma_enabled() && moe1_ok(1, k, d_model, e_ffn) && d_model % 256 == 0 &&
-               e_ffn % 256 == 0 && fa >= 1 && fa <= 28 && fw >= 0;
-  for (int p = 0; p < k && small; ++p) {
-    const QKWeight *g = qk_get(gate_h[p]), *u = qk_get(up_h[p]), *d = qk_get(down_h[p]);
-    if (!g || !u || !d) return IMIE_EARG;
-    small = g->qtype == 0 && u->qtype == 0 && d->qtype == 1;
-  }
-  if (small) {                                        // shapes are those of the layer (checked when it was bound)
+  if (!moe_shapes_ok(gate_h, up_h, down_h, k, d_model, e_ffn)) return IMIE_EARG;
+  if (moe_fused_ok(gate_h, up_h, down_h, k, fw) && moe1_ok(1, k, d_model, e_ffn) && fa >= 1 && fa <= 28 && fw >= 0) {
     if (g_mws.g.ensure((size_t)(k * e_ffn) * 8)) return IMIE_EARG;
     return moe1_launch(gate_h, up_h, down_h, 1, k, h_dev, gates_dev, d_model, e_ffn, fa, fw, out_dev, res, ao,
                        status_dev, st);

@@ -158,6 +158,36 @@ def test_bank_guard_poisons_layer(gpu):
     qk_gpu.free_all()
 
 
+@pytest.mark.parametrize("which", ["gate", "up", "down"])
+def test_bank_moe_refuses_rebound_handle_numbers(gpu, which):
+    """A bound expert's handle that has come to name a smaller matrix (all weights freed, others registered) is refused by
+    the continuation, as by every MoE call, and the layer is poisoned; nothing is read through it."""
+    from integer_inference_engine_amd import qk_gpu
+    W, hs, _, eh = _weights(27)
+    cos, sin = build_rope_tables(CAP, HD, base=50000, frac=FA)
+    bank = qk_gpu.ResidentAttentionCache(1, CAP, D, H, HKV, HD, FA, cos, sin)
+    bank.configure_moe_layer(0, E, USED, D, EFF)
+    for e in range(E):
+        bank.bind_moe_expert(0, e, *eh[e])
+    x = np.random.default_rng(28).integers(-(1 << 18), 1 << 18, size=(1, D), dtype=np.int64)
+    assert not bank.begin_moe_layer(0, hs["gain"], hs["router"], hs["wq"], hs["wk"], hs["wv"], hs["wo"], x, FW, 1, None,
+                                    True)
+    qk_gpu.free_all()
+    last = max(h for t in eh.values() for h in t)
+    shapes = {h: (D if k == 2 else EFF, k == 2) for t in eh.values() for k, h in enumerate(t)}
+    small = {t[("gate", "up", "down").index(which)] for t in eh.values()}
+    for h in range(last + 1):                           # the same numbers and kinds, one projection a row block short
+        rows, q6 = shapes.get(h, (64, False))
+        rows -= 64 if h in small else 0
+        assert qk_gpu.register_weight(qk.random_blocks(29, h, rows, 1, int(q6)), rows, 1, int(q6)) == h
+    with pytest.raises(qk_gpu.CudaContextError):
+        bank.continue_moe_layer(0, FW)
+    with pytest.raises(qk_gpu.CudaContextError):        # poisoned
+        bank.bind_moe_expert(0, 0, *eh[0])
+    bank.close()
+    qk_gpu.free_all()
+
+
 def test_token_executor_chains_layers_like_the_oracle(gpu):
     """ResidentMoeTokenExecutor (qk_cuda.py:738-868): two consecutive layers with one expert resident up front
     (lookup) and the rest loaded lazily on the device's cold report; result equals two oracle block steps. A bad
