@@ -1064,9 +1064,9 @@ __global__ __launch_bounds__(256, REP <= 4 ? 3 : 2) void dec_scores8_kernel(Attn
 // Decode PV (M == 1). Workgroup = (b, kv, chunk); per 64-key step the p digits of the REP heads are staged in LDS
 // as the A operand (row 4 (r % 4) + lp of head block r / 4); wave w owns dim tiles w and w + 4. RECOMP: e_j is
 // recomputed here from the score and the row maximum (dec_exp_kernel<REP, false> wrote no e); otherwise the
-// scores array holds e_j.
-template <int REP, bool RECOMP>
-__global__ __launch_bounds__(256, REP <= 4 ? 3 : 2) void dec_pv8_kernel(AttnDesc d) {
+// scores array holds e_j. WIDE: pages of more slots than a lane's 32-bit offset reaches (pv8_wide).
+template <int REP, bool RECOMP, bool WIDE = false>
+__global__ __launch_bounds__(256, REP <= 4 && !WIDE ? 3 : 2) void dec_pv8_kernel(AttnDesc d) {
   constexpr int RBH = (REP + 3) / 4;
   __shared__ __align__(16) int8_t sPd[RBH][16][64];
   __shared__ uint64_t s_z[REP], s_mp[4][REP];
@@ -1093,7 +1093,8 @@ __global__ __launch_bounds__(256, REP <= 4 ? 3 : 2) void dec_pv8_kernel(AttnDesc
   const bool pgreg = pi1 - pi0 < 64;
   const int64_t pgl = (pgreg && lane <= pi1 - pi0) ? d.pt[b * d.mp + pi0 + lane] : 0;
   const int64_t vplane = d.hd * d.P;                  // imie_kv8::v_off(slot, db, c) = db * vplane + c * P + slot
-  const uint32_t voff = (uint32_t)m * (uint32_t)d.P + 16u * (uint32_t)g;   // P < 2^27 (imie_attention_launch)
+  using VOff = std::conditional_t<WIDE, uint64_t, uint32_t>;
+  const VOff voff = (VOff)m * (VOff)d.P + 16u * (uint32_t)g;
   int64_t vtile[2];                                   // a tile past the head dim reads tile 0 (its MFMAs are skipped)
 #pragma unroll
   for (int tt = 0; tt < 2; ++tt) vtile[tt] = wave + 4 * tt < DT ? 16 * (wave + 4 * tt) * d.P : 0;
@@ -2430,6 +2431,10 @@ void imie_attn_qdigit_scratch(const AttnDesc& d, int8_t** qd, int** qlimbs) {
   *qlimbs = (int*)(*qd + rows * 8 * d.hd);
 }
 
+// whether dec_pv8_kernel's largest lane offset (dim 15 of a tile, 16-slot piece 3) leaves 32 bits; 64-bit offsets cost
+// that kernel registers (two waves per SIMD), so only such pages, of 286 million slots, take them
+static bool pv8_wide(const AttnDesc& d) { return 15 * d.P + 48 > (int64_t)UINT32_MAX; }
+
 static void pf_fused8_launch(const AttnDesc& d, hipStream_t st) {
   const int64_t npt = (d.M + kFfRows - 1) / kFfRows;
   if (d.hd == 128) {
@@ -2476,7 +2481,7 @@ int imie_attention_launch(AttnDesc d, hipStream_t st) {
     IMIE_HIP(hipGetLastError());
     // kv8 with several sequences: PV recomputes e from the scores (no write-back of e, the bytes a big batch is
     // bound by); one sequence: e is written back, which keeps the exponentials off PV's per-step latency chain
-    const bool recomp = d.kv32 && d.B > 1;
+    const bool wide = d.kv32 && pv8_wide(d), recomp = d.kv32 && d.B > 1 && !wide;
     if (recomp) {
       if (rep == 1) hipLaunchKernelGGL((dec_exp_kernel<1, false>), gd, dim3(256), 0, st, d);
       else if (rep == 2) hipLaunchKernelGGL((dec_exp_kernel<2, false>), gd, dim3(256), 0, st, d);
@@ -2494,6 +2499,11 @@ int imie_attention_launch(AttnDesc d, hipStream_t st) {
       else if (rep == 2) hipLaunchKernelGGL((dec_pv8_kernel<2, true>), gd, dim3(256), 0, st, d);
       else if (rep == 4) hipLaunchKernelGGL((dec_pv8_kernel<4, true>), gd, dim3(256), 0, st, d);
       else hipLaunchKernelGGL((dec_pv8_kernel<8, true>), gd, dim3(256), 0, st, d);
+    } else if (wide) {
+      if (rep == 1) hipLaunchKernelGGL((dec_pv8_kernel<1, false, true>), gd, dim3(256), 0, st, d);
+      else if (rep == 2) hipLaunchKernelGGL((dec_pv8_kernel<2, false, true>), gd, dim3(256), 0, st, d);
+      else if (rep == 4) hipLaunchKernelGGL((dec_pv8_kernel<4, false, true>), gd, dim3(256), 0, st, d);
+      else hipLaunchKernelGGL((dec_pv8_kernel<8, false, true>), gd, dim3(256), 0, st, d);
     } else if (d.kv32) {
       if (rep == 1) hipLaunchKernelGGL((dec_pv8_kernel<1, false>), gd, dim3(256), 0, st, d);
       else if (rep == 2) hipLaunchKernelGGL((dec_pv8_kernel<2, false>), gd, dim3(256), 0, st, d);
@@ -2512,13 +2522,16 @@ int imie_attention_launch(AttnDesc d, hipStream_t st) {
     return IMIE_OK;
   }
   if (d.kv32) {                                      // kv8 prefill: MFMA scores, softmax to p digits, MFMA PV
-    if (d.hd % 16 != 0 || !d.run_k || !d.run_v || d.P >= ((int64_t)1 << 27)) return IMIE_EARG;
-    if (d.hd <= 128 && pf_fused()) {
+    if (d.hd % 16 != 0 || !d.run_k || !d.run_v) return IMIE_EARG;
+    // the fused kernel addresses a page's block by 32-bit offsets; the separate kernels, for larger pages, by 64-bit ones.
+    // Those have no scratch for one row (a head layout that the decode kernels above do not take): refused.
+    if (d.hd <= 128 && 4 * d.hd * d.P <= (int64_t)UINT32_MAX && pf_fused()) {
       pf_fused8_launch(d, st);
       IMIE_HIP(hipGetLastError());
       imie_prof_mark(IMIE_K_ATTN, st, false);
       return IMIE_OK;
     }
+    if (d.M == 1) return IMIE_EARG;
     const int64_t nrt16 = (grows + 15) / 16, nkt8 = (d.Lmax + kPfKeys - 1) / kPfKeys;
     const int64_t nkg = (nkt8 + kPfTilesPerWg - 1) / kPfTilesPerWg;
     hipLaunchKernelGGL(pf_scores8_kernel, dim3((unsigned)(d.B * d.Hkv * nrt16), (unsigned)nkg), dim3(256), 0, st, d);
