@@ -222,6 +222,20 @@ Kept& kept() {
   static Kept k;
   return k;
 }
+// the pinned export buffer at `bytes` or more; false where there is no such memory (the export then takes the pageable way)
+bool kept_pin(size_t bytes) {
+  Kept& k = kept();
+  if (k.pin_cap >= bytes) return true;
+  if (k.pin) (void)hipHostFree(k.pin);
+  k.pin_cap = 0;
+  if (hipHostMalloc((void**)&k.pin, bytes) != hipSuccess) {
+    (void)hipGetLastError();                           // no launch is to report it
+    k.pin = nullptr;
+    return false;
+  }
+  k.pin_cap = bytes;
+  return true;
+}
 void kept_take(Net& n) {
   const NetBufs nb = net_bufs(n);
   for (int i = 0; i < kNetBufs; ++i) std::swap(*nb.b[i], kept().ws[i]);
@@ -692,14 +706,8 @@ int bonsai_prefill_forward_gpu(const int64_t* x_embed, int64_t T, int64_t d, int
     // to pinned memory behind the forward; the caller's arrays (usually fresh, so unmapped) are faulted in meanwhile,
     // unchanged, and filled once the call is known to be good.
     const size_t half = (size_t)n_layers * (size_t)(Hkv * T * hd) * 8;
-    const bool exp = out_k && out_v, pinned = exp && 2 * half <= kKeepPinned;
+    const bool exp = out_k && out_v, pinned = exp && 2 * half <= kKeepPinned && kept_pin(2 * half);
     if (pinned) {
-      if (kept().pin_cap < 2 * half) {
-        if (kept().pin) (void)hipHostFree(kept().pin);
-        kept().pin_cap = 0;
-        if (hipHostMalloc((void**)&kept().pin, 2 * half) != hipSuccess) { kept().pin = nullptr; rc = IMIE_EARG; break; }
-        kept().pin_cap = 2 * half;
-      }
       if (hipMemcpyAsync(kept().pin, n.kpool[0], 2 * half, hipMemcpyDeviceToHost, st) != hipSuccess) { rc = IMIE_EARG; break; }
       for (int64_t* a : {out_k, out_v})
         for (size_t o = 0; o < half; o += 4096) {
