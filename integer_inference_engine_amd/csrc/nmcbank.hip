@@ -685,6 +685,24 @@ int status_ensure(Bank& b, size_t bytes) {
   if (b.status.cap < bytes) b.status_clear = false;
   return b.status.ensure(bytes);
 }
+size_t published_bytes(const Bank& b, int n_ids, bool row) {
+  return (kIdsAt + (size_t)n_ids * 4 + 7) / 8 * 8 + (row ? (size_t)b.d_model * 8 : 0);
+}
+// The pinned buffer for n_ids ids and a row, reserved before any work is enqueued; where there is no pinned memory,
+// finish() reads back through pageable memory.
+void host_reserve(Bank& b, int n_ids) {
+  const size_t bytes = published_bytes(b, n_ids, true);
+  if (b.host_cap >= bytes) return;
+  if (b.host) (void)hipHostFree(b.host);
+  b.host = nullptr;
+  b.host_cap = 0;
+  if (hipHostMalloc((void**)&b.host, bytes) == hipSuccess) {
+    b.host_cap = bytes;
+  } else {
+    b.host = nullptr;
+    (void)hipGetLastError();                           // no launch is to report it
+  }
+}
 // validate the attention handles / window and reserve the layer's storage (qk_cuda.py:548-572 envelope)
 int attention_preflight(Bank& b, int layer, long long qh, long long kh, long long vh, long long oh, int window) {
   if (layer < 0 || layer >= b.n_layers || window == 0 || window < -1) return IMIE_EARG;
@@ -697,6 +715,7 @@ int attention_preflight(Bank& b, int layer, long long qh, long long kh, long lon
   if (nb[0] * 256 != b.d_model || nb[1] * 256 != b.d_model || nb[2] * 256 != b.d_model || of[0] != qw ||
       of[1] != kw || of[2] != kw || nb[3] * 256 != qw || of[3] != b.d_model)
     return IMIE_EARG;
+  host_reserve(b, L.used);
   if (ensure_layer_kv(b, L) || b.qkv.ensure((size_t)(qw + 2 * kw) * 8) || b.attn.ensure((size_t)qw * 8) ||
       b.ao.ensure((size_t)b.d_model * 8) || b.prob.ensure((size_t)(b.heads * b.max_len) * 8) ||
       b.part.ensure((size_t)(kNbMaxChunks * (qw + 2 * b.heads)) * 8) || status_ensure(b, kIdsAt))
@@ -757,27 +776,33 @@ int status_begin(Bank& b, hipStream_t st) {
 // and a hidden row (d_model words of `row`, to `row_out`) come back with it
 int finish(Bank& b, Layer& L, hipStream_t st, int n_ids = 0, int* ids = nullptr, const int64_t* row = nullptr,
            int64_t* row_out = nullptr) {
-  const size_t head = (kIdsAt + (size_t)n_ids * 4 + 7) / 8 * 8, bytes = head + (row ? (size_t)b.d_model * 8 : 0);
+  const size_t head = published_bytes(b, n_ids, false), bytes = published_bytes(b, n_ids, row != nullptr);
   auto fail = [&]() -> int { L.poisoned = true; return IMIE_EARG; };
-  if (b.host_cap < bytes) {
-    if (b.host) (void)hipHostFree(b.host);
-    b.host = nullptr;
-    b.host_cap = 0;
-    if (hipHostMalloc((void**)&b.host, bytes) != hipSuccess) { (void)hipStreamSynchronize(st); return fail(); }
-    b.host_cap = bytes;
+  std::vector<char> page;
+  const char* src = b.host;
+  if (b.host_cap >= bytes) {
+    hipLaunchKernelGGL(nb_publish_kernel, dim3(1), dim3(256), 0, st, (const uint64_t*)b.status.p, (int)(head / 8),
+                       (uint64_t*)b.host);
+    if (row)
+      hipLaunchKernelGGL(nb_publish_kernel, dim3((unsigned)((b.d_model + 255) / 256)), dim3(256), 0, st,
+                         (const uint64_t*)row, (int)b.d_model, (uint64_t*)(b.host + head));
+    if (hipGetLastError() != hipSuccess || hipStreamSynchronize(st) != hipSuccess) return fail();
+  } else {
+    page.resize(bytes);
+    src = page.data();
+    if (hipMemcpyAsync(page.data(), b.status.p, head, hipMemcpyDeviceToHost, st) != hipSuccess ||
+        (row && hipMemcpyAsync(page.data() + head, row, bytes - head, hipMemcpyDeviceToHost, st) != hipSuccess) ||
+        hipStreamSynchronize(st) != hipSuccess) {
+      (void)hipStreamSynchronize(st);
+      return fail();
+    }
   }
-  hipLaunchKernelGGL(nb_publish_kernel, dim3(1), dim3(256), 0, st, (const uint64_t*)b.status.p, (int)(head / 8),
-                     (uint64_t*)b.host);
-  if (row)
-    hipLaunchKernelGGL(nb_publish_kernel, dim3((unsigned)((b.d_model + 255) / 256)), dim3(256), 0, st,
-                       (const uint64_t*)row, (int)b.d_model, (uint64_t*)(b.host + head));
-  if (hipGetLastError() != hipSuccess || hipStreamSynchronize(st) != hipSuccess) return fail();
   int stat = 0;
-  memcpy(&stat, b.host, 4);
+  memcpy(&stat, src, 4);
   if (stat) { L.poisoned = true; return 3; }
   b.status_clear = true;
-  if (n_ids) memcpy(ids, b.host + kIdsAt, (size_t)n_ids * 4);
-  if (row) memcpy(row_out, b.host + head, (size_t)b.d_model * 8);
+  if (n_ids) memcpy(ids, src + kIdsAt, (size_t)n_ids * 4);
+  if (row) memcpy(row_out, src + head, (size_t)b.d_model * 8);
   return IMIE_OK;
 }
 

@@ -33,6 +33,36 @@ def prefill(gpu, shim):
         shim.arm(1)                                     # the second, larger call finds no pinned memory
 
 
+def bank(gpu, shim):
+    import numpy as np
+    from integer_inference_engine_amd import qk_gpu
+    from oracle import fixedpoint as fx, nmc_block as onb, qk
+    from oracle.rope import apply_interleaved, build_rope_tables
+    from tests import test_gpu_nmc_bank as t
+    W, hs, experts, eh = t._weights(41)
+    cos, sin = build_rope_tables(t.CAP, t.HD, base=50000, frac=t.FA)
+    for armed in (0, 1):
+        shim.arm(armed)
+        cache = qk_gpu.ResidentAttentionCache(1, t.CAP, t.D, t.H, t.HKV, t.HD, t.FA, cos, sin)
+        cache.configure_moe_layer(0, t.E, t.USED, t.D, t.EFF)
+        for e in range(t.E):
+            cache.bind_moe_expert(0, e, *eh[e])
+        kc, vc = (np.zeros((t.HKV, t.CAP, t.HD), dtype=np.int64) for _ in range(2))
+        x = np.random.default_rng(42).integers(-(1 << 18), 1 << 18, size=(1, t.D), dtype=np.int64)
+        want, _, _, _, kc[:, 0], vc[:, 0] = onb.block_step(x, W, kc, vc, 0, None, True, cos, sin, t.CFG, experts)
+        assert not cache.begin_moe_layer(0, hs["gain"], hs["router"], hs["wq"], hs["wk"], hs["wv"], hs["wo"], x, t.FW, 1,
+                                         None, True)
+        assert np.array_equal(cache.continue_moe_layer(0, t.FW, publish=True), want)
+        got = cache.apply(0, hs["wq"], hs["wk"], hs["wv"], hs["wo"], x, t.FW, None, True)
+        q, k, v = (qk.linear(x, W[n], t.FW).reshape(-1, t.HD) for n in ("wq", "wk", "wv"))
+        q, k = (apply_interleaved(a[:, None, :], cos[1:2], sin[1:2], t.FA)[:, 0, :] for a in (q, k))
+        kc[:, 1], vc[:, 1] = k, v
+        att = onb.attention_step(q, kc, vc, 1, None, t.FA, fx.inv_sqrt_fp(t.HD, t.FA)).reshape(1, t.H * t.HD)
+        assert np.array_equal(got, qk.linear(att, W["wo"], t.FW))
+        cache.close()
+        print("bank", armed, "ok", flush=True)
+
+
 def main():
     shim = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)      # before the HIP runtime: its symbol comes first
     from integer_inference_engine_amd import gpu_native as gpu

@@ -23,7 +23,7 @@ int hipHostMalloc(void** p, size_t n, unsigned flags) {
 """
 
 
-@pytest.mark.parametrize("call", ["prefill"])
+@pytest.mark.parametrize("call", ["prefill", "bank"])
 def test_no_pinned_memory(gpu, tmp_path, call):
     (tmp_path / "shim.c").write_text(SHIM)
     so = tmp_path / "shim.so"
