@@ -136,6 +136,8 @@ int imie_attention_scores_probe(const int64_t *q, const int64_t *k, int64_t H, i
 int64_t bonsai_buf_upload_i64(const int64_t *host, int64_t n);
 const int64_t *imie_buf_device_ptr(int64_t handle);
 void imie_buf_free_all(void);
+/* Gives back what whole prefills keep between calls (at most 2 GiB of device and 256 MiB of pinned memory). */
+void imie_prefill_release(void);
 /* bonsai_q1_gpu.cu:3694-3819 `bonsai_prefill_forward_gpu` (gpu_native.py:161-172, 559-595). */
 int bonsai_prefill_forward_gpu(const int64_t *x_embed, int64_t T, int64_t d, int64_t n_layers, int64_t H, int64_t Hkv,
                                int64_t hd, int64_t dff, int64_t frac, int64_t eps, int64_t inv_sqrt,

@@ -79,6 +79,7 @@ SIGNATURES = {
     "bonsai_buf_upload_i64": (c_int64, [c_void_p, c_int64]),
     "imie_buf_device_ptr": (c_void_p, [c_int64]),
     "imie_buf_free_all": (None, []),
+    "imie_prefill_release": (None, []),
     "bonsai_prefill_forward_gpu": (c_int, [c_void_p] + [c_int64] * 10 + [c_void_p] * 11 + [c_int64] * 4
                                    + [c_void_p] * 3),
     "bonsai_decode_ctx_create": (c_int64, [c_int64] * 12 + [c_void_p] * 11 + [c_int64] * 4),

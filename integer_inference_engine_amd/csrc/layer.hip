@@ -204,7 +204,7 @@ NetBufs net_bufs(Net& n) {
 // What whole prefills (bonsai_prefill_forward_gpu) keep between calls: the workspaces, the cache's memory and a pinned
 // buffer for its export, handed to one call at a time under the library lock and idle when it returns (the call
 // synchronizes). Allocating and freeing some fifty buffers a call and exporting through pageable memory was half of a
-// 256-row, 12-layer call. Only sizes within the bounds stay; imie_buf_free_all gives them back.
+// 256-row, 12-layer call. Only sizes within the bounds stay; imie_prefill_release and imie_buf_free_all give them back.
 constexpr size_t kKeepDevice = (size_t)2 << 30, kKeepPinned = (size_t)256 << 20;
 struct Kept {
   DevBuf ws[kNetBufs], arena;
@@ -673,6 +673,13 @@ void imie_buf_free_all(void) {
   (void)hipStreamSynchronize(imie_stream());
   for (auto& e : bufs()) if (e.p) imie_free(e.p);
   bufs().clear();
+  kept().give_back();
+}
+
+// What whole prefills keep between calls goes back to the system; uploaded buffers and weights stay.
+void imie_prefill_release(void) {
+  std::lock_guard<std::recursive_mutex> lk(imie_lock());
+  (void)hipStreamSynchronize(imie_stream());
   kept().give_back();
 }
 

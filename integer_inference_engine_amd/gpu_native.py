@@ -321,6 +321,13 @@ def prefill_forward_gpu(x_embed, dims, w, g, frac, eps, inv_sqrt_fp, *, export_k
     return (out, k_arr, v_arr) if export_kv else out
 
 
+def release_prefill_workspace():
+    """Give back the memory that ``prefill_forward_gpu`` keeps between calls (weights and buffers stay)."""
+    lib = _dev()
+    if lib is not None:
+        lib.imie_prefill_release()
+
+
 def decode_ctx_create(dims, w, g, frac, eps, inv_sqrt_fp, cap):
     """Device decode context (gpu_native.py:483-506). dims = (B, n_layers, H, Hkv, hd, d, dff, vocab)."""
     lib = _dev()
