@@ -1845,10 +1845,18 @@ bool moe_fused_ok(const long long* gate_h, const long long* up_h, const long lon
 // A few tokens take moe1_gateup_kernel / moe1_down_kernel (every pair reads its expert's weights, no item lists, two
 // launches); more tokens share decoded weights in the grouped kernels below. At 128 experts of 768, top-8, hidden 2048,
 // this form against the grouped one for 1, 2, 3, 4 tokens: 23.5 / 41.3, 39 / 44.5, 57.5 / 58.6, 72 / 65 us.
+// Two tokens only while their pairs' weights are few, since this form reads and decodes an expert for each of them; beyond
+// eight experts a down workgroup needs two rounds of jobs, which count twice. Two tokens, d x e x experts a token (million
+// weights), this form against the grouped one: 2048 x 768 x 8 (75) 38.4 / 44.8 us, 8192 x 1024 x 2 (101) 67 / 73, 4096 x
+// 512 x 8 (101) 52.6 / 53.2, 4096 x 1536 x 4 (151) 64 / 57, 7168 x 2048 x 2 (176) 86 / 68, 4096 x 1024 x 8 (201) 71 / 64;
+// 2048 x 256 x 16 (50) 42 / 45, 2048 x 512 x 16 (101) 52 / 45. One token is faster up to 201 (8192 x 4096 x 2: 77 / 84).
 constexpr int kMoe1Tokens = 2;
+constexpr int64_t kMoe1Weights = (int64_t)96 << 20;
 bool moe1_ok(int64_t m, int64_t k, int64_t d_model, int64_t e_ffn) {
+  const int64_t rounds = (kMoe1Out / kMoe1Rows * k + 31) / 32;
   return m <= kMoe1Tokens && k <= kMoe1MaxK && m * k <= kMoe1Pairs && d_model / 256 <= kG1MaxNb &&
-         k * (e_ffn / 256) <= kG1MaxNb && d_model % kMoe1Out == 0;
+         k * (e_ffn / 256) <= kG1MaxNb && d_model % kMoe1Out == 0 &&
+         (m == 1 || m * k * 3 * d_model * e_ffn * rounds <= kMoe1Weights);
 }
 
 // handles already checked by the caller; res, ao: the residual and attention rows to add (both or none)

@@ -78,3 +78,25 @@ def test_moe_few_tokens(gpu, m, k, d, ffn, kind):
     want = qk.moe_ffn(h, sel, gates, experts, fa, FW)
     assert got is not None and np.array_equal(got, want)
     qk_gpu.free_all()
+
+
+@pytest.mark.parametrize("k,d,ffn", [(2, 8192, 1024), (2, 8192, 1280), (16, 2048, 256), (16, 2048, 512)])
+def test_moe_two_tokens_as_one_each(gpu, k, d, ffn):
+    """Two tokens at and beyond the weight volume where the grouped kernels take over, against one token each (the small
+    form, held to the oracle above): the same bits."""
+    from integer_inference_engine_amd import qk_gpu
+    rng = np.random.default_rng(d + ffn)
+    handles = [[qk_gpu.register_weight(qk.random_blocks(11, 3 * e + i, o, n // 256, t), o, n // 256, t)
+                for i, (o, n, t) in enumerate(((ffn, d, 0), (ffn, d, 0), (d, ffn, 1)))] for e in range(k + 1)]
+    h = rng.integers(-(1 << 12), 1 << 12, size=(2, d), dtype=np.int64)
+    sel = np.stack([rng.permutation(k + 1)[:k] for _ in range(2)])
+    gates = rng.integers(1, 1 << 16, size=(2, k), dtype=np.int64)
+
+    def call(tokens):
+        flat = sel[tokens].reshape(-1)
+        return qk_gpu.moe_ffn_batched(*([handles[e][i] for e in flat] for i in range(3)), len(tokens), k, h[tokens],
+                                      gates[tokens], d, ffn, 16, FW)
+
+    got, one = call([0, 1]), [call([t]) for t in range(2)]
+    assert got is not None and np.array_equal(got, np.concatenate(one)) and got.any()
+    qk_gpu.free_all()
