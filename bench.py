@@ -175,10 +175,11 @@ def decode_leg(so, torch, tokens: int, ctx: int = 4096, n_layers: int = 36, voca
     so.imie_profile_end()
     status = int(so.imie_net_status(net.h, 0, sp))
     last = int(ids.item())
+    planes = int(net.kv_planes().sum())            # over layers, K and V, kv heads
     net.close()
     c5 = c5_leg(so, torch, w, g, ebits, escale, c5_tokens) if c5_tokens > 0 else None
     wbytes = sum(o * (i // 128) * (16 + 4) for o, i in shapes.values()) * n_layers + vocab * (d // 128) * 20
-    kvbytes = n_layers * 2 * Hkv * ctx * hd * 3   # planes read: values below 2^23 leave the fourth empty, unread
+    kvbytes = planes * ctx * hd                    # the planes that are read, a byte an element each
     return {"tok_s": round(tokens / (ms / 1e3), 2), "ms_per_token": round(ms / tokens, 3),
             "host_enqueue_ms_per_token": round(t_host * 1e3 / tokens, 3), "eager_ms_per_token": round(ms_eager, 3),
             "mode": "HIP graph of one greedy step (embed, 36 layers, head, argmax), replayed", "tokens": tokens,
@@ -240,12 +241,13 @@ def c5_leg(so, torch, w, g, ebits, escale, tokens: int, B: int = 32, n_layers: i
     net.stream.synchronize()
     ms_s = e0.elapsed_time(e1)
     status |= net.status()
+    kv_read = int((net.kv_planes().sum(axis=(0, 1, 3)) * (lens + 2)).sum()) * hd   # the digit planes that are read
     net.close()
     kv_bytes = int((lens + 2).sum()) * n_layers * 2 * Hkv * hd * 4
     return {"sequences": B, "tokens_per_sequence": tokens, "layers": n_layers,
             "context_min": int(lens.min()), "context_max": int(lens.max()), "context_mean": round(float(lens.mean()), 1),
             "tok_s": round(B * tokens / (ms / 1e3), 1), "ms_per_step": round(ms / tokens, 3), "status": status,
-            "kv_GB": round(kv_bytes / 1e9, 1), "kv_read_GB_s": round(0.75 * kv_bytes / (ms / tokens / 1e3) / 1e9, 1),   # three of the four planes, as above
+            "kv_GB": round(kv_bytes / 1e9, 1), "kv_read_GB_s": round(kv_read / (ms / tokens / 1e3) / 1e9, 1),
             "setup_s": round(setup_s, 2), "kv": "kv8 digit planes (int8 x 4 per element), 64-slot pages",
             "sampled_tok_s": round(B * ns / (ms_s / 1e3), 1), "sampled_ms_per_step": round(ms_s / ns, 3),
             "sampled_mode": "top_p, qwen3-rec (T 0.6, top-k 20, top-p 0.95), device SHA-256 draws"}

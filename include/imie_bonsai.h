@@ -169,6 +169,9 @@ int imie_net_forward_dev(int64_t ctx, int64_t *x_dev, const int64_t *starts, int
 int imie_net_head_dev(int64_t ctx, const int64_t *x_dev, int64_t rows, int64_t *logits_dev, int64_t *ids_dev,
                       void *stream);
 int imie_net_status(int64_t ctx, int clear, void *stream);
+/* Digit planes (3 or 4) that attention reads of a kv8 cache, out [layers][2][B * Hkv] (K, V) on the host; rc 1 for an
+ * int64 cache. */
+int imie_net_kv_planes(int64_t ctx, int *out);
 int imie_net_export_kv(int64_t ctx, int64_t layer, int64_t b, int64_t count, int64_t *k_out, int64_t *v_out);
 /* Greedy decode of `steps` tokens on the device: embed -> all layers -> final norm + LM head -> lowest-index
  * argmax, per step (the host-driven loop of reference_bonsai.py:1200-1310 moved onto the GPU; no single

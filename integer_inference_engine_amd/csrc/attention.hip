@@ -759,7 +759,7 @@ __global__ __launch_bounds__(256) void dec_final_kernel(AttnDesc d) {
 // MFMA int32 sums are exact (|D| <= 64 * 128 * 128 per MFMA; partial sums bounded below 2^31 as noted); every
 // recombination into the int64 result wraps mod 2^64 like the oracle's int64 arithmetic.
 // max|K| / max|V| for the fail-loud bounds are the running maxima kept by the cache writes (run_k / run_v). They also
-// say how many digit planes can be nonzero: a cache whose maximum fits three balanced digits (kCap3: every one of an
+// say how many digit planes can be nonzero: a cache whose maximum fits three balanced digits (imie_kv8::kCap3: every one of an
 // 8B model's, whose normalised keys stay below 2^21) has a zero top plane, which is then neither read nor multiplied --
 // a quarter of the cache's bytes and of the MFMAs. Maxima that a reset clears go on counting in old_k / old_v: slots
 // of an earlier sequence keep their fourth plane for whoever starts behind them. The choice is made per workgroup, as two
@@ -767,7 +767,6 @@ __global__ __launch_bounds__(256) void dec_final_kernel(AttnDesc d) {
 // bound by the cache's bytes, prefill by MFMA issue; 32 sequences of 512 to 16000 positions: scores 232 -> 183 us, PV
 // 214 -> 170 us a layer; prefill of 2048 rows 362 + 255 -> 326 + 240 us, of 333 rows behind 5000 264 + 194 -> 226 + 167.
 // ---------------------------------------------------------------------------------------------------------
-constexpr uint64_t kCap3 = 127ull * ((256ull * 256 * 256 - 1) / 255);
 // digit planes of a cache with the running maximum `run` and the retired one `old` (nullptr: all four); wave-uniform,
 // by scalar loads (their own counter: no wait for the vector loads in flight)
 __device__ inline uint64_t sload_u64(const uint64_t* p) {
@@ -779,7 +778,7 @@ __device__ inline uint64_t sload_u64(const uint64_t* p) {
 __device__ inline int kv8_planes(const uint64_t* run, const uint64_t* old, int64_t bkv) {
   if (!run || !old) return 4;
   const uint64_t a = sload_u64(run + bkv), c = sload_u64(old + bkv);
-  return a <= kCap3 && c <= kCap3 ? 3 : 4;
+  return a <= imie_kv8::kCap3 && c <= imie_kv8::kCap3 ? 3 : 4;
 }
 
 __device__ inline int64_t bal_digit(int64_t x, int l) {

@@ -15,6 +15,9 @@ namespace imie_kv8 {
 
 constexpr int64_t kCap = 2139062143;
 
+// the largest |v| of three digits: a cache with this maximum has a zero top plane
+constexpr uint64_t kCap3 = 127ull * ((256ull * 256 * 256 - 1) / 255);
+
 __host__ __device__ inline bool fits(int64_t v) { return v >= -kCap && v <= kCap; }
 
 // balanced digits of v (|v| <= kCap), packed little-endian into a 32-bit word

@@ -1127,6 +1127,20 @@ int imie_net_status(int64_t ctx, int clear, void* stream) {
   return stat;
 }
 
+// Digit planes, 3 or 4, that attention reads of every layer, K or V, sequence and kv head of a kv8 cache, by their running
+// maxima: out [layers][2][B * Hkv] on the host. Synchronous.
+int imie_net_kv_planes(int64_t ctx, int* out) {
+  std::lock_guard<std::recursive_mutex> lk(imie_lock());
+  Net* n = net_get(ctx);
+  if (!n || !out || !n->kv32 || !n->kvrun.p) return IMIE_EARG;
+  IMIE_HIP(hipDeviceSynchronize());
+  const size_t nr = (size_t)(n->nl * 2 * n->B * n->Hkv);
+  std::vector<uint64_t> m(2 * nr);                     // running, then retired maxima
+  IMIE_HIP(hipMemcpy(m.data(), n->kvrun.p, 2 * nr * 8, hipMemcpyDeviceToHost));
+  for (size_t i = 0; i < nr; ++i) out[i] = std::max(m[i], m[nr + i]) <= imie_kv8::kCap3 ? 3 : 4;
+  return IMIE_OK;
+}
+
 // Copy sequence b's cached K/V of `layer` for positions [0, count) to host (Hkv, count, hd) int64.
 int imie_net_export_kv(int64_t ctx, int64_t layer, int64_t b, int64_t count, int64_t* k_out, int64_t* v_out) {
   std::lock_guard<std::recursive_mutex> lk(imie_lock());

@@ -141,6 +141,14 @@ class ResidentNet:
     def clear_status(self) -> None:
         self.lib.imie_net_status(self.h, 1, self._sp())
 
+    def kv_planes(self) -> np.ndarray:
+        """Digit planes (3 or 4) that attention reads of a kv8 cache: (n_layers, 2 for K and V, B, Hkv)."""
+        out = np.empty((self.nl, 2, self.B, self.Hkv), dtype=np.int32)
+        rc = self.lib.imie_net_kv_planes(self.h, out.ctypes.data)
+        if rc != 0:
+            raise RuntimeError(f"kv_planes rc={rc}: {_lib.last_error()}")
+        return out
+
     def export_kv(self, layer: int, b: int, count: int):
         k = np.empty((self.Hkv, count, self.hd), dtype=np.int64)
         v = np.empty_like(k)

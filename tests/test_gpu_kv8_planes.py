@@ -35,6 +35,11 @@ def _cache(seed, tag, cfg, n, edges):
     return out
 
 
+def _planes(seqs):
+    """seqs: per sequence the (n_layers, Hkv, n, hd) values; planes by their maxima, (n_layers, B, Hkv)."""
+    return np.stack([np.where(np.abs(s).max(axis=(2, 3)) <= CAP3, 3, 4) for s in seqs], axis=1)
+
+
 def _check(net, model, c, ks, vs, starts, M, seed):
     import torch
     xs = [q1_rows(*model["embed"], prng.uniform_int(seed, 20 + b, (M,), 0, 64)) for b in range(len(starts))]
@@ -67,6 +72,8 @@ def test_kv8_planes_by_maximum(gpu, layout, M):
     try:
         for b in range(3):
             net.seed(b, ks[b], vs[b])
+        got = net.kv_planes()
+        assert np.array_equal(got[:, 0], _planes(ks)) and np.array_equal(got[:, 1], _planes(vs))
         _check(net, model, c, ks, vs, starts, M, seed)
     finally:
         net.close()
@@ -90,6 +97,7 @@ def test_kv8_planes_behind_a_reset(gpu, M):
         net.seed(0, ks, vs)
         net.reset()
         net.reset()
+        assert (net.kv_planes() == 4).all()            # some value of every cached head lay beyond three digits
         _check(net, model, {"H": H, "Hkv": Hkv, "hd": hd}, [ks], [vs], [100], M, seed)
     finally:
         net.close()
