@@ -325,8 +325,6 @@ __global__ void attn_init_kernel(AttnDesc d) {
 //               (32 lanes x 4 dims); chunk PV sums -> part[chunk][row][dim], chunk max|p| / max|V| -> cmp / cvm
 //   D4 final  : out = (sum over chunks of part) >> f, plus the bound checks from the chunk maxima
 // ---------------------------------------------------------------------------------------------------------
-constexpr int kMaxRep = 8;
-
 __device__ inline int64_t page_off(const AttnDesc& d, int64_t b, int64_t kv, int64_t j) {
   int64_t pi, in;
   page_split(d, j, pi, in);
@@ -787,15 +785,6 @@ __device__ inline int64_t bal_digit(int64_t x, int l) {
     x = (int64_t)((uint64_t)x - (uint64_t)dg) >> 8;
   }
   return ((x + 128) & 255) - 128;
-}
-
-__device__ inline v4i pack16(const int8_t* v) {
-  v4i r;
-#pragma unroll
-  for (int k = 0; k < 4; ++k)
-    r[k] = (int)((uint32_t)(uint8_t)v[4 * k] | ((uint32_t)(uint8_t)v[4 * k + 1] << 8) |
-                 ((uint32_t)(uint8_t)v[4 * k + 2] << 16) | ((uint32_t)(uint8_t)v[4 * k + 3] << 24));
-  return r;
 }
 
 __device__ inline v4i mfma8(v4i a, v4i b, v4i c) { return __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, c, 0, 0, 0); }

@@ -52,26 +52,10 @@ struct MoeWs {
   int64_t grows = 0;
 } g_mws;
 
-// round(fp16 h * 2^fw) to the nearest integer, ties to even, without branches (lanes of different rows take
-// different exponents): a normal h is (1024 + mant) 2^(e - 25), a subnormal mant 2^-24. A left shift (sh >= 0) is
-// exact; a right shift by s rounds m >> s with the remainder against half; every shift of 12 or more gives 0 (m <
-// 2^11), so s is clamped to 12, as the 32-bit remainder arithmetic needs.
-__device__ inline int64_t fp16_fixed(uint32_t h, int fw) {
-  const uint32_t e = (h >> 10) & 31, mant = h & 0x3FF;
-  const uint32_t m = e == 0 ? mant : (mant | 0x400);
-  const int sh = (e == 0 ? 1 : (int)e) - 25 + fw;
-  const int64_t rp = (int64_t)m << (sh > 0 ? sh : 0);
-  const uint32_t s = sh < 0 ? (uint32_t)(-sh < 12 ? -sh : 12) : 1u;
-  const uint32_t q = m >> s, rem = m & ((1u << s) - 1u), half = 1u << (s - 1u);
-  const uint32_t rn = q + ((rem > half || (rem == half && (q & 1u))) ? 1u : 0u);
-  const int64_t r = sh >= 0 ? rp : (int64_t)rn;
-  return ((h >> 15) & 1) ? -r : r;
-}
-
-// fp16_fixed with the right-shift rounding done by the float unit: m 2^sh for sh < 0 is exact in single precision
-// (m < 2^11) and rint rounds it half to even like the integer rule (values below one half, where the integer rule
-// clamps its shift, round to 0 either way); sh >= 0 is the exact left shift. Branch-free, about half the integer
-// rule's instructions; exponent 31 is treated as finite exactly as there.
+// round(fp16 h * 2^fw) to the nearest integer, ties to even, without branches (lanes of different rows take different
+// exponents): a normal h is (1024 + mant) 2^(e - 25), a subnormal mant 2^-24. A left shift (sh >= 0) is exact; the right
+// shift's rounding is done by the float unit: m 2^sh is exact in single precision (m < 2^11) and rint rounds it half to
+// even. Exponent 31 is treated as finite.
 __device__ inline int64_t fp16_fixed_fast(uint32_t h, int fw) {
   const uint32_t e = (h >> 10) & 31, mant = h & 0x3FF;
   const uint32_t m = e == 0 ? mant : (mant | 0x400);
@@ -418,7 +402,6 @@ __global__ __launch_bounds__(256) void qk_prep_kernel(const int64_t* __restrict_
 }
 
 __global__ void qk_flag_reset_kernel(int* f) { *f = 0; }
-__global__ void qk_flags_reset_kernel(int* f, int n) { if ((int)threadIdx.x < n) f[threadIdx.x] = 0; }
 
 __device__ inline v4i mfma32(int64_t a, int64_t b, v4i c) {
   return __builtin_amdgcn_mfma_i32_16x16x32_i8((long)a, (long)b, c, 0, 0, 0);
@@ -1007,8 +990,8 @@ __device__ inline void q4_block_mfma(const Q4Lane& w, const int8_t* a, int gstri
   }
 }
 
-// Waves 0..3 walk the gate rows and 4..7 the up rows of the same 64 rows, two blocks ahead each; their results meet in
-// LDS for the SiLU pass, a thread per (token, row).
+// Waves 0..3 walk the gate rows and 4..7 the up rows of the same 64 rows, one block ahead each (two were slower, see
+// above); their results meet in LDS for the SiLU pass, a thread per (token, row).
 __global__ __launch_bounds__(512, 4) void moe_gateup_kernel(const MoeItem* __restrict__ items, const int* __restrict__ ptok,
                                                          const int* __restrict__ ppair, const int8_t* __restrict__ xd,
                                                          const int* __restrict__ Lrow, int64_t rows, int64_t K,
@@ -1210,7 +1193,6 @@ __global__ __launch_bounds__(256, 4) void moe_down_kernel(const MoeItem* __restr
   }
 }
 
-// int8-MFMA path on/off (IMIE_QK_MFMA=0 forces the VALU kernel; tests compare both)
 // ---------------------------------------------------------------------------------------------------------
 // Single-row products (decode): a Q4_K / Q6_K weight against one activation row, and the MoE block of a few tokens.
 // One launch each: every workgroup peels the row's balanced base-256 digits into LDS itself (no prep launch, no flag
@@ -1672,6 +1654,7 @@ __global__ __launch_bounds__(512) void moe1_down_kernel(Moe1Args a) {
   }
 }
 
+// int8-MFMA path on/off (IMIE_QK_MFMA=0 forces the VALU kernel; tests compare both)
 bool qk_mfma_enabled() {
   static const bool v = [] { const char* e = getenv("IMIE_QK_MFMA"); return !(e && atoi(e) == 0); }();
   return v;

@@ -603,6 +603,8 @@ __global__ __launch_bounds__(NT) void q1_gemv_mfma_kernel(
   }
 }
 
+// Straightforward exact kernel (thread per output), an in-library cross-check of the others. Reads the natural
+// (N, nb, 16) layout.
 __global__ void q1_linear_simple_kernel(const int64_t* __restrict__ x, const uint8_t* __restrict__ bits,
                                         const int64_t* __restrict__ scale, int64_t T, int64_t N, int64_t nb,
                                         int frac, int64_t* __restrict__ out) {
@@ -2597,7 +2599,6 @@ static int q1_apply_multi(const Q1Weight* const* ws, int cnt, const int64_t* x_d
   }
   // Work split: waves = tile groups of R tiles; grid.y splits the slabs when there are too few tile groups
   // to keep ~8 waves per CU busy (decode-sized matvecs).
-  // R = 4 only for single-token launches (four tokens x four tiles would exceed the register budget)
   const int R = ntiles_all >= 4 * 16384 ? 4 : (ntiles_all >= 2 * 8192 ? 2 : 1);
   Q1Segs sg = {};
   sg.cnt = cnt;

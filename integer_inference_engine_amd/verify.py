@@ -21,7 +21,7 @@ MI355X design: the artifact is resident (``artifact.register_artifact``), the pr
 all T positions, the LM head writes the (T, vocab) logits into HBM, and the selection (``imie_sample_dev``: argmax,
 penalties, or the seeded sampler) and the row digests (``imie_logits_digest_dev``) run on the device over the rows
 that predict output tokens. Only token ids and 32-byte digests cross PCIe (below 32 rows the rows themselves are
-hashed on the host, which is faster than one serial device SHA-256 lane). The cached replay runs the device decode
+hashed on the host, which is faster than the device's serial SHA-256 chain, two lanes a row). The cached replay runs the device decode
 loop (``imie_net_decode_dev`` / ``imie_net_decode_sampled_dev``); the device verifier has no host compute path.
 """
 from __future__ import annotations
