@@ -60,8 +60,8 @@ def test_hbm_read_peak_calibration_is_plausible(gpu):
 
 @pytest.mark.parametrize("N,nb,T", [(16, 4, 1), (37, 3, 1), (256, 32, 1), (1024, 96, 1), (100, 5, 3), (64, 8, 7),
                                     # decode-sized launches whose waves request 4 / 2 slabs at once, with a short
-                                    # last slab range (10 = 4 + 4 + 2 slabs, 25 = 12 * 2 + 1)
-                                    (24576, 40, 1), (24576, 32, 1), (4096, 100, 1)])
+                                    # last slab range (10 = 4 + 4 + 2 slabs, 3 = 2 + 1); 25 slabs in the one-row kernel
+                                    (24576, 40, 1), (24576, 32, 1), (16640, 12, 1), (4096, 100, 1)])
 def test_q1_apply_matches_oracle_shapes(gpu, N, nb, T):
     seed = N * 1000 + nb * 10 + T
     bits = prng.uniform_bytes(seed, 1, (N, nb, 16))
@@ -73,11 +73,12 @@ def test_q1_apply_matches_oracle_shapes(gpu, N, nb, T):
 
 
 @pytest.mark.parametrize("N,nb,T,xmag", [
-    (64, 200, 3, 45),      # 50 slabs over 8 K-splits x 3 tokens: no staged limbs, every limb group from memory
-    (64, 128, 4, 45),      # 16 staged slab-tokens: limbs 0-3 from LDS, limbs 4-7 from memory
+    (64, 200, 3, 45),      # several rows: limbs 0-3 from LDS, limbs 4-7 from memory; one slab a range
+    (64, 128, 4, 45),
     (64, 128, 4, 62),
     (24576, 40, 1, 45),    # decode launch, 4 slabs requested at once, two limb groups
-    (4096, 100, 1, 62),    # decode launch, 2 slabs at once, eight limbs
+    (16640, 12, 1, 62),    # decode launch, 2 slabs at once, eight limbs
+    (4096, 100, 1, 62),    # one-row kernel, eight limbs
 ])
 def test_q1_limb_groups_from_lds_and_memory(gpu, N, nb, T, xmag):
     seed = N + nb + T + xmag

@@ -1,4 +1,5 @@
-"""Q1_0 GEMM path (T >= 8 tokens: int8 MFMA with tokens in the M dimension) vs the oracle, byte for byte."""
+"""Q1_0 GEMM path (T >= 9 tokens: int8 MFMA with tokens in the M dimension) vs the oracle, byte for byte; its lower edge
+against the few-row kernel of 8 tokens."""
 import numpy as np
 import pytest
 
@@ -9,7 +10,7 @@ pytestmark = pytest.mark.gpu
 I64_MIN, I64_MAX = -(1 << 63), (1 << 63) - 1
 
 
-@pytest.mark.parametrize("N,nb,T", [(16, 1, 8), (37, 3, 9), (200, 5, 64), (1000, 8, 100), (129, 32, 300),
+@pytest.mark.parametrize("N,nb,T", [(16, 1, 8), (16, 1, 9), (37, 3, 9), (200, 5, 64), (1000, 8, 100), (129, 32, 300),
                                     (4096, 32, 64)])
 def test_gemm_shapes(gpu, N, nb, T):
     seed = N * 7 + nb * 3 + T
@@ -192,8 +193,8 @@ def test_gemm_sign_copy_partial_ranges(gpu, nb, s):
     assert got is not None and np.array_equal(got, q1_linear(x, bits, scale, 16))
 
 
-# ---- 8 <= T <= 64: the batched-decode kernel (one token tile, K ranges of 1 / 2 / 4 blocks) ----------------------
-@pytest.mark.parametrize("N,nb,T", [(300, 12, 8), (300, 12, 16), (257, 5, 17), (1000, 8, 32), (64, 13, 33),
+# ---- 9 <= T <= 64: the batched-decode kernel (one token tile, K ranges of 1 / 2 / 4 blocks) ----------------------
+@pytest.mark.parametrize("N,nb,T", [(300, 12, 8), (300, 12, 9), (300, 12, 16), (257, 5, 17), (1000, 8, 32), (64, 13, 33),
                                     (513, 4, 48), (4096, 32, 64), (40, 96, 31)])
 def test_gemm_batched_decode_shapes(gpu, N, nb, T):
     seed = N * 13 + nb * 7 + T
