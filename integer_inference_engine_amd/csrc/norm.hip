@@ -438,7 +438,8 @@ int bonsai_rmsnorm_gpu(const int64_t* x, int64_t rows, int64_t cols, int64_t fra
 // Host evaluation of the RMSNorm kernels' exact helpers (CPU test hooks, no reference counterpart):
 // floor(sqrt(hi * 2^64 + lo)), floor((2^64 - 1) / d) and floor((hi * 2^64 + lo) / d) (low 64 bits).
 // The fused producer (RMSNorm that also writes the next Q1 matvec's digit table, used by the resident decode
-// for fewer than imie_q1::kGemmMinT rows) with bonsai_rmsnorm_gpu's host contract: same outputs and rc, the table goes to a workspace.
+// for fewer than imie_q1::kGemmMinT rows) with bonsai_rmsnorm_gpu's host contract: same outputs and rc, the table
+// goes to a workspace.
 // cols must be a multiple of 128 and at most 4096.
 int imie_rmsnorm_fused_gpu(const int64_t* x, int64_t rows, int64_t cols, int64_t frac, int64_t eps,
                            const int64_t* gain, int64_t* out) {
